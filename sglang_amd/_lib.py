@@ -12,6 +12,27 @@ from pathlib import Path
 
 import torch
 
+
+class _NotBuilt:
+    """Stands in for the extension module where it has not been built: every use raises."""
+
+    def __init__(self, error):
+        self._error = error
+
+    def __getattr__(self, name):
+        raise RuntimeError(
+            "sglang_amd/_native.so is missing or does not load: build it first (python -m sglang_amd.build). "
+            "There is no non-HIP fallback for these operators."
+        ) from self._error
+
+
+try:
+    # the per-layer operators' host path (csrc/host.cpp); its functions return None for calls that need
+    # conversions or an error message, which the Python functions around them then give
+    from . import _native as native
+except ImportError as _error:
+    native = _NotBuilt(_error)
+
 # SGLQ_LIBRARY points at another build of the same C ABI (kernel development)
 LIB_PATH = Path(os.environ.get("SGLQ_LIBRARY") or Path(__file__).resolve().parent / "libsglq.so")
 
@@ -103,6 +124,7 @@ def load() -> ctypes.CDLL:
     lib.sglq_debug_last_gemm_kernel.restype = ctypes.c_char_p
     lib.sglq_debug_last_gemm_hw_scaled.argtypes = []
     lib.sglq_debug_last_gemm_hw_scaled.restype = ctypes.c_int
+    native.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in native.entry_points()})
     _lib = lib
     if os.environ.get("SGLQ_NO_TUNED_CONFIGS", "0") != "1":
         # per-(N, K) kernel selections shipped beside the package (sglang_amd/quantization/configs/)

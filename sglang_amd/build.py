@@ -3,7 +3,9 @@
 ``python -m sglang_amd.build`` compiles the operator sources under ``csrc/`` into
 ``sglang_amd/libsglq.so`` (plain C ABI, ``include/sglq.h``; does not link against torch) and
 the measurement kernels (``csrc/bench_kernels.hip``: MFMA ceiling loop, clock probe, streaming
-passes) into ``sglang_amd/libsglq_bench.so``, which only ``bench.py`` loads.
+passes) into ``sglang_amd/libsglq_bench.so``, which only ``bench.py`` loads.  ``csrc/host.cpp``, the
+operators' host path, becomes the extension module ``sglang_amd/_native.so`` (host code only, against
+torch's headers; it calls libsglq through the addresses that ``_lib.load()`` hands it).
 """
 
 from __future__ import annotations
@@ -12,12 +14,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libsglq.so"
 BENCH_LIB_PATH = PKG_DIR / "libsglq_bench.so"
+NATIVE_PATH = PKG_DIR / "_native.so"
 SOURCES = ["common.hip", "quant.hip", "moe.hip", "gemm.hip"]
 BENCH_SOURCES = ["bench_kernels.hip"]
 
@@ -38,6 +42,33 @@ def find_hipcc() -> str:
         if cand and os.path.exists(cand):
             return cand
     raise RuntimeError("hipcc not found (looked at $HIPCC, PATH and /opt/rocm/bin/hipcc)")
+
+
+def native_command() -> list:
+    """The compiler call for csrc/host.cpp."""
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    includes = [root / "include", root / "include" / "torch" / "csrc" / "api" / "include", Path(rocm) / "include",
+                sysconfig.get_paths()["include"]]
+    return [
+        os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+        "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+        *[a for p in includes for a in ("-isystem", str(p))],
+        str(CSRC / "host.cpp"), "-o", str(NATIVE_PATH),
+        f"-L{root / 'lib'}", "-lc10", "-ltorch_cpu", "-ltorch_python", "-lc10_hip", "-ltorch_hip",
+    ]
+
+
+def build_native(verbose: bool = False) -> Path:
+    cmd = native_command()
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    out = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if out.returncode != 0:
+        raise RuntimeError("the host path did not compile:\n" + out.stdout)
+    return NATIVE_PATH
 
 
 def build(verbose: bool = False, jobs: int = 4) -> Path:
@@ -69,6 +100,7 @@ def build(verbose: bool = False, jobs: int = 4) -> Path:
     out = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if out.returncode != 0:
         raise RuntimeError("link of the measurement kernels failed:\n" + out.stdout)
+    build_native(verbose)
     return LIB_PATH
 
 

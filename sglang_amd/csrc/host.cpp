@@ -1,0 +1,599 @@
+// The host path of the operators that a model calls once per layer and step: argument checks,
+// outputs, scratch, stream, and the calls into libsglq, in one C++ call per operator.
+//
+// What bounds a decode-sized call is this path, not the GPU: through ctypes a linear of one to a few
+// hundred rows took 17-37 us of Python (two launches of together 5-25 us on the GPU), most of it tensor
+// properties read one attribute at a time, views (`.T`, `.view`), three `torch.empty`, two trips through
+// the dispatcher and the conversion of 18 arguments per ctypes call.  From here: 1 x 2112 x 7168 block-FP8
+// linear 17.4 -> 8.0 us a pass (GPU-bound now), 16 x 14336 x 4096 INT8 with bias 26.2 -> 16.0, the two
+// operators on 333 x 4096 x 7168 35.5 -> 28.7, small shapes 25-36 -> 7-13.
+//
+// Every function here takes exactly the calls that need no conversion and no error message: tensors on
+// the GPU in the layouts the kernels read.  For anything else (another layout, a shape or dtype that the
+// operator refuses, a dispatch mode or autograd in the way) it returns None, and the Python function it
+// was called from composes the same operators with torch or raises.
+//
+// The library's entry points arrive as addresses (`bind`), so that the shared object that `_lib.load()`
+// opened is the one that runs.
+#include <Python.h>
+
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <ATen/core/grad_mode.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <ATen/ops/add.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+
+#include <cstdint>
+#include <memory>
+#include <mutex>
+#include <unordered_map>
+#include <vector>
+
+#include "../../include/sglq.h"
+
+namespace {
+
+// ---------------------------------------------------------------------------
+// the library's entry points
+// ---------------------------------------------------------------------------
+#define SGLQ_HOST_ENTRY_POINTS(X)                                                                                   \
+  X(sglq_per_token_group_quant_fp8)                                                                                 \
+  X(sglq_per_token_group_quant_int8)                                                                                \
+  X(sglq_per_token_group_quant_fp8_pow2)                                                                            \
+  X(sglq_per_token_quant_fp8)                                                                                       \
+  X(sglq_per_token_quant_int8)                                                                                      \
+  X(sglq_fp8_blockwise_scaled_mm)                                                                                   \
+  X(sglq_fp8_blockwise_scaled_mm_bias)                                                                              \
+  X(sglq_fp8_blockwise_scaled_mm_ue8m0)                                                                             \
+  X(sglq_int8_blockwise_scaled_mm)                                                                                  \
+  X(sglq_int8_blockwise_scaled_mm_bias)                                                                             \
+  X(sglq_int8_scaled_mm)                                                                                            \
+  X(sglq_fp8_scaled_mm)                                                                                             \
+  X(sglq_w8a8_block_fp8_linear)                                                                                     \
+  X(sglq_w8a8_int8_linear)                                                                                          \
+  X(sglq_w8a8_fp8_linear)
+
+struct EntryPoints {
+#define X(name) decltype(&::name) name = nullptr;
+  SGLQ_HOST_ENTRY_POINTS(X)
+#undef X
+};
+EntryPoints lib;
+bool bound = false;
+
+// ---------------------------------------------------------------------------
+// scratch: per device and stream, so that two streams never share it; a mutex per buffer keeps the
+// launches of one operator together when two threads use one stream
+// ---------------------------------------------------------------------------
+constexpr int64_t SPLITK_BYTES = 64 << 20;  // what the GEMMs' selection rules were measured with
+// Quantized activations in front of it: kept for the sizes where an allocation would be felt (16 MiB is
+// 4096 rows of 4096, or 512 rows of 28672), allocated per call above.
+constexpr int64_t CODES_BYTES = (16 << 20) + (1 << 20);
+constexpr size_t MAX_WORKSPACES = 64;  // beyond as many (device, stream) pairs scratch is allocated per call
+
+struct Workspace {
+  at::Tensor buffer;
+  char* base = nullptr;
+  std::mutex lock;
+};
+
+struct StreamKey {
+  int device;
+  void* stream;
+  bool operator==(const StreamKey& o) const { return device == o.device && stream == o.stream; }
+};
+struct StreamKeyHash {
+  size_t operator()(const StreamKey& k) const { return std::hash<void*>()(k.stream) * 31 + (size_t)k.device; }
+};
+std::mutex workspaces_lock;
+std::unordered_map<StreamKey, std::shared_ptr<Workspace>, StreamKeyHash> workspaces;
+
+at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dtype, c10::Device device) {
+  return at::detail::empty_cuda(sizes, dtype, device, std::nullopt);
+}
+
+std::shared_ptr<Workspace> workspace_of(c10::Device device, void* stream) {
+  std::lock_guard<std::mutex> guard(workspaces_lock);
+  auto it = workspaces.find(StreamKey{device.index(), stream});
+  if (it != workspaces.end()) return it->second;
+  auto w = std::make_shared<Workspace>();
+  w->buffer = empty({CODES_BYTES + SPLITK_BYTES}, at::kByte, device);
+  w->base = static_cast<char*>(w->buffer.data_ptr());
+  if (workspaces.size() < MAX_WORKSPACES) workspaces.emplace(StreamKey{device.index(), stream}, w);
+  return w;
+}
+
+// ---------------------------------------------------------------------------
+// arguments
+// ---------------------------------------------------------------------------
+using at::Tensor;
+
+constexpr auto FP8 = at::kFloat8_e4m3fn;
+
+inline int dtype_code(at::ScalarType t) {
+  switch (t) {
+    case at::kBFloat16: return SGLQ_BF16;
+    case at::kHalf: return SGLQ_FP16;
+    case at::kFloat: return SGLQ_FP32;
+    default: return -1;
+  }
+}
+inline bool is_16bit(at::ScalarType t) { return t == at::kBFloat16 || t == at::kHalf; }
+
+// A plain tensor (or Parameter) on the GPU; subclasses with behaviour of their own stay with Python.
+inline const Tensor* gpu_tensor(PyObject* o) {
+  if (!THPVariable_CheckExact(o)) return nullptr;
+  const Tensor& t = THPVariable_Unpack(o);
+  return t.is_cuda() && t.layout() == at::kStrided ? &t : nullptr;
+}
+inline bool optional_tensor(PyObject* o, const Tensor*& t) {
+  t = nullptr;
+  if (o == Py_None) return true;
+  t = gpu_tensor(o);
+  return t != nullptr;
+}
+
+// Whether a call may go past torch's dispatcher: nothing is watching it, nothing needs a gradient.
+template <typename... T>
+inline bool direct(const T&... tensors) {
+  if (!bound || c10::impl::dispatch_mode_enabled()) return false;
+  if (!at::GradMode::is_enabled()) return true;
+  return !(... || tensors.requires_grad());
+}
+inline bool no_grad_of(const Tensor* t) { return t == nullptr || !t->requires_grad() || !at::GradMode::is_enabled(); }
+
+// Current stream and, where the tensors live on another GPU than the current one, that GPU made current.
+struct Launch {
+  c10::Device device;
+  c10::DeviceIndex previous = -1;
+  void* stream;
+  explicit Launch(c10::Device d) : device(d) {
+    const c10::DeviceIndex current = c10::hip::current_device();
+    if (current != d.index()) {
+      previous = current;
+      c10::hip::set_device(d.index());
+    }
+    stream = static_cast<void*>(c10::hip::getCurrentHIPStream(d.index()).stream());
+  }
+  ~Launch() {
+    if (previous >= 0) c10::hip::set_device(previous);
+  }
+};
+
+struct ReleaseGil {
+  PyThreadState* state;
+  ReleaseGil() : state(PyEval_SaveThread()) {}
+  ~ReleaseGil() { PyEval_RestoreThread(state); }
+};
+
+inline int64_t round256(int64_t v) { return (v + 255) & ~int64_t(255); }
+
+inline PyObject* none() { Py_RETURN_NONE; }
+
+// [..., K] -> [..., n]
+inline std::vector<int64_t> output_shape(const Tensor& x, int64_t n) {
+  std::vector<int64_t> s(x.sizes().begin(), x.sizes().end());
+  s.back() = n;
+  return s;
+}
+
+// C++ exceptions (the allocator's out-of-memory among them) become torch's Python errors.
+template <typename F>
+PyObject* guarded(F&& body) {
+  HANDLE_TH_ERRORS
+  return body();
+  END_HANDLE_TH_ERRORS
+}
+
+inline bool aligned(const Tensor& t, uintptr_t bytes) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & (bytes - 1)) == 0; }
+
+// Activations [..., K] as the quantization kernels read them.
+inline bool activations(const Tensor& x) {
+  return is_16bit(x.scalar_type()) && x.dim() >= 1 && x.is_contiguous() && x.numel() > 0 && aligned(x, 16);
+}
+inline bool bias_fits(const Tensor* bias, int64_t n, at::ScalarType dtype, const Tensor& like) {
+  return bias == nullptr || (bias->scalar_type() == dtype && bias->is_contiguous() && bias->numel() == n && bias->device() == like.device());
+}
+
+// ---------------------------------------------------------------------------
+// block-scaled linears: x [..., K], weight [N, K] as stored, weight_scale [ceil(N/128), K/128]
+// ---------------------------------------------------------------------------
+enum BlockMode { BLOCK_FP8 = 0, BLOCK_FP8_POW2 = 1, BLOCK_INT8 = 2 };
+
+// Weights whose scales are known to be powers of two (the Python side reads them back once per tensor)
+struct WeightKey {
+  const void* ptr;
+  int64_t rows, cols;
+  uint32_t version;
+  bool operator==(const WeightKey& o) const { return ptr == o.ptr && rows == o.rows && cols == o.cols && version == o.version; }
+};
+struct WeightKeyHash {
+  size_t operator()(const WeightKey& k) const { return std::hash<const void*>()(k.ptr) * 31 + k.version; }
+};
+std::mutex pow2_lock;
+std::unordered_map<WeightKey, bool, WeightKeyHash> pow2_weights;
+
+inline WeightKey weight_key(const Tensor& t) { return {t.data_ptr(), t.size(0), t.size(1), (uint32_t)t._version()}; }
+
+PyObject* note_pow2_scales(PyObject*, PyObject* arg) {
+  return guarded([&]() -> PyObject* {
+    const Tensor* t = gpu_tensor(arg);
+    if (t && t->dim() == 2 && !t->is_inference()) {
+      std::lock_guard<std::mutex> guard(pow2_lock);
+      if (pow2_weights.size() > 4096) pow2_weights.clear();
+      pow2_weights.emplace(weight_key(*t), true);
+    }
+    return none();
+  });
+}
+
+// block_linear(x, weight, weight_scale, bias | None, mode, eps) -> [..., N]
+PyObject* block_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 6) return PyErr_Format(PyExc_TypeError, "block_linear takes 6 arguments");
+  return guarded([&]() -> PyObject* {
+    const Tensor *xp = gpu_tensor(args[0]), *wp = gpu_tensor(args[1]), *sp = gpu_tensor(args[2]), *bias;
+    if (!xp || !wp || !sp || !optional_tensor(args[3], bias)) return none();
+    const long mode = PyLong_AsLong(args[4]);
+    const float eps = (float)PyFloat_AsDouble(args[5]);
+    const Tensor &x = *xp, &w = *wp, &s = *sp;
+    if (!direct(x, w, s) || !no_grad_of(bias)) return none();
+    if (!activations(x) || w.dim() != 2 || s.dim() != 2 || !w.is_contiguous() || s.scalar_type() != at::kFloat) return none();
+    if (w.scalar_type() != (mode == BLOCK_INT8 ? at::kChar : FP8)) return none();
+    const int64_t k = x.size(-1), m = x.numel() / k, n = w.size(0), kb = k / 128;
+    if (w.size(1) != k || k % 128 != 0 || n % 8 != 0 || n == 0 || s.size(0) != (n + 127) / 128 || s.size(1) != kb) return none();
+    if (s.stride(1) != 1 && kb > 1) return none();
+    if (w.device() != x.device() || s.device() != x.device() || !aligned(w, 16)) return none();
+    const at::ScalarType dtype = x.scalar_type();
+    if (!bias_fits(bias, n, dtype, x)) return none();
+    if (mode == BLOCK_FP8_POW2) {
+      if (dtype != at::kBFloat16 || n % 64 != 0 || s.is_inference()) return none();
+      std::lock_guard<std::mutex> guard(pow2_lock);
+      if (pow2_weights.find(weight_key(s)) == pow2_weights.end()) return none();
+    }
+    const int64_t need = round256(m * k) + round256(m * kb * 4);
+    Tensor out;
+    int rc;
+    {
+      ReleaseGil unlocked;
+      Launch here(x.device());
+      out = empty(output_shape(x, n), dtype, here.device);
+      auto ws = workspace_of(here.device, here.stream);
+      Tensor large;
+      if (need > CODES_BYTES) large = empty({need}, at::kByte, here.device);
+      std::lock_guard<std::mutex> one_operator(ws->lock);
+      const int code = dtype_code(dtype);
+      void* out_p = out.data_ptr();
+      const void *x_p = x.data_ptr(), *w_p = w.data_ptr(), *bias_p = bias ? bias->data_ptr() : nullptr;
+      const float* s_p = static_cast<const float*>(s.data_ptr());
+      const int64_t sn = s.stride(0);
+      if (mode == BLOCK_FP8 && need <= CODES_BYTES) {
+        // codes, scales and split-K partial sums in one piece: the same 64 MiB for the latter whatever the codes take
+        rc = lib.sglq_w8a8_block_fp8_linear(x_p, code, w_p, k, s_p, 1, sn, bias_p, out_p, n, code, m, n, k, eps, ws->base,
+                                            need + SPLITK_BYTES, here.stream);
+      } else {
+        char* codes = need > CODES_BYTES ? static_cast<char*>(large.data_ptr()) : ws->base;
+        float* scales = reinterpret_cast<float*>(codes + round256(m * k));
+        void* partial = ws->base + CODES_BYTES;
+        if (mode == BLOCK_INT8) {  // row-major activation scales
+          rc = lib.sglq_per_token_group_quant_int8(x_p, code, codes, scales, m, k, 128, kb, 1, eps, -128.0f, 127.0f, here.stream);
+          if (rc == 0 && bias_p)
+            rc = lib.sglq_int8_blockwise_scaled_mm_bias(codes, k, w_p, k, scales, kb, 1, s_p, 1, sn, bias_p, out_p, n, code, m, n, k, partial,
+                                                        SPLITK_BYTES, here.stream);
+          else if (rc == 0)
+            rc = lib.sglq_int8_blockwise_scaled_mm(codes, k, w_p, k, scales, kb, 1, s_p, 1, sn, out_p, n, code, m, n, k, partial, SPLITK_BYTES,
+                                                   here.stream);
+        } else if (mode == BLOCK_FP8_POW2) {
+          rc = lib.sglq_per_token_group_quant_fp8_pow2(x_p, code, codes, scales, m, k, 1, m, eps, -448.0f, 448.0f, here.stream);
+          if (rc == 0)
+            rc = lib.sglq_fp8_blockwise_scaled_mm_ue8m0(codes, k, w_p, k, scales, 1, m, s_p, 1, sn, out_p, n, code, m, n, k, partial,
+                                                        SPLITK_BYTES, here.stream);
+        } else {
+          rc = lib.sglq_per_token_group_quant_fp8(x_p, code, codes, scales, m, k, 128, 1, m, eps, -448.0f, 448.0f, here.stream);
+          if (rc == 0 && bias_p)
+            rc = lib.sglq_fp8_blockwise_scaled_mm_bias(codes, k, w_p, k, scales, 1, m, s_p, 1, sn, bias_p, out_p, n, code, m, n, k, partial,
+                                                       SPLITK_BYTES, here.stream);
+          else if (rc == 0)
+            rc = lib.sglq_fp8_blockwise_scaled_mm(codes, k, w_p, k, scales, 1, m, s_p, 1, sn, out_p, n, code, m, n, k, partial, SPLITK_BYTES,
+                                                  here.stream);
+        }
+      }
+      if (rc == 0 && bias && mode == BLOCK_FP8_POW2) {
+        at::NoGradGuard no_grad;
+        out.add_(*bias);
+      }
+    }
+    return rc == 0 ? THPVariable_Wrap(std::move(out)) : none();
+  });
+}
+
+// token_linear(x, weight_kn, weight_scale, bias | None, is_int8) -> [..., N]: per-token activation scales,
+// per-channel weight scales; weight_kn [K, N] column-major
+PyObject* token_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 5) return PyErr_Format(PyExc_TypeError, "token_linear takes 5 arguments");
+  return guarded([&]() -> PyObject* {
+    const Tensor *xp = gpu_tensor(args[0]), *wp = gpu_tensor(args[1]), *sp = gpu_tensor(args[2]), *bias;
+    if (!xp || !wp || !sp || !optional_tensor(args[3], bias)) return none();
+    const bool int8 = args[4] == Py_True;
+    const Tensor &x = *xp, &w = *wp, &s = *sp;
+    if (!direct(x, w, s) || !no_grad_of(bias)) return none();
+    if (!activations(x) || w.dim() != 2 || w.stride(0) != 1 || w.scalar_type() != (int8 ? at::kChar : FP8)) return none();
+    const int64_t k = x.size(-1), m = x.numel() / k, n = w.size(1);
+    if (w.size(0) != k || k % 16 != 0 || n % 8 != 0 || n <= 1) return none();
+    const int64_t ldb = w.stride(1);
+    if (ldb % 16 != 0 || ldb < k || !aligned(w, 16)) return none();
+    if (s.scalar_type() != at::kFloat || !s.is_contiguous() || s.numel() != n || !aligned(s, 16)) return none();
+    if (w.device() != x.device() || s.device() != x.device()) return none();
+    const at::ScalarType dtype = x.scalar_type();
+    if (!bias_fits(bias, n, dtype, x)) return none();
+    const int64_t need = round256(m * k) + round256(m * 4);
+    Tensor out;
+    int rc;
+    {
+      ReleaseGil unlocked;
+      Launch here(x.device());
+      out = empty(output_shape(x, n), dtype, here.device);
+      auto ws = workspace_of(here.device, here.stream);
+      Tensor large;
+      if (need > CODES_BYTES) large = empty({need}, at::kByte, here.device);
+      std::lock_guard<std::mutex> one_operator(ws->lock);
+      const int code = dtype_code(dtype);
+      const void *x_p = x.data_ptr(), *w_p = w.data_ptr(), *bias_p = bias ? bias->data_ptr() : nullptr;
+      const float* s_p = static_cast<const float*>(s.data_ptr());
+      if (need <= CODES_BYTES) {
+        rc = (int8 ? lib.sglq_w8a8_int8_linear : lib.sglq_w8a8_fp8_linear)(x_p, code, w_p, ldb, s_p, bias_p, out.data_ptr(), n, code, m, n, k,
+                                                                           ws->base, need + SPLITK_BYTES, here.stream);
+      } else {
+        char* codes = static_cast<char*>(large.data_ptr());
+        float* scales = reinterpret_cast<float*>(codes + round256(m * k));
+        rc = int8 ? lib.sglq_per_token_quant_int8(x_p, code, codes, scales, nullptr, m, k, here.stream)
+                  : lib.sglq_per_token_quant_fp8(x_p, code, codes, scales, m, k, here.stream);
+        if (rc == 0)
+          rc = (int8 ? lib.sglq_int8_scaled_mm : lib.sglq_fp8_scaled_mm)(codes, k, w_p, ldb, scales, s_p, bias_p, out.data_ptr(), n, code, m, n, k,
+                                                                         ws->base + CODES_BYTES, SPLITK_BYTES, here.stream);
+      }
+    }
+    return rc == 0 ? THPVariable_Wrap(std::move(out)) : none();
+  });
+}
+
+// ---------------------------------------------------------------------------
+// the operators one by one
+// ---------------------------------------------------------------------------
+inline bool out_dtype_of(PyObject* o, at::ScalarType& t) {
+  if (!THPDtype_Check(o)) return false;
+  t = reinterpret_cast<THPDtype*>(o)->scalar_type;
+  return is_16bit(t);
+}
+
+// What the three GEMM operators ask of their operands (check_mm_common in sgl_kernel/gemm.py).
+inline bool mm_operands(const Tensor& a, const Tensor& b, at::ScalarType elem) {
+  if (a.dim() != 2 || b.dim() != 2 || a.scalar_type() != elem || b.scalar_type() != elem) return false;
+  const int64_t m = a.size(0), k = a.size(1), n = b.size(1);
+  if (m == 0 || n == 0 || k == 0 || b.size(0) != k || k % 16 != 0 || n % 8 != 0) return false;
+  if (a.stride(1) != 1 || b.stride(0) != 1 || (m > 1 && a.stride(0) % 16 != 0) || (n > 1 && b.stride(1) % 16 != 0)) return false;
+  return a.device() == b.device();
+}
+inline bool vector_like(const Tensor& t) {
+  return t.is_contiguous() && (t.dim() == 1 || (t.dim() == 2 && (t.size(0) == 1 || t.size(1) == 1)));
+}
+
+// blockwise_mm(a, b, scales_a, scales_b, out_dtype, bias | None, dispatched) -> [M, N]
+// `dispatched`: called from the operator's implementation, behind torch's dispatcher.
+PyObject* blockwise_mm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 7) return PyErr_Format(PyExc_TypeError, "blockwise_mm takes 7 arguments");
+  return guarded([&]() -> PyObject* {
+    const Tensor *ap = gpu_tensor(args[0]), *bp = gpu_tensor(args[1]), *sap = gpu_tensor(args[2]), *sbp = gpu_tensor(args[3]), *bias;
+    at::ScalarType dtype;
+    if (!ap || !bp || !sap || !sbp || !optional_tensor(args[5], bias) || !out_dtype_of(args[4], dtype)) return none();
+    const Tensor &a = *ap, &b = *bp, &sa = *sap, &sb = *sbp;
+    if (!bound || (args[6] != Py_True && (!direct(a, b, sa, sb) || !no_grad_of(bias)))) return none();
+    if (!mm_operands(a, b, FP8)) return none();
+    const int64_t m = a.size(0), k = a.size(1), n = b.size(1), kb = (k + 127) / 128, nb = (n + 127) / 128;
+    if (sa.scalar_type() != at::kFloat || sb.scalar_type() != at::kFloat || sa.dim() != 2 || sb.dim() != 2) return none();
+    if (sa.size(0) != m || sa.size(1) != kb || sb.size(0) != kb || sb.size(1) != nb) return none();
+    if ((sa.stride(0) != 1 && !vector_like(sa)) || (sb.stride(0) != 1 && !vector_like(sb))) return none();
+    if (sa.device() != a.device() || sb.device() != a.device() || !bias_fits(bias, n, dtype, a)) return none();
+    Tensor out;
+    int rc;
+    {
+      ReleaseGil unlocked;
+      Launch here(a.device());
+      out = empty({m, n}, dtype, here.device);
+      auto ws = workspace_of(here.device, here.stream);
+      std::lock_guard<std::mutex> one_operator(ws->lock);
+      const int64_t lda = m > 1 ? a.stride(0) : k, ldb = n > 1 ? b.stride(1) : k;
+      const float *sa_p = static_cast<const float*>(sa.data_ptr()), *sb_p = static_cast<const float*>(sb.data_ptr());
+      void* partial = ws->base + CODES_BYTES;
+      if (bias)
+        rc = lib.sglq_fp8_blockwise_scaled_mm_bias(a.data_ptr(), lda, b.data_ptr(), ldb, sa_p, sa.stride(0), sa.stride(1), sb_p, sb.stride(0),
+                                                   sb.stride(1), bias->data_ptr(), out.data_ptr(), n, dtype_code(dtype), m, n, k, partial,
+                                                   SPLITK_BYTES, here.stream);
+      else
+        rc = lib.sglq_fp8_blockwise_scaled_mm(a.data_ptr(), lda, b.data_ptr(), ldb, sa_p, sa.stride(0), sa.stride(1), sb_p, sb.stride(0),
+                                              sb.stride(1), out.data_ptr(), n, dtype_code(dtype), m, n, k, partial, SPLITK_BYTES, here.stream);
+    }
+    return rc == 0 ? THPVariable_Wrap(std::move(out)) : none();
+  });
+}
+
+// rowcol_mm(a, b, scales_a, scales_b, out_dtype, bias | None, is_int8, dispatched) -> [M, N]
+PyObject* rowcol_mm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 8) return PyErr_Format(PyExc_TypeError, "rowcol_mm takes 8 arguments");
+  return guarded([&]() -> PyObject* {
+    const Tensor *ap = gpu_tensor(args[0]), *bp = gpu_tensor(args[1]), *sap = gpu_tensor(args[2]), *sbp = gpu_tensor(args[3]), *bias;
+    at::ScalarType dtype;
+    if (!ap || !bp || !sap || !sbp || !optional_tensor(args[5], bias) || !out_dtype_of(args[4], dtype)) return none();
+    const bool int8 = args[6] == Py_True;
+    const Tensor &a = *ap, &b = *bp, &sa = *sap, &sb = *sbp;
+    if (!bound || (args[7] != Py_True && (!direct(a, b, sa, sb) || !no_grad_of(bias)))) return none();
+    if (!mm_operands(a, b, int8 ? at::kChar : FP8)) return none();
+    const int64_t m = a.size(0), k = a.size(1), n = b.size(1);
+    if (sa.scalar_type() != at::kFloat || sb.scalar_type() != at::kFloat || sa.numel() != m || sb.numel() != n) return none();
+    if (!sa.is_contiguous() || !sb.is_contiguous() || sa.device() != a.device() || sb.device() != a.device()) return none();
+    if (!bias_fits(bias, n, dtype, a)) return none();
+    Tensor out;
+    int rc;
+    {
+      ReleaseGil unlocked;
+      Launch here(a.device());
+      out = empty({m, n}, dtype, here.device);
+      auto ws = workspace_of(here.device, here.stream);
+      std::lock_guard<std::mutex> one_operator(ws->lock);
+      rc = (int8 ? lib.sglq_int8_scaled_mm : lib.sglq_fp8_scaled_mm)(
+          a.data_ptr(), m > 1 ? a.stride(0) : k, b.data_ptr(), n > 1 ? b.stride(1) : k, static_cast<const float*>(sa.data_ptr()),
+          static_cast<const float*>(sb.data_ptr()), bias ? bias->data_ptr() : nullptr, out.data_ptr(), n, dtype_code(dtype), m, n, k,
+          ws->base + CODES_BYTES, SPLITK_BYTES, here.stream);
+    }
+    return rc == 0 ? THPVariable_Wrap(std::move(out)) : none();
+  });
+}
+
+inline PyObject* pair_of(Tensor a, Tensor b) {
+  PyObject* first = THPVariable_Wrap(std::move(a));
+  if (!first) return nullptr;
+  PyObject* second = THPVariable_Wrap(std::move(b));
+  PyObject* t = second ? PyTuple_New(2) : nullptr;
+  if (!t) {
+    Py_DECREF(first);
+    Py_XDECREF(second);
+    return nullptr;
+  }
+  PyTuple_SET_ITEM(t, 0, first);
+  PyTuple_SET_ITEM(t, 1, second);
+  return t;
+}
+
+// group_quant_fp8(x, group_size, eps, column_major_scales, padded) -> (codes, scales): the buffers of
+// sglang_per_token_group_quant_fp8 in its fp32 layouts; column-major scales for 2-D inputs.
+PyObject* group_quant_fp8(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 5) return PyErr_Format(PyExc_TypeError, "group_quant_fp8 takes 5 arguments");
+  return guarded([&]() -> PyObject* {
+    const Tensor* xp = gpu_tensor(args[0]);
+    if (!xp || !direct(*xp)) return none();
+    const Tensor& x = *xp;
+    const long group = PyLong_AsLong(args[1]);
+    const float eps = (float)PyFloat_AsDouble(args[2]);
+    if (PyErr_Occurred()) return nullptr;
+    const bool column = PyObject_IsTrue(args[3]) == 1, padded = PyObject_IsTrue(args[4]) == 1;
+    const int code = dtype_code(x.scalar_type());
+    if (code < 0 || x.dim() != 2 || !x.is_contiguous() || x.numel() == 0 || group <= 0 || x.size(1) % group != 0) return none();
+    const int64_t m = x.size(0), k = x.size(1), g = k / group;
+    Tensor q, s;
+    int rc;
+    {
+      ReleaseGil unlocked;
+      Launch here(x.device());
+      q = empty({m, k}, FP8, here.device);
+      if (column) {
+        const int64_t rows = padded ? (m + 3) / 4 * 4 : m;
+        s = empty({g, rows}, at::kFloat, here.device);
+        const int64_t sizes[2] = {m, g}, strides[2] = {1, rows};
+        s.unsafeGetTensorImpl()->set_sizes_and_strides(at::IntArrayRef(sizes, 2), at::IntArrayRef(strides, 2));
+      } else {
+        s = empty({m, g}, at::kFloat, here.device);
+      }
+      rc = lib.sglq_per_token_group_quant_fp8(x.data_ptr(), code, q.data_ptr(), static_cast<float*>(s.data_ptr()), m, k, (int)group, s.stride(0),
+                                              s.stride(1), eps, -448.0f, 448.0f, here.stream);
+    }
+    return rc == 0 ? pair_of(std::move(q), std::move(s)) : none();
+  });
+}
+
+// token_quant(x, is_int8) -> (codes, scales [..., 1])
+PyObject* token_quant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 2) return PyErr_Format(PyExc_TypeError, "token_quant takes 2 arguments");
+  return guarded([&]() -> PyObject* {
+    const Tensor* xp = gpu_tensor(args[0]);
+    if (!xp || !direct(*xp)) return none();
+    const Tensor& x = *xp;
+    const bool int8 = args[1] == Py_True;
+    const int code = dtype_code(x.scalar_type());
+    if (code < 0 || x.dim() < 1 || (!int8 && x.dim() != 2) || !x.is_contiguous() || x.numel() == 0) return none();
+    const int64_t k = x.size(-1), m = x.numel() / k;
+    if (!int8 && k % 8 != 0) return none();
+    Tensor q, s;
+    int rc;
+    {
+      ReleaseGil unlocked;
+      Launch here(x.device());
+      q = empty(x.sizes(), int8 ? at::kChar : FP8, here.device);
+      s = empty(output_shape(x, 1), at::kFloat, here.device);
+      float* s_p = static_cast<float*>(s.data_ptr());
+      rc = int8 ? lib.sglq_per_token_quant_int8(x.data_ptr(), code, q.data_ptr(), s_p, nullptr, m, k, here.stream)
+                : lib.sglq_per_token_quant_fp8(x.data_ptr(), code, q.data_ptr(), s_p, m, k, here.stream);
+    }
+    return rc == 0 ? pair_of(std::move(q), std::move(s)) : none();
+  });
+}
+
+// ---------------------------------------------------------------------------
+// bind({name: address}); release_workspaces()
+// ---------------------------------------------------------------------------
+PyObject* bind(PyObject*, PyObject* table) {
+  EntryPoints e;
+#define X(name)                                                                                                  \
+  {                                                                                                              \
+    PyObject* v = PyDict_Check(table) ? PyDict_GetItemString(table, #name) : nullptr;                            \
+    if (!v) return PyErr_Format(PyExc_KeyError, "bind: the address of %s is missing", #name);                    \
+    e.name = reinterpret_cast<decltype(e.name)>(PyLong_AsVoidPtr(v));                                            \
+    if (!e.name) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_ValueError, "bind: %s is null", #name);  \
+  }
+  SGLQ_HOST_ENTRY_POINTS(X)
+#undef X
+  lib = e;
+  bound = true;
+  return none();
+}
+
+PyObject* entry_points(PyObject*, PyObject*) {
+  PyObject* names = PyList_New(0);
+  if (!names) return nullptr;
+#define X(name)                                             \
+  {                                                         \
+    PyObject* s = PyUnicode_FromString(#name);              \
+    if (!s || PyList_Append(names, s) < 0) {                \
+      Py_XDECREF(s);                                        \
+      Py_DECREF(names);                                     \
+      return nullptr;                                       \
+    }                                                       \
+    Py_DECREF(s);                                           \
+  }
+  SGLQ_HOST_ENTRY_POINTS(X)
+#undef X
+  return names;
+}
+
+PyObject* release_workspaces(PyObject*, PyObject*) {
+  return guarded([&]() -> PyObject* {
+    std::unordered_map<StreamKey, std::shared_ptr<Workspace>, StreamKeyHash> old;
+    {
+      std::lock_guard<std::mutex> guard(workspaces_lock);
+      old.swap(workspaces);
+    }
+    return none();
+  });
+}
+
+#define FAST(f) reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL
+PyMethodDef methods[] = {
+    {"bind", bind, METH_O, "bind({name: address}) of the library's entry points"},
+    {"entry_points", entry_points, METH_NOARGS, "the names that bind() wants"},
+    {"release_workspaces", release_workspaces, METH_NOARGS, "give the kept scratch buffers back to torch's allocator"},
+    {"note_pow2_scales", note_pow2_scales, METH_O, "remember that a weight's block scales are powers of two"},
+    {"block_linear", FAST(block_linear), "quantize and multiply with a block-scaled weight, or None"},
+    {"token_linear", FAST(token_linear), "quantize per token and multiply with a per-channel-scaled weight, or None"},
+    {"blockwise_mm", FAST(blockwise_mm), "block-scaled FP8 GEMM, or None"},
+    {"rowcol_mm", FAST(rowcol_mm), "per-token / per-channel-scaled GEMM, or None"},
+    {"group_quant_fp8", FAST(group_quant_fp8), "per-token-group FP8 quantization, or None"},
+    {"token_quant", FAST(token_quant), "per-token quantization, or None"},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "Host path of the per-layer operators", -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&module); }

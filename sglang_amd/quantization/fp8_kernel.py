@@ -9,7 +9,7 @@ import torch
 from typing import Optional, Tuple
 
 from .. import _lib
-from .._lib import DTYPE_CODE
+from .._lib import DTYPE_CODE, native
 from ..sgl_kernel import sgl_per_tensor_quant_fp8, sgl_per_token_group_quant_fp8, sgl_per_token_quant_fp8
 
 # gfx950 implements the OCP formats: e4m3fn with maximum 448 (fp8_kernel.py:71-85
@@ -58,6 +58,10 @@ def sglang_per_token_group_quant_fp8(
     scale_ue8m0: bool = False,
 ):
     """fp8_kernel.py:344-372."""
+    if not scale_ue8m0:
+        pair = native.group_quant_fp8(x, group_size, eps, column_major_scales, scale_tma_aligned)
+        if pair is not None:
+            return pair
     assert x.shape[-1] % group_size == 0, "the last dimension of `x` cannot be divisible by `group_size`"
     assert x.is_contiguous(), "`x` is not contiguous"
     x_q = torch.empty_like(x, device=x.device, dtype=fp8_dtype)
@@ -81,6 +85,10 @@ per_token_group_quant_fp8 = sglang_per_token_group_quant_fp8
 
 def sglang_per_token_quant_fp8(x: torch.Tensor, dtype: torch.dtype = fp8_dtype):
     """fp8_kernel.py:375-391."""
+    if dtype is fp8_dtype:
+        pair = native.token_quant(x, False)
+        if pair is not None:
+            return pair
     assert x.is_contiguous(), "`x` is not contiguous"
     x_q = torch.empty_like(x, device=x.device, dtype=dtype)
     x_s = torch.empty(x.shape[0], 1, device=x.device, dtype=torch.float32)
@@ -251,6 +259,7 @@ def check_pow2_scales(Bs: torch.Tensor, what: str = "Bs") -> None:
     once per tensor (address, shape and version counter; one device round trip), not under stream capture."""
     key = (Bs.device.type, Bs.data_ptr(), tuple(Bs.shape), Bs._version)
     if key in _pow2_checked:
+        native.note_pow2_scales(Bs)
         return
     if Bs.is_cuda and torch.cuda.is_current_stream_capturing():
         return
@@ -261,6 +270,7 @@ def check_pow2_scales(Bs: torch.Tensor, what: str = "Bs") -> None:
     if len(_pow2_checked) > 4096:
         _pow2_checked.clear()
     _pow2_checked.add(key)
+    native.note_pow2_scales(Bs)
 
 
 def w8a8_block_fp8_matmul_deepgemm(

@@ -8,6 +8,7 @@ from typing import List, Optional
 
 import torch
 
+from .._lib import native
 from ..sgl_kernel import fp8_blockwise_scaled_mm, fp8_scaled_mm
 from ..sgl_kernel.gemm import block_fp8_linear, fp8_blockwise_scaled_mm_bias, fp8_linear
 from .fp8_kernel import (
@@ -45,6 +46,9 @@ def w8a8_block_fp8_linear(
     diverts them to its Triton kernel, :193-199)."""
     assert input_scale is None
     assert list(block_size) == [128, 128], "only 128x128 weight blocks are built"
+    output = native.block_linear(input, weight, weight_scale, bias, 0, 1e-10)
+    if output is not None:
+        return output
     input_2d = input.view(-1, input.shape[-1])
     output_shape = [*input.shape[:-1], weight.shape[0]]
     fusable_bias = bias is None or (bias.dtype == input_2d.dtype and bias.is_contiguous() and bias.numel() == weight.shape[0])
@@ -119,6 +123,10 @@ def apply_fp8_linear(
       chooses between the sgl_kernel GEMM and torch._scaled_mm in the reference; this library has
       one GEMM and uses it for either value."""
     del input_scale_ub, pad_output, cutlass_fp8_supported
+    if input_scale is None and not compressed_tensor_quant:
+        output = native.token_linear(input, weight, weight_scale, bias, False)
+        if output is not None:
+            return output
     input_2d = input.view(-1, input.shape[-1])
     output_shape = [*input.shape[:-1], weight.shape[1]]
     if compressed_tensor_quant:
@@ -177,6 +185,11 @@ def deepgemm_w8a8_block_fp8_linear_with_fallback(
     Without: fp32 scales with the row count padded to a multiple of four (`scale_tma_aligned=True`) and this
     library's block-scaled kernel, which takes the scales' strides as they are."""
     assert input_scale is None
+    if input.dtype == torch.bfloat16 and weight.shape[0] % 64 == 0 and list(block_size) == [128, 128]:
+        # (the scale buffer's padding to four rows is for the reference's TMA loads; nothing here reads it)
+        output = native.block_linear(input, weight, weight_scale, bias, 1 if DEEPGEMM_SCALE_UE8M0 else 0, 1e-10)
+        if output is not None:
+            return output
     if not (input.dtype == torch.bfloat16 and weight.shape[0] % 64 == 0 and weight.shape[1] % 128 == 0):
         return triton_w8a8_block_fp8_linear(input, weight, block_size, weight_scale, input_scale, bias)
     input_2d = input.view(-1, input.shape[-1])

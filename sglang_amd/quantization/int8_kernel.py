@@ -10,10 +10,14 @@ from typing import List, Optional, Tuple
 import torch
 
 from .. import _lib
-from .._lib import DTYPE_CODE
+from .._lib import DTYPE_CODE, native
 
 
 def per_token_quant_int8(x, scale_dtype=torch.float32, cal_sum=False):
+    if scale_dtype is torch.float32 and not cal_sum:
+        pair = native.token_quant(x, True)
+        if pair is not None:
+            return pair
     assert x.is_contiguous()
     if not x.is_cuda:
         raise RuntimeError("per_token_quant_int8: x must be a CUDA tensor")

@@ -7,6 +7,7 @@ from typing import List, Optional
 
 import torch
 
+from .._lib import native
 from .int8_kernel import per_token_group_quant_int8, w8a8_block_int8_matmul
 
 
@@ -19,6 +20,10 @@ def apply_w8a8_block_int8_linear(
     bias: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
     assert input_scale is None
+    if list(block_size) == [128, 128]:
+        output = native.block_linear(input, weight, weight_scale, bias, 2, 1e-10)
+        if output is not None:
+            return output
     input_2d = input.view(-1, input.shape[-1])
     output_shape = [*input.shape[:-1], weight.shape[0]]
     q_input, x_scale = per_token_group_quant_int8(input_2d, block_size[1])

@@ -6,6 +6,7 @@ from typing import Optional
 
 import torch
 
+from .._lib import native
 from ..sgl_kernel import int8_scaled_mm
 from ..sgl_kernel.gemm import int8_linear
 from .int8_kernel import per_token_quant_int8
@@ -33,6 +34,9 @@ def apply_w8a8_int8_linear(
     """W8A8Int8LinearMethod.apply (w8a8_int8.py:371-391): per-token INT8 quantization
     of x followed by int8_scaled_mm with the transposed weight view; decode rows take both steps in one
     operator with the same result."""
+    output = native.token_linear(x, weight, weight_scale, bias, True)
+    if output is not None:
+        return output
     if _fusable(x, weight):
         return int8_linear(x.view(-1, x.shape[-1]), weight, weight_scale, bias).view(*x.shape[:-1], weight.shape[1])
     x_q, x_scale = per_token_quant_int8(x)

@@ -15,7 +15,7 @@ from typing import Optional
 import torch
 
 from .. import _lib
-from .._lib import DTYPE_CODE
+from .._lib import DTYPE_CODE, native
 
 FP8 = torch.float8_e4m3fn
 
@@ -133,6 +133,9 @@ def check_tensor_quant_fp8(input, output_q, output_s, require_cuda=True):
 # op implementations (CUDA dispatch key = ROCm device tensors)
 # ---------------------------------------------------------------------------
 def _int8_scaled_mm_impl(mat_a, mat_b, scales_a, scales_b, out_dtype, bias=None):
+    out = native.rowcol_mm(mat_a, mat_b, scales_a, scales_b, out_dtype, bias, True, True)
+    if out is not None:
+        return out
     check_mm_common(mat_a, mat_b, out_dtype, torch.int8, "Int8")
     _check(mat_a.size(1) % 16 == 0, "mat_a.size(1) must be multiple of 16 for memory alignment")
     _check(mat_b.size(0) % 16 == 0, "mat_b.size(0) must be multiple of 16 for memory alignment")
@@ -152,6 +155,9 @@ def _int8_scaled_mm_impl(mat_a, mat_b, scales_a, scales_b, out_dtype, bias=None)
 
 
 def _fp8_scaled_mm_impl(mat_a, mat_b, scales_a, scales_b, out_dtype, bias=None):
+    out = native.rowcol_mm(mat_a, mat_b, scales_a, scales_b, out_dtype, bias, False, True)
+    if out is not None:
+        return out
     check_mm_common(mat_a, mat_b, out_dtype, FP8, "Float8_e4m3fn")
     check_rowcol_scales(mat_a, mat_b, scales_a, scales_b, out_dtype, bias)
     m, k = mat_a.shape
@@ -169,6 +175,9 @@ def _fp8_scaled_mm_impl(mat_a, mat_b, scales_a, scales_b, out_dtype, bias=None):
 
 
 def _fp8_blockwise_scaled_mm_impl(mat_a, mat_b, scales_a, scales_b, out_dtype):
+    out = native.blockwise_mm(mat_a, mat_b, scales_a, scales_b, out_dtype, None, True)
+    if out is not None:
+        return out
     check_mm_common(mat_a, mat_b, out_dtype, FP8, "Float8_e4m3fn")
     check_blockwise_scales(mat_a, mat_b, scales_a, scales_b)
     m, k = mat_a.shape
@@ -212,6 +221,9 @@ def fp8_blockwise_scaled_mm_ue8m0(mat_a, mat_b, scales_a, scales_b, out_dtype):
 def fp8_blockwise_scaled_mm_bias(mat_a, mat_b, scales_a, scales_b, out_dtype, bias):
     """fp8_blockwise_scaled_mm followed by the caller's `output += bias`
     (fp8_utils.py:207-211) in one kernel; no counterpart among the reference's ops."""
+    out = native.blockwise_mm(mat_a, mat_b, scales_a, scales_b, out_dtype, bias, True)
+    if out is not None:
+        return out
     check_mm_common(mat_a, mat_b, out_dtype, FP8, "Float8_e4m3fn")
     check_blockwise_scales(mat_a, mat_b, scales_a, scales_b)
     m, k = mat_a.shape
@@ -404,17 +416,29 @@ for _name, _schema in _SCHEMAS.items():
 
 
 # ---------------------------------------------------------------------------
-# public wrappers: same names, argument order and forwarding as the reference
+# public wrappers: same names, argument order and forwarding as the reference.  Plain calls
+# go straight to the host path that the operators' implementations end in; torch's dispatcher
+# (about 8 us with a Python implementation behind it) is left to those that something watches
+# or that need an error message.
 # ---------------------------------------------------------------------------
 def int8_scaled_mm(mat_a, mat_b, scales_a, scales_b, out_dtype, bias=None):
+    out = native.rowcol_mm(mat_a, mat_b, scales_a, scales_b, out_dtype, bias, True, False)
+    if out is not None:
+        return out
     return torch.ops.sgl_kernel.int8_scaled_mm.default(mat_a, mat_b, scales_a, scales_b, out_dtype, bias)
 
 
 def fp8_blockwise_scaled_mm(mat_a, mat_b, scales_a, scales_b, out_dtype):
+    out = native.blockwise_mm(mat_a, mat_b, scales_a, scales_b, out_dtype, None, False)
+    if out is not None:
+        return out
     return torch.ops.sgl_kernel.fp8_blockwise_scaled_mm.default(mat_a, mat_b, scales_a, scales_b, out_dtype)
 
 
 def fp8_scaled_mm(mat_a, mat_b, scales_a, scales_b, out_dtype, bias=None):
+    out = native.rowcol_mm(mat_a, mat_b, scales_a, scales_b, out_dtype, bias, False, False)
+    if out is not None:
+        return out
     return torch.ops.sgl_kernel.fp8_scaled_mm.default(mat_a, mat_b, scales_a, scales_b, out_dtype, bias)
 
 
