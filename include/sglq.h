@@ -275,6 +275,17 @@ int sglq_fp8_blockwise_scaled_grouped_mm(const void* a, int64_t lda, const void*
                                          int64_t num_experts, int64_t total_m, int64_t N, int64_t K, void* workspace,
                                          int64_t workspace_bytes, void* stream);
 
+/* The row tile height that sglq_fp8_blockwise_scaled_grouped_mm takes for these sizes, and that entry point
+ * with a tile plan that is already there (sglq_prepare_moe_layer writes one): two GEMMs over the same groups
+ * share it where their heights agree. */
+int64_t sglq_grouped_plan_rows(int64_t num_experts, int64_t total_m, int64_t K);
+int sglq_fp8_blockwise_scaled_grouped_mm_planned(const void* a, int64_t lda, const void* b, int64_t ldb,
+                                                 int64_t b_expert_stride, const float* sfa, int64_t sfa_stride_m,
+                                                 int64_t sfa_stride_k, const float* sfb, int64_t sfb_expert_stride,
+                                                 int64_t sfb_stride_k, int64_t sfb_stride_n, void* out, int64_t ldo,
+                                                 int out_dtype, int64_t plan_rows, int64_t num_experts, int64_t total_m,
+                                                 int64_t N, int64_t K, void* plan, int64_t plan_bytes, void* stream);
+
 /* The data movement around the grouped GEMM in an MoE layer
  * (python/sglang/srt/layers/moe/cutlass_moe.py:140-222).
  *
@@ -304,11 +315,25 @@ int sglq_prepare_moe_input(const int32_t* topk_ids, int32_t* expert_offsets, int
                            int32_t* problem_sizes1, int32_t* problem_sizes2, int32_t* input_permutation,
                            int32_t* output_permutation, int64_t topk_length, int64_t topk, int64_t num_experts,
                            int64_t n, int64_t k, void* stream);
+/* One expert layer's tables in one launch, for callers that go on to the grouped GEMMs at once: what
+ * sglq_prepare_moe_input writes to expert_offsets, problem_sizes1/2 and output_permutation (ids outside
+ * [0, num_experts) get -1 there), and the tile plan that sglq_fp8_blockwise_scaled_grouped_mm_planned reads,
+ * for row tiles of plan_rows rows: 16 * (plan_max_tiles + 1) bytes, 16-byte aligned,
+ * plan_max_tiles = topk_length / plan_rows + num_experts.  Up to 32768 slots and 512 experts
+ * (SGLQ_EUNSUPPORTED above: call sglq_prepare_moe_input). */
+int sglq_prepare_moe_layer(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1,
+                           int32_t* problem_sizes2, int32_t* output_permutation, int64_t topk_length,
+                           int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows, int64_t plan_max_tiles,
+                           void* plan, void* stream);
 int sglq_shuffle_rows(const void* input, const int32_t* dst2src_map, void* output, int64_t num_src_rows,
                       int64_t num_dst_rows, int64_t row_bytes, void* stream);
 int sglq_silu_and_mul(const void* input, int dtype, void* output, int64_t num_tokens, int64_t d, void* stream);
 int sglq_apply_shuffle_mul_sum(const void* input, void* output, const int32_t* permutation, const void* factors,
                                int dtype, int64_t m, int64_t topk, int64_t row, int64_t num_src_rows, void* stream);
+
+/* ... with fp32 factors, rounded to dtype first (the caller's `topk_weights.to(out_dtype)`, cutlass_moe.py:222). */
+int sglq_apply_shuffle_mul_sum_f32(const void* input, void* output, const int32_t* permutation, const float* factors,
+                                   int dtype, int64_t m, int64_t topk, int64_t row, int64_t num_src_rows, void* stream);
 
 /* sgl_per_token_group_quant_fp8 with group 128 (per_token_group_quant_8bit.cu:72-113) followed by
  * the two shuffle_rows calls that replicate codes and scales into expert-major order

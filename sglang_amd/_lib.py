@@ -80,6 +80,12 @@ SIGNATURES = {
     "sglq_tuned_clear": [],
     "sglq_per_token_group_quant_fp8_scatter": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_float, c_void_p],
     "sglq_silu_and_mul_group_quant_fp8": [c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int64, c_float, c_void_p],
+    "sglq_prepare_moe_layer": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,
+                               c_void_p, c_void_p],
+    "sglq_fp8_blockwise_scaled_grouped_mm_planned": [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p,
+                                                     c_int64, c_int64, c_int64, c_void_p, c_int64, c_int, c_int64, c_int64, c_int64, c_int64,
+                                                     c_int64, c_void_p, c_int64, c_void_p],
+    "sglq_apply_shuffle_mul_sum_f32": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p],
     "sglq_apply_shuffle_mul_sum": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p],
     "sglq_int8_blockwise_scaled_mm": [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64,
                                       c_void_p, c_int64, c_int, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p],
@@ -110,6 +116,8 @@ def load() -> ctypes.CDLL:
         fn.restype = c_int
     lib.sglq_last_error.restype = c_char_p
     lib.sglq_last_error.argtypes = []
+    lib.sglq_grouped_plan_rows.argtypes = [c_int64, c_int64, c_int64]
+    lib.sglq_grouped_plan_rows.restype = c_int64
     lib.sglq_abi_version.restype = c_int
     lib.sglq_abi_version.argtypes = []
     lib.sglq_debug_set_direct_lds.argtypes = [c_int]

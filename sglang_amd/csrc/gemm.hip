@@ -3603,15 +3603,32 @@ extern "C" int sglq_fp8_blockwise_scaled_mm_bias(const void* a, int64_t lda, con
                                          workspace_bytes, stream);
 }
 
-extern "C" int sglq_fp8_blockwise_scaled_grouped_mm(const void* a, int64_t lda, const void* b, int64_t ldb,
-                                                    int64_t b_expert_stride, const float* sfa, int64_t sfa_stride_m,
-                                                    int64_t sfa_stride_k, const float* sfb, int64_t sfb_expert_stride,
-                                                    int64_t sfb_stride_k, int64_t sfb_stride_n, void* out, int64_t ldo,
-                                                    int out_dtype, const int32_t* problem_sizes,
-                                                    const int32_t* expert_offsets, int64_t num_experts, int64_t total_m,
-                                                    int64_t N, int64_t K, void* workspace, int64_t workspace_bytes,
-                                                    void* stream) {
-  using namespace sglq;
+// Row tile height from the average group: the experts' row counts are device data.
+// Measured with 256 experts of 4096 x 7168 (one launch streams every expert's weight once,
+// 7.5 GB) and equal groups: below about 12 rows per expert the 128-row kernel's 64-row tiles
+// are fastest (1.30-1.32 ms, 5.7-5.8 TB/s, against 1.43-1.45 ms); from there to 128 rows per
+// expert the pipelined kernel with 128-row tiles (1.46 ms at 16 rows, 1.57 ms at 64, 1.76 ms
+// at 128, where the unpipelined 128-row tiles need 1.48, 2.23 and 3.99 ms and the pipelined
+// 256-row ones 2.1-2.2 ms whatever their fill); above 128 rows per expert two 128-row tiles
+// cost what one 256-row tile costs and the 256-row tile computes faster (2.26 against
+// 2.51 ms at 256 rows, 7.7 against 8.1 ms at 1024).
+static int grouped_tile_rows(int64_t total_m, int64_t num_experts, int64_t K, bool& pipelined) {
+  const int64_t avg = total_m / num_experts;
+  if (g_grouped_tile) {  // test hook; 130 = the pipelined kernel with 128-row tiles
+    pipelined = g_grouped_tile == 256 || g_grouped_tile == 130;
+    return g_grouped_tile == 130 ? 128 : g_grouped_tile;
+  }
+  pipelined = avg >= 12 && K >= 384;
+  return pipelined ? (avg > 128 ? 256 : 128) : avg < 12 ? 64 : 128;
+}
+
+// `plan_rows` > 0: `workspace` already holds the tile plan for row tiles of that height
+// (sglq_grouped_plan_rows, sglq_prepare_moe_layer), and problem_sizes and expert_offsets are not read.
+static int grouped_entry(const void* a, int64_t lda, const void* b, int64_t ldb, int64_t b_expert_stride, const float* sfa,
+                         int64_t sfa_stride_m, int64_t sfa_stride_k, const float* sfb, int64_t sfb_expert_stride, int64_t sfb_stride_k,
+                         int64_t sfb_stride_n, void* out, int64_t ldo, int out_dtype, const int32_t* problem_sizes,
+                         const int32_t* expert_offsets, int64_t num_experts, int64_t total_m, int64_t N, int64_t K, void* workspace,
+                         int64_t workspace_bytes, int64_t plan_rows, void* stream) {
   const char* name = "fp8_blockwise_scaled_grouped_mm";
   if (num_experts < 0) {
     set_error("%s: negative number of experts", name);
@@ -3620,7 +3637,7 @@ extern "C" int sglq_fp8_blockwise_scaled_grouped_mm(const void* a, int64_t lda, 
   int rc = gemm_common_checks(name, a, lda, b, ldb, out, ldo, total_m, N, K, 2);
   if (rc < 0 || num_experts == 0) return SGLQ_OK;
   if (rc) return rc;
-  if (!sfa || !sfb || !problem_sizes || !expert_offsets) {
+  if (!sfa || !sfb || (plan_rows == 0 && (!problem_sizes || !expert_offsets))) {
     set_error("%s: null scale, problem_sizes or expert_offsets pointer", name);
     return SGLQ_EINVAL;
   }
@@ -3636,24 +3653,11 @@ extern "C" int sglq_fp8_blockwise_scaled_grouped_mm(const void* a, int64_t lda, 
     set_error("%s: the experts' weights must be 16-byte aligned, fewer than 2^20 experts", name);
     return SGLQ_EINVAL;
   }
-  // Row tile height from the average group: the experts' row counts are device data.
-  // Measured with 256 experts of 4096 x 7168 (one launch streams every expert's weight once,
-  // 7.5 GB) and equal groups: below about 12 rows per expert the 128-row kernel's 64-row tiles
-  // are fastest (1.30-1.32 ms, 5.7-5.8 TB/s, against 1.43-1.45 ms); from there to 128 rows per
-  // expert the pipelined kernel with 128-row tiles (1.46 ms at 16 rows, 1.57 ms at 64, 1.76 ms
-  // at 128, where the unpipelined 128-row tiles need 1.48, 2.23 and 3.99 ms and the pipelined
-  // 256-row ones 2.1-2.2 ms whatever their fill); above 128 rows per expert two 128-row tiles
-  // cost what one 256-row tile costs and the 256-row tile computes faster (2.26 against
-  // 2.51 ms at 256 rows, 7.7 against 8.1 ms at 1024).
-  const int64_t avg = total_m / num_experts;
   bool pipelined;
-  int bm;
-  if (g_grouped_tile) {  // test hook; 130 = the pipelined kernel with 128-row tiles
-    pipelined = g_grouped_tile == 256 || g_grouped_tile == 130;
-    bm = g_grouped_tile == 130 ? 128 : g_grouped_tile;
-  } else {
-    pipelined = avg >= 12 && K >= 384;
-    bm = pipelined ? (avg > 128 ? 256 : 128) : avg < 12 ? 64 : 128;
+  const int bm = grouped_tile_rows(total_m, num_experts, K, pipelined);
+  if (plan_rows != 0 && plan_rows != bm) {
+    set_error("%s: the plan is for row tiles of %lld, this call takes %d", name, (long long)plan_rows, bm);
+    return SGLQ_EINVAL;
   }
   if (pipelined && K < 384) {
     set_error("%s: the pipelined kernel needs K >= 384", name);
@@ -3683,8 +3687,9 @@ extern "C" int sglq_fp8_blockwise_scaled_grouped_mm(const void* a, int64_t lda, 
   p.num_experts = (int)num_experts;
   p.ws = workspace;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  grouped_plan_kernel<<<dim3(1), dim3(256), 0, st>>>(problem_sizes, expert_offsets, (int)num_experts, (int)total_m, bm,
-                                                     (int)max_tiles, static_cast<int*>(workspace));
+  if (plan_rows == 0)
+    grouped_plan_kernel<<<dim3(1), dim3(256), 0, st>>>(problem_sizes, expert_offsets, (int)num_experts, (int)total_m, bm,
+                                                       (int)max_tiles, static_cast<int*>(workspace));
   if (pipelined) {
     g_last_kernel = bm == 256 ? "grouped_plan_kernel+gemm_pipe_kernel<grouped>" : "grouped_plan_kernel+gemm_pipe_kernel<grouped, 128 rows>";
     p.tiles_m = (int)max_tiles;
@@ -3712,6 +3717,38 @@ extern "C" int sglq_fp8_blockwise_scaled_grouped_mm(const void* a, int64_t lda, 
     else launch_grouped_cfg<KIND_FP8_BLOCK, 128, 128, 2, 2, SGLQ_FP16>(p, (int)max_tiles, st);
   }
   return finish(name);
+}
+
+extern "C" int sglq_fp8_blockwise_scaled_grouped_mm(const void* a, int64_t lda, const void* b, int64_t ldb,
+                                                    int64_t b_expert_stride, const float* sfa, int64_t sfa_stride_m,
+                                                    int64_t sfa_stride_k, const float* sfb, int64_t sfb_expert_stride,
+                                                    int64_t sfb_stride_k, int64_t sfb_stride_n, void* out, int64_t ldo,
+                                                    int out_dtype, const int32_t* problem_sizes,
+                                                    const int32_t* expert_offsets, int64_t num_experts, int64_t total_m,
+                                                    int64_t N, int64_t K, void* workspace, int64_t workspace_bytes,
+                                                    void* stream) {
+  return grouped_entry(a, lda, b, ldb, b_expert_stride, sfa, sfa_stride_m, sfa_stride_k, sfb, sfb_expert_stride, sfb_stride_k, sfb_stride_n,
+                       out, ldo, out_dtype, problem_sizes, expert_offsets, num_experts, total_m, N, K, workspace, workspace_bytes, 0, stream);
+}
+
+extern "C" int64_t sglq_grouped_plan_rows(int64_t num_experts, int64_t total_m, int64_t K) {
+  bool pipelined;
+  return num_experts > 0 && total_m >= 0 ? grouped_tile_rows(total_m, num_experts, K, pipelined) : 0;
+}
+
+extern "C" int sglq_fp8_blockwise_scaled_grouped_mm_planned(const void* a, int64_t lda, const void* b, int64_t ldb,
+                                                            int64_t b_expert_stride, const float* sfa, int64_t sfa_stride_m,
+                                                            int64_t sfa_stride_k, const float* sfb, int64_t sfb_expert_stride,
+                                                            int64_t sfb_stride_k, int64_t sfb_stride_n, void* out, int64_t ldo,
+                                                            int out_dtype, int64_t plan_rows, int64_t num_experts,
+                                                            int64_t total_m, int64_t N, int64_t K, void* plan,
+                                                            int64_t plan_bytes, void* stream) {
+  if (plan_rows <= 0) {
+    set_error("fp8_blockwise_scaled_grouped_mm_planned: plan_rows must be what sglq_grouped_plan_rows returns");
+    return SGLQ_EINVAL;
+  }
+  return grouped_entry(a, lda, b, ldb, b_expert_stride, sfa, sfa_stride_m, sfa_stride_k, sfb, sfb_expert_stride, sfb_stride_k, sfb_stride_n,
+                       out, ldo, out_dtype, nullptr, nullptr, num_experts, total_m, N, K, plan, plan_bytes, plan_rows, stream);
 }
 
 extern "C" int sglq_int8_blockwise_scaled_mm(const void* a, int64_t lda, const void* b, int64_t ldb, const float* sfa,

@@ -23,6 +23,7 @@
 #include <ATen/core/grad_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/ops/add.h>
+#include <ATen/ops/fill.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -53,6 +54,15 @@ namespace {
   X(sglq_int8_blockwise_scaled_mm_bias)                                                                             \
   X(sglq_int8_scaled_mm)                                                                                            \
   X(sglq_fp8_scaled_mm)                                                                                             \
+  X(sglq_prepare_moe_input)                                                                                         \
+  X(sglq_prepare_moe_layer)                                                                                         \
+  X(sglq_grouped_plan_rows)                                                                                         \
+  X(sglq_fp8_blockwise_scaled_grouped_mm)                                                                           \
+  X(sglq_fp8_blockwise_scaled_grouped_mm_planned)                                                                   \
+  X(sglq_per_token_group_quant_fp8_scatter)                                                                         \
+  X(sglq_silu_and_mul_group_quant_fp8)                                                                              \
+  X(sglq_apply_shuffle_mul_sum)                                                                                     \
+  X(sglq_apply_shuffle_mul_sum_f32)                                                                                 \
   X(sglq_w8a8_block_fp8_linear)                                                                                     \
   X(sglq_w8a8_int8_linear)                                                                                          \
   X(sglq_w8a8_fp8_linear)
@@ -531,6 +541,101 @@ PyObject* token_quant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 }
 
 // ---------------------------------------------------------------------------
+// experts(a, w1_q, w2_q, w1_scale, w2_scale, topk_weights, topk_ids, expert_offsets, problem_sizes1,
+// problem_sizes2) -> [m, k]: cutlass_fused_experts_fp8 (moe/cutlass_moe.py) as six launches where the tables
+// fit one block (prepare, quantize to expert rows, GEMM, SiLU and quantize, GEMM, combine) from twelve, and
+// one allocation beside the result's from eleven: a layer of a few tokens was bound by about 95 us of host
+// time around 30-50 us of GPU work.
+// ---------------------------------------------------------------------------
+inline bool int32_buffer(const Tensor& t, int64_t count, const Tensor& like) {
+  return t.scalar_type() == at::kInt && t.is_contiguous() && t.numel() >= count && t.device() == like.device();
+}
+inline bool expert_weight(const Tensor& w, int64_t e, int64_t k, int64_t n, const Tensor& scale, const Tensor& like) {
+  return w.dim() == 3 && w.scalar_type() == FP8 && w.size(0) == e && w.size(1) == k && w.size(2) == n && w.stride(1) == 1 &&
+         w.stride(2) % 16 == 0 && w.stride(2) >= k && w.stride(0) % 16 == 0 && aligned(w, 16) && w.device() == like.device() &&
+         scale.dim() == 3 && scale.scalar_type() == at::kFloat && scale.size(0) == e && scale.size(1) == (k + 127) / 128 &&
+         scale.size(2) == (n + 127) / 128 && scale.device() == like.device();
+}
+
+PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 10) return PyErr_Format(PyExc_TypeError, "experts takes 10 arguments");
+  return guarded([&]() -> PyObject* {
+    const Tensor* t[10];
+    for (int i = 0; i < 10; ++i) {
+      t[i] = gpu_tensor(args[i]);
+      if (!t[i]) return none();
+    }
+    const Tensor &x = *t[0], &w1 = *t[1], &w2 = *t[2], &s1 = *t[3], &s2 = *t[4], &weights = *t[5], &ids = *t[6], &offsets = *t[7],
+                 &sizes1 = *t[8], &sizes2 = *t[9];
+    if (!direct(x, w1, w2, s1, s2, weights)) return none();
+    if (!activations(x) || x.dim() != 2 || w1.dim() != 3 || w2.dim() != 3 || ids.dim() != 2 || weights.dim() != 2) return none();
+    const int64_t m = x.size(0), k = x.size(1), e = w1.size(0), n = w2.size(1), topk = ids.size(1), rows = m * topk;
+    if (e == 0 || n == 0 || topk == 0 || k % 128 != 0 || n % 128 != 0 || ids.size(0) != m || rows >= (int64_t(1) << 31)) return none();
+    if (!expert_weight(w1, e, k, 2 * n, s1, x) || !expert_weight(w2, e, n, k, s2, x)) return none();
+    const bool float_weights = weights.scalar_type() == at::kFloat;
+    if ((!float_weights && weights.scalar_type() != x.scalar_type()) || !weights.is_contiguous() || weights.size(0) != m ||
+        weights.size(1) != topk || weights.device() != x.device())
+      return none();
+    if (!int32_buffer(ids, rows, x) || !int32_buffer(offsets, e + 1, x) || !int32_buffer(sizes1, 3 * e, x) || !int32_buffer(sizes2, 3 * e, x))
+      return none();
+    const int code = dtype_code(x.scalar_type());
+    const int64_t plan_rows = lib.sglq_grouped_plan_rows(e, rows, k), plan_rows2 = lib.sglq_grouped_plan_rows(e, rows, n);
+    const bool one_block = rows <= 32768 && e <= 512;
+    const bool shared_plan = one_block && plan_rows == plan_rows2;
+    const int64_t plan_bytes = round256(16 * (rows / 16 + e + 1));
+    // expert-major rows: quantized activations (dead once GEMM 1 has run) under GEMM 2's output, GEMM 1's
+    // output, the quantized intermediate
+    const int64_t codes1 = round256(rows * k), scales1 = round256(rows * (k / 128) * 4), c2 = round256(rows * k * 2);
+    const int64_t c1 = round256(rows * 2 * n * 2), codes2 = round256(rows * n), scales2 = round256(rows * (n / 128) * 4);
+    const int64_t head = codes1 + scales1 > c2 ? codes1 + scales1 : c2, map = round256(rows * 4);
+    Tensor out;
+    int rc;
+    {
+      ReleaseGil unlocked;
+      Launch here(x.device());
+      out = empty({m, k}, x.scalar_type(), here.device);
+      Tensor arena = empty({head + c1 + codes2 + scales2 + plan_bytes + map + (one_block ? 0 : map)}, at::kByte, here.device);
+      char* base = static_cast<char*>(arena.data_ptr());
+      char *q1 = base, *y1 = base + head, *q2 = y1 + c1, *plan = q2 + codes2 + scales2;
+      float *f1 = reinterpret_cast<float*>(q1 + codes1), *f2 = reinterpret_cast<float*>(q2 + codes2);
+      int32_t* slot_map = reinterpret_cast<int32_t*>(plan + plan_bytes);
+      const int32_t* ids_p = static_cast<const int32_t*>(ids.data_ptr());
+      int32_t *off_p = static_cast<int32_t*>(offsets.data_ptr()), *ps1 = static_cast<int32_t*>(sizes1.data_ptr()),
+              *ps2 = static_cast<int32_t*>(sizes2.data_ptr());
+      if (one_block) {
+        rc = lib.sglq_prepare_moe_layer(ids_p, off_p, ps1, ps2, slot_map, rows, e, n, k, plan_rows, rows / plan_rows + e, plan, here.stream);
+      } else {
+        at::NoGradGuard no_grad;
+        arena.narrow(0, reinterpret_cast<char*>(slot_map) - base, rows * 4).fill_(255);  // -1: slots routed to nobody
+        rc = lib.sglq_prepare_moe_input(ids_p, off_p, nullptr, ps1, ps2, reinterpret_cast<int32_t*>(plan + plan_bytes + map), slot_map, rows,
+                                        topk, e, n, k, here.stream);
+      }
+      auto grouped = [&](const void* q, const float* f, const Tensor& w, const Tensor& s, void* y, const int32_t* sizes, int64_t depth,
+                         int64_t width, int64_t tile_rows, bool planned) {
+        const float* s_p = static_cast<const float*>(s.data_ptr());
+        const int64_t ldb = w.stride(2), bs = e > 1 ? w.stride(0) : width * depth;
+        return planned ? lib.sglq_fp8_blockwise_scaled_grouped_mm_planned(q, depth, w.data_ptr(), ldb, bs, f, depth / 128, 1, s_p, s.stride(0),
+                                                                          s.stride(1), s.stride(2), y, width, code, tile_rows, e, rows, width,
+                                                                          depth, plan, plan_bytes, here.stream)
+                       : lib.sglq_fp8_blockwise_scaled_grouped_mm(q, depth, w.data_ptr(), ldb, bs, f, depth / 128, 1, s_p, s.stride(0),
+                                                                  s.stride(1), s.stride(2), y, width, code, sizes, off_p, e, rows, width, depth,
+                                                                  plan, plan_bytes, here.stream);
+      };
+      if (rc == 0) rc = lib.sglq_per_token_group_quant_fp8_scatter(x.data_ptr(), code, q1, f1, slot_map, m, k, topk, rows, 1e-10f, here.stream);
+      if (rc == 0) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, one_block);
+      if (rc == 0) rc = lib.sglq_silu_and_mul_group_quant_fp8(y1, code, q2, f2, rows, n, 1e-10f, here.stream);
+      if (rc == 0) rc = grouped(q2, f2, w2, s2, base, ps2, n, k, plan_rows2, shared_plan);
+      if (rc == 0 && float_weights)
+        rc = lib.sglq_apply_shuffle_mul_sum_f32(base, out.data_ptr(), slot_map, static_cast<const float*>(weights.data_ptr()), code, m, topk, k,
+                                                rows, here.stream);
+      else if (rc == 0)
+        rc = lib.sglq_apply_shuffle_mul_sum(base, out.data_ptr(), slot_map, weights.data_ptr(), code, m, topk, k, rows, here.stream);
+    }
+    return rc == 0 ? THPVariable_Wrap(std::move(out)) : none();
+  });
+}
+
+// ---------------------------------------------------------------------------
 // bind({name: address}); release_workspaces()
 // ---------------------------------------------------------------------------
 PyObject* bind(PyObject*, PyObject* table) {
@@ -590,6 +695,7 @@ PyMethodDef methods[] = {
     {"rowcol_mm", FAST(rowcol_mm), "per-token / per-channel-scaled GEMM, or None"},
     {"group_quant_fp8", FAST(group_quant_fp8), "per-token-group FP8 quantization, or None"},
     {"token_quant", FAST(token_quant), "per-token quantization, or None"},
+    {"experts", FAST(experts), "an expert layer, or None"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "Host path of the per-layer operators", -1, methods, nullptr, nullptr, nullptr, nullptr};

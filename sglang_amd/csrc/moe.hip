@@ -1,6 +1,8 @@
 // The data movement around the grouped (MoE) block-scaled FP8 GEMM on gfx950: routing
 // tables from the top-k expert ids, row gathers into expert-major order, SiLU-and-multiply
 // between the two GEMMs, and the weighted combine back to token order.  All HBM-bound.
+#include <type_traits>
+
 #include "sglq_common.h"
 
 namespace sglq {
@@ -171,6 +173,113 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_place_kernel(const int* __res
 }
 
 // ---------------------------------------------------------------------------
+// The same tables, the -1 default of output_permutation and the grouped GEMMs' tile plan from one block,
+// for up to 32768 slots and 512 experts.  A decode step's layer is a chain of short dependent launches,
+// each of 2-5 us whatever it does (16 tokens, 32 experts: the fill of c_map, the three launches above and
+// two plan launches were 28 of the layer's 273 us); one block does their work in one of them.
+// Sixteen waves take consecutive ranges of slots and keep their ids in registers; counts per (wave, expert)
+// through LDS atomics (sums: the order does not matter), a running sum over waves and experts, then every
+// wave walks its slots again in order: lanes that name the same expert find each other with one ballot per
+// id bit, so positions follow slot order as above.
+// ---------------------------------------------------------------------------
+constexpr int TABLE_THREADS = 1024, TABLE_WAVES = TABLE_THREADS / 64, TABLE_STEPS = 32;
+constexpr int TABLE_MAX_SLOTS = TABLE_THREADS * TABLE_STEPS, TABLE_MAX_EXPERTS = 512;
+
+__global__ __launch_bounds__(TABLE_THREADS) void moe_tables_kernel(const int* __restrict__ topk_ids, int* __restrict__ expert_offsets,
+                                                                   int* __restrict__ ps1, int* __restrict__ ps2,
+                                                                   int* __restrict__ output_permutation, int topk_length,
+                                                                   int num_experts, int id_bits, int n, int k, int* __restrict__ plan,
+                                                                   int plan_rows, int plan_max_tiles) {
+  extern __shared__ int counts[];  // [TABLE_WAVES][num_experts]: first the counts, then the next position of each
+  __shared__ int wave_rows[TABLE_WAVES], wave_tiles[TABLE_WAVES];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int steps = (topk_length + TABLE_THREADS - 1) / TABLE_THREADS;  // 64 slots each, per wave
+  const int first = wave * steps * 64;
+  int id[TABLE_STEPS];
+#pragma unroll
+  for (int s = 0; s < TABLE_STEPS; ++s) {
+    const int i = first + s * 64 + lane;
+    id[s] = s < steps && i < topk_length ? topk_ids[i] : -1;
+  }
+  for (int i = tid; i < TABLE_WAVES * num_experts; i += TABLE_THREADS) counts[i] = 0;
+  __syncthreads();
+  int* mine = counts + wave * num_experts;
+#pragma unroll
+  for (int s = 0; s < TABLE_STEPS; ++s)
+    if ((uint32_t)id[s] < (uint32_t)num_experts) atomicAdd(mine + id[s], 1);
+  __syncthreads();
+  // one thread per expert (num_experts <= 512): rows and tiles, then their running sums over the block
+  int rows = 0, tiles = 0;
+  if (tid < num_experts) {
+#pragma unroll
+    for (int w = 0; w < TABLE_WAVES; ++w) {
+      const int c = counts[w * num_experts + tid];
+      counts[w * num_experts + tid] = rows;  // this expert's slots in earlier waves
+      rows += c;
+    }
+    tiles = (rows + plan_rows - 1) / plan_rows;
+  }
+  int row_sum = rows, tile_sum = tiles;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int r = __shfl_up(row_sum, d), t = __shfl_up(tile_sum, d);
+    row_sum += lane >= d ? r : 0;
+    tile_sum += lane >= d ? t : 0;
+  }
+  if (lane == 63) {
+    wave_rows[wave] = row_sum;
+    wave_tiles[wave] = tile_sum;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < TABLE_WAVES; ++w) {
+    row_sum += w < wave ? wave_rows[w] : 0;
+    tile_sum += w < wave ? wave_tiles[w] : 0;
+  }
+  if (tid < num_experts) {
+    const int begin = row_sum - rows;
+    if (tid == 0) expert_offsets[0] = 0;
+    expert_offsets[tid + 1] = row_sum;
+    ps1[3 * tid] = rows;
+    ps1[3 * tid + 1] = 2 * n;
+    ps1[3 * tid + 2] = k;
+    ps2[3 * tid] = rows;
+    ps2[3 * tid + 1] = k;
+    ps2[3 * tid + 2] = n;
+#pragma unroll
+    for (int w = 0; w < TABLE_WAVES; ++w) counts[w * num_experts + tid] += begin;
+    // (the layout grouped_plan_kernel writes: expert, first row, end row)
+    for (int i = 0, slot = tile_sum - tiles; i < tiles && slot < plan_max_tiles; ++i, ++slot)
+      reinterpret_cast<v4i*>(plan)[1 + slot] = v4i{tid, begin + i * plan_rows, row_sum, 0};
+    if (tid == num_experts - 1) plan[0] = tile_sum < plan_max_tiles ? tile_sum : plan_max_tiles;
+  }
+  __syncthreads();
+  const uint64_t below = (1ull << lane) - 1ull;
+#pragma unroll
+  for (int s = 0; s < TABLE_STEPS; ++s) {
+    if (s >= steps) break;
+    const int e = id[s];
+    const bool live = (uint32_t)e < (uint32_t)num_experts;
+    uint64_t same = __ballot(live);
+    for (int b = 0; b < id_bits; ++b) {
+      const uint64_t set = __ballot((e >> b) & 1);
+      same &= ((e >> b) & 1) ? set : ~set;
+    }
+    const int i = first + s * 64 + lane;
+    int pos = -1;
+    if (live) {
+      const int rank = __popcll(same & below);
+      pos = mine[e] + rank;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (live && (same & below) == 0) mine[e] += __popcll(same);  // (the wave's LDS operations run in this order)
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (i < topk_length) output_permutation[i] = pos;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // shuffle_rows (prepare_moe_input.cu:168-244): output[d] = input[dst2src_map[d]], rows of
 // row_bytes bytes.  16-byte pieces when rows and pointers allow, 4-byte or single bytes
 // otherwise; a linear walk over (row, piece) pairs, so short rows (the 224-byte scale rows)
@@ -235,12 +344,18 @@ __global__ __launch_bounds__(256) void silu_and_mul_scalar_kernel(const uint16_t
 // with one fused multiply-add per term (:293-295), rounded once to the 16-bit type.
 // A lane owns 8 consecutive elements of one output row; lanes walk (row, chunk) pairs linearly,
 // so rows of any length fill the waves.
+// FACTOR = float: the factors as the router leaves them, rounded to the 16-bit type here instead of by
+// a conversion kernel in front (one launch of a decode step's chain).
 // ---------------------------------------------------------------------------
-template <int DT>
+template <int DT, typename FACTOR = uint16_t>
 __global__ __launch_bounds__(256) void shuffle_mul_sum_kernel(const uint16_t* __restrict__ in, uint16_t* __restrict__ out,
                                                               const int* __restrict__ perm,
-                                                              const uint16_t* __restrict__ factors, int64_t m, int topk,
+                                                              const FACTOR* __restrict__ factors, int64_t m, int topk,
                                                               int64_t row, int64_t num_src_rows) {
+  auto factor = [&](int64_t slot) -> float {
+    if constexpr (std::is_same<FACTOR, float>::value) return to_f32_16<DT>(from_f32_16<DT>(factors[slot]));
+    else return to_f32_16<DT>(factors[slot]);
+  };
   const int64_t cpr = row >> 3;  // chunks per row
   const int64_t total = m * cpr;
   for (int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x; id < total; id += (int64_t)gridDim.x * 256) {
@@ -258,7 +373,7 @@ __global__ __launch_bounds__(256) void shuffle_mul_sum_kernel(const uint16_t* __
       for (int u = 0; u < 8; ++u) {
         const int64_t slot = i * topk + (j0 + u < topk ? j0 + u : topk - 1);
         src[u] = perm[slot];
-        f[u] = factors ? to_f32_16<DT>(factors[slot]) : 1.0f;
+        f[u] = factors ? factor(slot) : 1.0f;
       }
       v4u v[8];
 #pragma unroll
@@ -318,6 +433,32 @@ extern "C" int sglq_prepare_moe_input(const int32_t* topk_ids, int32_t* expert_o
     moe_place_kernel<<<dim3((uint32_t)num_experts, (uint32_t)parts), dim3(MOE_THREADS), 0, st>>>(
         topk_ids, expert_offsets, input_permutation, output_permutation, topk_length, (int)topk, span, aligned);
   }
+  return check_moe_launch(name);
+}
+
+extern "C" int sglq_prepare_moe_layer(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1,
+                                      int32_t* problem_sizes2, int32_t* output_permutation, int64_t topk_length,
+                                      int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows, int64_t plan_max_tiles,
+                                      void* plan, void* stream) {
+  const char* name = "prepare_moe_layer";
+  if (topk_length <= 0 || num_experts <= 0 || n < 0 || k < 0 || n >= (1ll << 30) || k >= (1ll << 31) || plan_rows <= 0 ||
+      plan_max_tiles <= 0 || plan_max_tiles >= (1ll << 27)) {
+    set_error("%s: bad sizes", name);
+    return SGLQ_EINVAL;
+  }
+  if (topk_length > TABLE_MAX_SLOTS || num_experts > TABLE_MAX_EXPERTS) {
+    set_error("%s: up to %d slots and %d experts (larger layers: sglq_prepare_moe_input)", name, TABLE_MAX_SLOTS, TABLE_MAX_EXPERTS);
+    return SGLQ_EUNSUPPORTED;
+  }
+  if (!topk_ids || !expert_offsets || !problem_sizes1 || !problem_sizes2 || !output_permutation || !plan ||
+      (reinterpret_cast<uintptr_t>(plan) & 15)) {
+    set_error("%s: null pointer, or a plan that is not 16-byte aligned", name);
+    return SGLQ_EINVAL;
+  }
+  int id_bits = 0;
+  while ((1 << id_bits) < num_experts) ++id_bits;
+  moe_tables_kernel<<<dim3(1), dim3(TABLE_THREADS), (size_t)TABLE_WAVES * num_experts * sizeof(int), static_cast<hipStream_t>(stream)>>>(
+      topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, (int)topk_length, (int)num_experts, id_bits, (int)n, (int)k, static_cast<int*>(plan), (int)plan_rows, (int)plan_max_tiles);
   return check_moe_launch(name);
 }
 
@@ -381,9 +522,8 @@ extern "C" int sglq_silu_and_mul(const void* input, int dtype, void* output, int
   return check_moe_launch(name);
 }
 
-extern "C" int sglq_apply_shuffle_mul_sum(const void* input, void* output, const int32_t* permutation, const void* factors,
-                                          int dtype, int64_t m, int64_t topk, int64_t row, int64_t num_src_rows,
-                                          void* stream) {
+static int shuffle_mul_sum_entry(const void* input, void* output, const int32_t* permutation, const void* factors, bool f32_factors,
+                                 int dtype, int64_t m, int64_t topk, int64_t row, int64_t num_src_rows, void* stream) {
   const char* name = "apply_shuffle_mul_sum";
   if (m < 0 || topk <= 0 || row < 0 || num_src_rows < 0 || topk >= (1 << 20) || m >= (1ll << 31)) {
     set_error("%s: bad sizes", name);
@@ -408,12 +548,29 @@ extern "C" int sglq_apply_shuffle_mul_sum(const void* input, void* output, const
   const dim3 grid((uint32_t)blocks), block(256);
   const uint16_t* in = static_cast<const uint16_t*>(input);
   uint16_t* out = static_cast<uint16_t*>(output);
-  const uint16_t* f = static_cast<const uint16_t*>(factors);
-  if (dtype == SGLQ_BF16) shuffle_mul_sum_kernel<SGLQ_BF16><<<grid, block, 0, st>>>(in, out, permutation, f, m, (int)topk, row, num_src_rows);
-  else if (dtype == SGLQ_FP16) shuffle_mul_sum_kernel<SGLQ_FP16><<<grid, block, 0, st>>>(in, out, permutation, f, m, (int)topk, row, num_src_rows);
+#define SGLQ_COMBINE(DT, F)                                                                                                   \
+  shuffle_mul_sum_kernel<DT, F><<<grid, block, 0, st>>>(in, out, permutation, static_cast<const F*>(factors), m, (int)topk, row, \
+                                                        num_src_rows)
+  if (dtype == SGLQ_BF16 && f32_factors) SGLQ_COMBINE(SGLQ_BF16, float);
+  else if (dtype == SGLQ_BF16) SGLQ_COMBINE(SGLQ_BF16, uint16_t);
+  else if (dtype == SGLQ_FP16 && f32_factors) SGLQ_COMBINE(SGLQ_FP16, float);
+  else if (dtype == SGLQ_FP16) SGLQ_COMBINE(SGLQ_FP16, uint16_t);
+#undef SGLQ_COMBINE
   else {
     set_error("%s: dtype must be Half or BFloat16", name);
     return SGLQ_EUNSUPPORTED;
   }
   return check_moe_launch(name);
+}
+
+extern "C" int sglq_apply_shuffle_mul_sum(const void* input, void* output, const int32_t* permutation, const void* factors,
+                                          int dtype, int64_t m, int64_t topk, int64_t row, int64_t num_src_rows,
+                                          void* stream) {
+  return shuffle_mul_sum_entry(input, output, permutation, factors, false, dtype, m, topk, row, num_src_rows, stream);
+}
+
+extern "C" int sglq_apply_shuffle_mul_sum_f32(const void* input, void* output, const int32_t* permutation, const float* factors,
+                                              int dtype, int64_t m, int64_t topk, int64_t row, int64_t num_src_rows,
+                                              void* stream) {
+  return shuffle_mul_sum_entry(input, output, permutation, factors, true, dtype, m, topk, row, num_src_rows, stream);
 }
