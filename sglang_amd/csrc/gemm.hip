@@ -3263,12 +3263,19 @@ struct TunedEntry {
 constexpr int MAX_TUNED = 1024;
 static TunedEntry g_tuned[MAX_TUNED];
 static int g_num_tuned = 0;
+// entries of one (kind, N, K) are chained from a bucket (the shipped tables are some 600 entries: a walk over all of
+// them cost every call about a microsecond), in the order they were added
+constexpr int TUNED_BUCKETS = 512;
+static int16_t g_tuned_head[TUNED_BUCKETS], g_tuned_tail[TUNED_BUCKETS], g_tuned_next[MAX_TUNED];  // index + 1, 0 = none
 static std::shared_mutex g_tuned_lock;
+static uint32_t tuned_bucket(int kind, int64_t n, int64_t k) {
+  return (uint32_t)(((uint64_t)n * 0x9e3779b97f4a7c15ull + (uint64_t)k * 0xc2b2ae3d27d4eb4full + (uint64_t)kind) >> 40) % TUNED_BUCKETS;
+}
 
 static bool tuned_lookup(int kind, int64_t m, int64_t n, int64_t k, int& tile, int& splits) {
   std::shared_lock<std::shared_mutex> guard(g_tuned_lock);
-  for (int i = 0; i < g_num_tuned; ++i) {
-    const TunedEntry& e = g_tuned[i];
+  for (int i = g_tuned_head[tuned_bucket(kind, n, k)]; i > 0; i = g_tuned_next[i - 1]) {
+    const TunedEntry& e = g_tuned[i - 1];
     if (e.kind == kind && e.n == n && e.k == k && m >= e.m_lo && m <= e.m_hi) {
       tile = e.tile;
       splits = e.splits;
@@ -3486,6 +3493,7 @@ extern "C" void sglq_debug_force_splits(int splits) { g_force_splits = splits; }
 extern "C" int sglq_tuned_clear(void) {
   std::unique_lock<std::shared_mutex> guard(g_tuned_lock);
   g_num_tuned = 0;
+  for (int i = 0; i < TUNED_BUCKETS; ++i) g_tuned_head[i] = g_tuned_tail[i] = 0;
   return SGLQ_OK;
 }
 extern "C" int sglq_tuned_add(int kind, int64_t N, int64_t K, int64_t m_lo, int64_t m_hi, int tile, int splits) {
@@ -3502,6 +3510,11 @@ extern "C" int sglq_tuned_add(int kind, int64_t N, int64_t K, int64_t m_lo, int6
     return SGLQ_EUNSUPPORTED;
   }
   g_tuned[g_num_tuned++] = TunedEntry{kind, N, K, m_lo, m_hi, tile, splits};
+  const uint32_t bucket = tuned_bucket(kind, N, K);
+  g_tuned_next[g_num_tuned - 1] = 0;
+  if (g_tuned_tail[bucket]) g_tuned_next[g_tuned_tail[bucket] - 1] = (int16_t)g_num_tuned;
+  else g_tuned_head[bucket] = (int16_t)g_num_tuned;
+  g_tuned_tail[bucket] = (int16_t)g_num_tuned;
   return SGLQ_OK;
 }
 
@@ -3917,7 +3930,13 @@ extern "C" int sglq_w8a8_block_fp8_linear(const void* x, int in_dtype, const voi
     // and from 5 rows on it loses nearly everywhere (8 x 4096 x 7168: 9.2 -> 10.1 us).  A forced 16- or 32-row
     // block (test hook) takes the single kernel for any M <= 8.
     const int blocks = nib > 0 ? (int)((N + 16 * nib - 1) / (16 * nib)) : 0;
-    const bool pays = g_force_tile != 0 || (M <= 4 && blocks >= num_cus() && 2 * blocks <= 5 * num_cus());
+    // On K <= 4096 the single kernel wins with fewer blocks as well, by the launch it saves (2.4-3.5 us for a program
+    // that launches call by call, 1.6 us in a graph): up to 4 rows, and 5 to 8 rows where the repeated arithmetic stays
+    // small, M K <= 8192 or N <= 4096 (call by call / in a graph: 1 x 1600 x 1024 7.7 -> 4.4 / 4.8 -> 3.4 us,
+    // 6 x 17920 x 768 7.9 -> 6.5 / 7.9 -> 7.0, 8 x 4096 x 4096 7.5 -> 6.5 / 8.2 -> 7.1; but 8 x 512 x 8192 7.6 -> 9.5 / 7.9 -> 9.8).
+    const bool one_round = M <= 4 && blocks >= num_cus() && 2 * blocks <= 5 * num_cus();
+    const bool short_k = K <= 4096 && N >= 1024 && (M <= 4 ? 2 * blocks <= 5 * num_cus() : (M * K <= 8192 || N <= 4096));
+    const bool pays = g_force_tile != 0 || one_round || short_k;
     if (nib > 0 && pays) {
       p.lda = (uint32_t)(K * 2);  // row stride of the 16-bit activations in bytes
       p.a_bytes = (uint32_t)(M * K * 2);
@@ -4021,7 +4040,10 @@ static int tokenquant_linear_entry(const char* name, const void* x, int in_dtype
     // Every block reads the M rows once more for their maxima (M K 2 bytes from L2 per block) before its first
     // MFMA; against that stand the quantization launch (2.4-2.8 us) and the codes' round trip.  A forced 16- or
     // 32-row block (test hook) takes the single kernel for any M <= 8.
-    const bool pays = g_force_tile != 0 || M <= SGLQ_TOKENQUANT_FUSED_ROWS;
+    // From 3 rows on only where the call is short enough for the launch it saves to weigh more than the arithmetic that
+    // every block repeats: M K <= 8192 on N <= 4096 (call by call / in a graph: 4 x 2048 x 768 7.1 -> 4.4 / 5.2 -> 4.6 us,
+    // 8 x 1024 x 1024 7.5 -> 5.2 / 5.3 -> 5.7).
+    const bool pays = g_force_tile != 0 || M <= SGLQ_TOKENQUANT_FUSED_ROWS || (M * K <= 8192 && N <= 4096);
     if (nib > 0 && pays) {
       p.lda = (uint32_t)(K * 2);  // row stride of the 16-bit activations in bytes
       p.a_bytes = (uint32_t)(M * K * 2);
