@@ -22,7 +22,8 @@ CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libsglq.so"
 BENCH_LIB_PATH = PKG_DIR / "libsglq_bench.so"
 NATIVE_PATH = PKG_DIR / "_native.so"
-SOURCES = ["common.hip", "quant.hip", "moe.hip", "gemm.hip"]
+SOURCES = ["gemm.hip", "gemm_ring_fp8_block.hip", "gemm_ring_fp8_block_pow2.hip", "gemm_ring_fp8_rowcol.hip", "gemm_ring_i8_rowcol.hip",
+           "gemm_ring_i8_block.hip", "common.hip", "quant.hip", "moe.hip"]
 BENCH_SOURCES = ["bench_kernels.hip"]
 
 HIPCC_FLAGS = [
@@ -71,7 +72,7 @@ def build_native(verbose: bool = False) -> Path:
     return NATIVE_PATH
 
 
-def build(verbose: bool = False, jobs: int = 4) -> Path:
+def build(verbose: bool = False, jobs: int = 8) -> Path:
     hipcc = find_hipcc()
     obj_dir = PKG_DIR / "build"
     obj_dir.mkdir(exist_ok=True)

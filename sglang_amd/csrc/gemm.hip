@@ -24,274 +24,12 @@
 #include <shared_mutex>
 #include <type_traits>
 
+#include "gemm_device.h"
+#include "gemm_ring.h"
 #include "quant_device.h"
 #include "sglq_common.h"
 
 namespace sglq {
-
-constexpr int KIND_FP8_BLOCK = 0;   // a4: sum_kb P_kb * sfa[m,kb] * sfb[kb,n/128]
-constexpr int KIND_FP8_ROWCOL = 1;  // a6: sa[m] * (sb[n] * acc) + bias[n]
-constexpr int KIND_I8_ROWCOL = 2;   // a5: float(acc) * (sb[n] * sa[m]) + bias[n]
-constexpr int KIND_I8_RAW = 3;      // INT32 accumulators
-constexpr int KIND_I8_BLOCK = 4;    // block-scaled INT8: sum_kb float(P_kb) * sfa[m,kb] * sfb[kb,n/128]
-// KIND_FP8_BLOCK whose scales are all powers of two (UE8M0 values held as fp32): the MFMA applies them itself
-// (v_mfma_scale_f32_16x16x128_f8f6f4 takes an exponent byte per lane for each operand) and accumulates in place,
-// so there is no scale-and-accumulate pass behind every MFMA.  Only the 256- and 128-row pipelined kernels are
-// built for it; everywhere else such scales run as KIND_FP8_BLOCK (the same sums folded per K block: equal to the
-// in-place accumulation up to the order of the additions, not bit for bit).
-constexpr int KIND_FP8_BLOCK_POW2 = 5;
-
-constexpr bool is_block(int kind) { return kind == KIND_FP8_BLOCK || kind == KIND_I8_BLOCK || kind == KIND_FP8_BLOCK_POW2; }
-constexpr bool fp8_operands(int kind) { return kind == KIND_FP8_BLOCK || kind == KIND_FP8_ROWCOL || kind == KIND_FP8_BLOCK_POW2; }
-// the biased exponent of a positive power of two = its UE8M0 code, in byte 0 as the scaled MFMA reads it
-SGLQ_DEV int ue8m0_of(float pow2) { return (int)(__builtin_bit_cast(uint32_t, pow2) >> 23); }
-// ... of an activation scale as the kernels hold it: the eight bits from `shift` on, 23 for an fp32 power of two, 8 (kb % 4)
-// for a word of four UE8M0 codes (GemmArgs::sa_packed) and K block kb
-SGLQ_DEV int ue8m0_at(float word, int shift) { return (int)((__builtin_bit_cast(uint32_t, word) >> shift) & 0xffu); }
-constexpr bool float_acc(int kind) { return fp8_operands(kind) || kind == KIND_I8_BLOCK; }
-
-constexpr uint32_t OOB = 0x80000000u;  // offset beyond any buffer this library accepts
-constexpr uint32_t SC_NONE = 0x40000000u;  // scalar offset beyond any scale tensor (at most 2^31 / 32 bytes)
-
-struct GemmArgs {
-  const char* a;   // [M, K] bytes, row stride lda
-  const char* b;   // [N, K] bytes, row stride ldb (column-major [K, N])
-  const float* sa; // block: sfa; rowcol: scales_a [M]
-  const float* sb; // block: sfb; rowcol: scales_b [N]
-  const void* bias;
-  void* out;
-  int64_t sa_stride_m, sa_stride_k;  // block scales
-  int64_t sb_stride_k, sb_stride_n;
-  int64_t ldo;
-  uint32_t lda, ldb;
-  uint32_t a_bytes, b_bytes;
-  int M, N, K;
-  int tiles_m, tiles_n;
-  void* ws;        // split-K partial sums [splits][M][N], fp32 or int32; grouped GEMM: the tile plan
-  int splits;
-  int64_t b_expert_stride, sb_expert_stride;  // grouped GEMM: bytes / floats between experts' weights / weight scales
-  int num_experts;
-  int stream_out;  // the output is larger than the last-level cache: store it with the non-temporal hint
-  int pow2_scales;  // block-scaled FP8: every scale is a power of two (KIND_FP8_BLOCK_POW2 where it is built)
-  // ... and the activation scales come as UE8M0 codes, four K blocks to an int32 word: word (m, kb / 4) sits at
-  // sa[m * sa_stride_m + (kb / 4) * sa_stride_k], byte kb % 4 of it is K block kb's code (what
-  // sglq_per_token_group_quant_fp8_ue8m0 writes).  Read as they are by the KIND_FP8_BLOCK_POW2 kernels; every
-  // other kernel gets them expanded to fp32 first (expand_packed_scales).
-  int sa_packed;
-  float* sa_expanded;  // room for [M, K / 128] fp32 scales (sa_packed only)
-  float quant_eps;  // fused quantization (gemm_stream_quant_kernel): lower bound of a group's abs-max
-};
-
-// Grouped GEMM tile plan in the workspace (int32): [0] = number of row tiles, then from [4] on
-// one entry of four per row tile: expert, first row, end row (both absolute rows of A and C).
-constexpr int PLAN_HEADER = 4, PLAN_ENTRY = 4;
-
-// s_waitcnt immediate: wait until at most `vm` vector-memory loads are outstanding
-// and all LDS / scalar-memory operations are done (vmcnt is split over bits 3:0 and 15:14).
-constexpr int waitcnt_vm_lgkm0(int vm) { return (vm & 0xf) | (((vm >> 4) & 3) << 14) | (7 << 4); }
-// ... and one that waits for LDS / scalar-memory operations only
-// Tile rows per band of the tile walk (tile_of_block).  Measured with the profiler's FETCH_SIZE counter (bytes
-// that miss the XCDs' L2s) on the 256-row kernels at M = 4096: bands of 4 rows fetch 6 % less than bands of 8
-// on 7168 x 16384 (224-wide tiles) and 20 % less on 2112 x 7168 (192-wide tiles), the same on 24576 x 1536 and
-// 4096 x 7168 (with 32 tiles in flight per XCD, 4 x 8 and 8 x 4 touch the same number of rows when the tile is
-// square); bands of 16 fetch 40-70 % more.  Launch times move by less than 2 % between 4 and 8 and by +2-3 %
-// with 16: these kernels are not bound by that traffic.
-#ifndef SGLQ_GROUP_M
-#define SGLQ_GROUP_M 4
-#endif
-#ifndef SGLQ_STREAM_NSTAGE
-#define SGLQ_STREAM_NSTAGE 3
-#endif
-constexpr int waitcnt_lgkm0_only() { return 0xf | (3 << 14) | (7 << 4); }
-
-// Global -> LDS copies written as assembly (16 or 4 bytes per lane; lane l lands at
-// lds_dst + l * size).  The decode kernel keeps several stages of such copies in flight and
-// waits for them with explicit vmcnt counts; copies issued through the compiler's builtin
-// are tracked by its wait-count pass, which cannot tell the ring's stages apart and would
-// drain every copy in flight before each LDS read.
-SGLQ_DEV v4u make_rsrc_sgpr(const void* ptr, uint32_t bytes) {
-  const uint64_t a = reinterpret_cast<uint64_t>(ptr);
-  return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
-             (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xffffu)),
-             (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-}
-SGLQ_DEV void lds_copy16(v4u rsrc, uint32_t lds_dst, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" : : "s"(lds_dst), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-SGLQ_DEV void lds_copy4(v4u rsrc, uint32_t lds_dst, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds" : : "s"(lds_dst), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-SGLQ_DEV uint32_t lds_addr(const void* p) {
-  return (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)p);
-}
-
-SGLQ_DEV int swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-
-// One 128-byte K block of a block-scaled kind: the product of a weight and an activation
-// fragment from a zero accumulator.  FP8: one MFMA, fp32 result.  INT8: two MFMAs, exact
-// int32 result, returned as its bit pattern so that the conversion to float can wait until
-// the result is folded into the accumulator (block_value) instead of stalling on the MFMA.
-template <int KIND>
-SGLQ_DEV v4f block_mfma(const v8i& w, const v8i& a) {
-  if constexpr (KIND == KIND_I8_BLOCK) {
-    const v4i w0 = {w[0], w[1], w[2], w[3]}, w1 = {w[4], w[5], w[6], w[7]};
-    const v4i a0 = {a[0], a[1], a[2], a[3]}, a1 = {a[4], a[5], a[6], a[7]};
-    v4i t = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0, a0, v4i{0, 0, 0, 0}, 0, 0, 0);
-    t = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1, a1, t, 0, 0, 0);
-    return __builtin_bit_cast(v4f, t);
-  } else {
-    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, a, v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
-  }
-}
-template <int KIND>
-SGLQ_DEV float block_value(float raw) {
-  if constexpr (KIND == KIND_I8_BLOCK) return (float)__builtin_bit_cast(int, raw);
-  else return raw;
-}
-
-template <int OUT_DT>
-SGLQ_DEV void store4(void* out, int64_t idx, float v0, float v1, float v2, float v3) {
-  if constexpr (OUT_DT == SGLQ_BF16) {
-    typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
-    bf4 o = {(__bf16)v0, (__bf16)v1, (__bf16)v2, (__bf16)v3};
-    *reinterpret_cast<bf4*>(reinterpret_cast<__bf16*>(out) + idx) = o;
-  } else {
-    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-    h4 o = {(_Float16)v0, (_Float16)v1, (_Float16)v2, (_Float16)v3};
-    *reinterpret_cast<h4*>(reinterpret_cast<_Float16*>(out) + idx) = o;
-  }
-}
-
-// fp32 -> output type -> fp32
-template <int OUT_DT>
-SGLQ_DEV float round_out(float v) {
-  if constexpr (OUT_DT == SGLQ_BF16) return (float)(__bf16)v;
-  else return (float)(_Float16)v;
-}
-
-template <int OUT_DT>
-SGLQ_DEV void load_bias4(const void* bias, int n, float (&b)[4]) {
-  if constexpr (OUT_DT == SGLQ_BF16) {
-    const uint16_t* p = reinterpret_cast<const uint16_t*>(bias) + n;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) b[j] = u2f((uint32_t)p[j] << 16);
-  } else {
-    const _Float16* p = reinterpret_cast<const _Float16*>(bias) + n;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) b[j] = (float)p[j];
-  }
-}
-
-// Map the linear block id to an output tile: consecutive ids are dealt round-robin
-// to the 8 XCDs by the dispatcher, so give every XCD one contiguous range of tiles
-// (its L2 then sees a compact set of A rows and B columns), and walk each range in
-// bands of GROUP_M tile-rows.
-SGLQ_DEV void tile_of_block(int pid, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int total = tiles_m * tiles_n;
-  const int q = total >> 3, rem = total & 7;
-  const int xcd = pid & 7, idx = pid >> 3;
-  int tile = xcd * q + (xcd < rem ? xcd : rem) + idx;
-  constexpr int GROUP_M = SGLQ_GROUP_M;
-  const int width = GROUP_M * tiles_n;
-  const int group = tile / width;
-  const int first_m = group * GROUP_M;
-  const int gsz = (tiles_m - first_m) < GROUP_M ? (tiles_m - first_m) : GROUP_M;
-  const int in_group = tile - group * width;
-  tm = first_m + in_group % gsz;
-  tn = in_group / gsz;
-}
-
-// Scale, add bias and store four consecutive outputs C[m][n..n+3] from their accumulators.
-// BLOCK_BIAS (block-scaled kinds only): 1 / 0 = the caller knows at compile time that there
-// is / is not a bias, -1 = look at p.bias.
-template <int KIND, int OUT_DT, int BLOCK_BIAS = -1, typename acc_t>
-SGLQ_DEV void finish4(const GemmArgs& p, int m, int n, const acc_t& a, float sam) {
-  const int64_t idx = (int64_t)m * p.ldo + n;
-  if constexpr (KIND == KIND_I8_RAW) {
-    *reinterpret_cast<v4i*>(reinterpret_cast<int32_t*>(p.out) + idx) = a;
-  } else if constexpr (is_block(KIND)) {
-    if (BLOCK_BIAS == 1 || (BLOCK_BIAS == -1 && p.bias)) {
-      // the caller's `output += bias` on the rounded GEMM result (fp8_utils.py:210-211), fused:
-      // round to the output type, add the bias in fp32, round again
-      float bv[4], o[4];
-      load_bias4<OUT_DT>(p.bias, n, bv);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = round_out<OUT_DT>(a[e]) + bv[e];
-      store4<OUT_DT>(p.out, idx, o[0], o[1], o[2], o[3]);
-    } else {
-      store4<OUT_DT>(p.out, idx, a[0], a[1], a[2], a[3]);
-    }
-  } else {
-    float o[4], bv[4] = {0.f, 0.f, 0.f, 0.f};
-    const v4f sbn = *reinterpret_cast<const v4f*>(p.sb + n);
-    if (p.bias) load_bias4<OUT_DT>(p.bias, n, bv);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if constexpr (KIND == KIND_I8_ROWCOL) o[e] = __builtin_fmaf((float)a[e], sbn[e] * sam, bv[e]);
-      else o[e] = __builtin_fmaf(sam, sbn[e] * a[e], bv[e]);
-    }
-    store4<OUT_DT>(p.out, idx, o[0], o[1], o[2], o[3]);
-  }
-}
-
-// Split-K: store a wave's raw accumulators as partial sums of split `split` in the
-// workspace, laid out [split][M][N] (fp32 or int32); splitk_reduce_kernel finishes them.
-template <int MI, int NI, typename acc_t>
-SGLQ_DEV void store_partials(const GemmArgs& p, acc_t (&acc)[MI][NI], int split, int m_base, int n_base, int r16, int g) {
-  asm volatile("" : "+v"(r16), "+v"(g));  // keep the address arithmetic here (see epilogue_via_lds)
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    const int m = m_base + i * 16 + r16;
-    if (m >= p.M) continue;
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const int n = n_base + j * 16 + g * 4;
-      if (n >= p.N) continue;
-      acc_t* dst = reinterpret_cast<acc_t*>(reinterpret_cast<char*>(p.ws) + (((int64_t)split * p.M + m) * p.N + n) * 4);
-      *dst = acc[i][j];
-    }
-  }
-}
-
-// The same for the 256-row kernels, as buffer stores that need neither branches nor 64-bit
-// addresses: a row beyond M lies beyond the split's extent and is dropped by the bounds
-// check, a column beyond N gets an offset that is.  The host keeps (M + 256) N 4 below 2 GiB.
-template <int MI, int NI, typename acc_t>
-SGLQ_DEV void store_partials_bounded(const GemmArgs& p, acc_t (&acc)[MI][NI], int split, int m_base, int n_base, int r16, int g) {
-  asm volatile("" : "+v"(r16), "+v"(g));  // keep the address arithmetic here (see epilogue_via_lds)
-  const uint32_t row_bytes = (uint32_t)p.N * 4u, split_bytes = (uint32_t)p.M * row_bytes;
-  const __amdgpu_buffer_rsrc_t rw = make_rsrc(reinterpret_cast<char*>(p.ws) + (int64_t)split * split_bytes, split_bytes);
-  const int n_lane = n_base + g * 4;
-  const uint32_t off = (uint32_t)(m_base + r16) * row_bytes + (uint32_t)n_lane * 4u;
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const uint32_t voff = (n_lane + j * 16 < p.N) ? off + (uint32_t)(i * 16) * row_bytes + (uint32_t)(j * 64) : OOB;
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, acc[i][j]), rw, voff, 0, 0);
-    }
-  }
-}
-
-// Scale, add bias and store a wave's accumulators.  acc[i][j][e] belongs to
-// C[m_base + 16 i + r16][n_base + 16 j + 4 g + e].
-template <int KIND, int OUT_DT, int MI, int NI, int BLOCK_BIAS = -1, typename acc_t>
-SGLQ_DEV void epilogue(const GemmArgs& p, acc_t (&acc)[MI][NI], int m_base, int n_base, int r16, int g) {
-  asm volatile("" : "+v"(r16), "+v"(g));  // keep the address arithmetic here (see epilogue_via_lds)
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    const int m = m_base + i * 16 + r16;
-    if (m >= p.M) continue;
-    float sam = 1.f;
-    if constexpr (KIND == KIND_FP8_ROWCOL || KIND == KIND_I8_ROWCOL) sam = p.sa[m];
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const int n = n_base + j * 16 + g * 4;
-      if (n >= p.N) continue;  // N % 8 == 0 (% 4 for 32-bit outputs) is checked on the host: a run of 4 is in or out as a whole
-      finish4<KIND, OUT_DT, BLOCK_BIAS>(p, m, n, acc[i][j], sam);
-    }
-  }
-}
 
 // Epilogue of the 256-row kernels for 16-bit outputs, in two halves of 128 rows: every
 // wave converts one half of its accumulators (fragment rows i < MI / 2, then the rest; scales
@@ -3305,9 +3043,147 @@ static int stream_choice(const GemmArgs& p) {
   return 0;
 }
 
+// gemm_ring_kernel (gemm_ring.h) on tile shape `config`.
+constexpr int RING_TILE = 300;  // kernel codes RING_TILE + config of sglq_debug_force_tile and sglq_tuned_add
+template <int KIND, int OUT_DT>
+static void launch_ring(GemmArgs& p, int config, hipStream_t st) {
+  expand_packed_scales(p, st);
+  g_last_kernel = "gemm_ring_kernel";
+  if constexpr (KIND == KIND_FP8_BLOCK) {
+    // (power-of-two scales in the matrix instruction where the other kernels have it too; up to 128 rows and on K below
+    // three K blocks the folds are hidden behind the operand intake, and the result is the fp32-scale entry point's bit for bit)
+    if (p.M > 128 && p.K >= 384 && hw_scaled<KIND, OUT_DT>(p)) launch_ring_fp8_block_pow2(p, config, OUT_DT, st);
+    else launch_ring_fp8_block(p, config, OUT_DT, st);
+  } else if constexpr (KIND == KIND_FP8_ROWCOL) {
+    launch_ring_fp8_rowcol(p, config, OUT_DT, st);
+  } else if constexpr (KIND == KIND_I8_ROWCOL) {
+    launch_ring_i8_rowcol(p, config, OUT_DT, st);
+  } else if constexpr (KIND == KIND_I8_BLOCK) {
+    launch_ring_i8_block(p, config, OUT_DT, st);
+  }
+}
+
+// Modelled time (us) of gemm_ring_kernel on tile shape `config`: what a launch pays, then per round of the CUs a fixed
+// part (first operands, epilogue) and the K blocks, which take longer the fuller the rounds are.  Coefficients fitted
+// (non-negative least squares on the relative error) to 88 shapes per kind, M = 17 ... 4096, N = 512 ... 32768,
+// K = 512 ... 16384, three weights in turn: 3-10 % rms; the shape it picks is within 0.5 % of the best one on average
+// and within 7 % everywhere.
+struct RingCost {
+  float launch, round, step, full;
+};
+static const RingCost ring_cost_fp8_block[RING_CONFIGS] = {
+    {1.72f, 1.89f, .1714f, .0075f}, {1.80f, 2.20f, .1912f, .0165f}, {1.76f, 2.60f, .2279f, .0178f}, {1.81f, 2.62f, .2320f, .0322f},
+    {1.48f, 2.68f, .2954f, .0273f}, {1.71f, 2.59f, .2459f, .0996f}, {1.51f, 3.02f, .4203f, .0833f}, {1.38f, 3.33f, .4741f, .0961f},
+    {1.81f, 2.55f, .3102f, .0389f}, {1.44f, 3.23f, .3272f, .0688f}, {1.54f, 3.12f, .3329f, .1233f}, {1.88f, 3.24f, .4414f, .1622f},
+    {1.92f, 3.16f, .4877f, .1930f}, {1.75f, 3.70f, .5542f, .2552f}, {1.68f, 2.24f, .1379f, .0238f}, {2.05f, 2.02f, .1998f, .0284f}};
+static const RingCost ring_cost_i8_block[RING_CONFIGS] = {
+    {1.73f, 1.81f, .1834f, .0082f}, {1.79f, 2.24f, .2065f, .0156f}, {1.68f, 2.80f, .2264f, .0183f}, {1.75f, 2.71f, .2518f, .0306f},
+    {1.49f, 2.63f, .3325f, .0306f}, {1.69f, 2.67f, .2801f, .0949f}, {1.51f, 2.93f, .4928f, .0801f}, {1.26f, 3.31f, .5563f, .0927f},
+    {1.82f, 2.46f, .3562f, .0437f}, {1.47f, 3.24f, .4034f, .0705f}, {1.43f, 3.24f, .4561f, .1065f}, {1.91f, 3.26f, .5853f, .1468f},
+    {1.88f, 3.46f, .6708f, .1500f}, {1.87f, 3.68f, .7814f, .2126f}, {1.67f, 2.40f, .1277f, .0261f}, {2.06f, 2.15f, .1954f, .0330f}};
+// (per-row / per-column kinds, and block scales that the matrix instruction applies)
+static const RingCost ring_cost_in_place[RING_CONFIGS] = {
+    {1.60f, 1.91f, .1913f, .0006f}, {1.73f, 2.27f, .2132f, .0127f}, {1.56f, 2.82f, .2497f, .0130f}, {1.61f, 2.86f, .2699f, .0225f},
+    {1.23f, 2.79f, .2456f, .0447f}, {1.56f, 2.62f, .2485f, .0923f}, {1.36f, 3.31f, .3249f, .1334f}, {1.21f, 3.87f, .3615f, .1469f},
+    {1.63f, 2.52f, .2862f, .0373f}, {1.24f, 3.43f, .3014f, .0675f}, {1.50f, 3.45f, .3272f, .1177f}, {1.95f, 3.63f, .3464f, .1921f},
+    {1.95f, 3.69f, .4055f, .2110f}, {1.89f, 4.38f, .4805f, .2767f}, {1.57f, 2.41f, .1358f, .0207f}, {2.01f, 2.11f, .2147f, .0279f}};
+static int ring_best(const RingCost* table, const GemmArgs& p, double& cost) {
+  int best = 0;
+  cost = 1e30;
+  const double nkb = (double)((p.K + 127) >> 7);
+  for (int i = 0; i < RING_CONFIGS; ++i) {
+    const int64_t tiles = (int64_t)((p.M + RING_BM[i] - 1) / RING_BM[i]) * ((p.N + RING_BN[i] - 1) / RING_BN[i]);
+    const int64_t rounds = (tiles + num_cus() - 1) / num_cus();
+    const double full = (double)tiles / (double)(rounds * num_cus());
+    const double c = table[i].launch + rounds * (table[i].round + nkb * (table[i].step + table[i].full * full));
+    if (c < cost) {
+      cost = c;
+      best = i;
+    }
+  }
+  return best;
+}
+
+// Whether gemm_ring_kernel takes the problem, and on which tile shape (-1: one of the other kernels), from its model
+// and fits (same shapes) of what the kernel that the rules of launch_kind would choose takes:
+//   * 17 .. 64 rows: only where that is gemm_skinny_kernel with K split (48 x 10752 x 768: 9.4 -> 5.8 us, 48 x 11072 x
+//     13312: 42.5 -> 34.5) or on K >= 2048 (64 x 57344 x 8192: 102 -> 92); gemm_stream_kernel's narrow blocks are faster
+//     (27 x 2048 x 14464: 10.1 against 20.4 us), except the 32-row blocks that exactly fill one round on K >= 8192;
+//   * 65 .. 512 rows on few tiles with a long K: the weight-streaming kernels spread K over the CUs (206 x 576 x 9088:
+//     12.0 against 18.0 us);
+//   * tiles of 256 rows wherever those fill the chip well (3254 x 17344 x 512: 43 against 52 us);
+//   * up to 128 rows on 48 MiB and more the pipelined 128-row kernel stays (its first two K blocks cover the HBM latency);
+//   * K that is no multiple of 128 (per-row / per-column kinds): always, the alternative is gemm_kernel's copies through
+//     the compiler's wait counts (297 x 1488 x 2336: 17.4 us for the linear).
+template <int KIND, int OUT_DT>
+static int ring_choice(const GemmArgs& p) {
+  double cost;
+  const bool hw = can_hw_scale<KIND, OUT_DT>(p);
+  const RingCost* table = KIND == KIND_I8_BLOCK ? ring_cost_i8_block : (is_block(KIND) && !hw) ? ring_cost_fp8_block : ring_cost_in_place;
+  if (p.K & 127) return p.K < 256 && p.M <= 16 ? -1 : ring_best(table, p, cost);
+  if (p.M <= 16) return -1;
+  const int64_t weight_bytes = (int64_t)p.N * p.K;
+  const int nkb = p.K >> 7;
+  auto skinny_us = [](double model) { return KIND == KIND_I8_BLOCK ? 3.7 + 1.24 * model : is_block(KIND) ? 3.7 + 1.07 * model : 4.4 + 0.81 * model; };
+  if (p.M <= 64) {
+    const int nib = stream_rows<KIND>(p);
+    const bool fills_one_round = p.M > 32 && nib == 2 && p.K >= 8192 && weight_bytes > (30 << 20);
+    if (nib != 0 && !fills_one_round) return -1;
+    const int config = ring_best(table, p, cost);
+    if (nib != 0) return config;
+    const int t64 = (p.N + 63) / 64;
+    const bool narrow = p.M > 32 && (p.N <= 4096 || (4 * t64 > 3 * num_cus() && t64 <= num_cus() && nkb <= 40));  // (as in launch_skinny)
+    const int splits = skinny_splits(p.M, p.N, p.K, narrow ? 64 : 128);
+    if (p.K < 512 || (p.K < 2048 && splits == 1)) return -1;
+    return cost < skinny_us(skinny_cost(p.M, p.N, p.K, narrow ? 64 : 128, splits)) ? config : -1;
+  }
+  if (p.M <= 128 && weight_bytes >= (48 << 20) && p.K >= 384) return -1;
+  const int config = ring_best(table, p, cost);
+  double other = 1e30;
+  if (p.M <= 512) {
+    const double wide = skinny_cost(p.M, p.N, p.K, 128, skinny_splits(p.M, p.N, p.K, 128));
+    const double narrow = skinny_cost(p.M, p.N, p.K, 64, skinny_splits(p.M, p.N, p.K, 64));
+    const double skinny = wide < narrow ? wide : narrow;
+    other = 0.97 * skinny_us(skinny);
+    const int tiles32 = ((p.M + 31) / 32) * ((p.N + 63) / 64);
+    if (tiles32 <= num_cus() && p.K >= 512) {
+      const double stream = 4.0 + (KIND == KIND_I8_BLOCK ? 0.172 : 0.16) * nkb;
+      if (stream < other) other = stream;
+    }
+  }
+  // 256-row tiles, fitted like the ring's (2-6 % rms)
+  if (p.M > 128 && p.K >= 384) {
+    struct WideCost {
+      int bm, bn;
+      float launch, round, step, full;
+    };
+    static const WideCost fp8_block[] = {{192, 192, 3.3f, 3.3f, .45f, .58f}, {256, 192, 4.0f, 4.1f, .26f, 1.06f}, {256, 224, 5.0f, 3.8f, .44f, 1.06f}, {256, 256, 7.8f, 2.1f, .84f, .74f}};
+    static const WideCost i8_block[] = {{256, 192, 3.5f, 4.4f, .64f, .94f}, {256, 192, 3.5f, 4.4f, .64f, .94f}, {256, 224, 5.5f, 3.7f, 1.10f, .70f}, {256, 256, 11.3f, 12.4f, 1.79f, 0.f}};
+    static const WideCost in_place[] = {{256, 192, 3.4f, 5.4f, .27f, .86f}, {256, 192, 3.4f, 5.4f, .27f, .86f}, {256, 224, 4.6f, 5.7f, .49f, .76f}, {256, 256, 5.6f, 6.3f, .90f, .42f}};
+    const WideCost* wide = KIND == KIND_I8_BLOCK ? i8_block : (is_block(KIND) && !hw) ? fp8_block : in_place;
+    if (((p.M + 255) / 256) * ((p.N + 255) / 256) >= 140) {
+      for (int i = p.bias ? 1 : 0; i < 4; ++i) {
+        const int64_t tiles = (int64_t)((p.M + wide[i].bm - 1) / wide[i].bm) * ((p.N + wide[i].bn - 1) / wide[i].bn);
+        const int64_t rounds = (tiles + num_cus() - 1) / num_cus();
+        const double full = (double)tiles / (double)(rounds * num_cus());
+        const double c = wide[i].launch + rounds * (wide[i].round + nkb * (wide[i].step + wide[i].full * full));
+        if (0.95 * c < other) other = 0.95 * c;  // (on several rounds the ring's model is a few per cent low)
+      }
+    }
+  }
+  return cost < other ? config : -1;
+}
+
 template <int KIND, int OUT_DT>
 static void launch_kind(GemmArgs& p, int64_t ws_bytes, hipStream_t st) {
   pick_selection(KIND, p);
+  if constexpr (KIND != KIND_I8_RAW) {
+    const int config = !g_use_dma ? -1 : t_tile >= RING_TILE ? t_tile - RING_TILE : (t_tile == 0 && t_splits == 0) ? ring_choice<KIND, OUT_DT>(p) : -1;
+    if (config >= 0) {
+      launch_ring<KIND, OUT_DT>(p, config, st);
+      return;
+    }
+  }
   if ((p.K & 127) == 0 && p.M <= 64 && g_use_dma && (t_tile == 0 || t_tile == 16 || t_tile == 32) &&
       launch_stream<KIND, OUT_DT>(p, st))
     return;
@@ -3500,6 +3376,7 @@ extern "C" int sglq_tuned_add(int kind, int64_t N, int64_t K, int64_t m_lo, int6
   static const int tiles[] = {0, 16, 32, 64, 66, 68, 69, 128, 130, 192, 193, 224, 256, 257, 258, 259};
   bool known = false;
   for (int t : tiles) known = known || t == tile;
+  known = known || (tile >= RING_TILE && tile < RING_TILE + RING_CONFIGS);
   if (kind < 0 || kind > 4 || N <= 0 || K <= 0 || m_lo < 0 || m_hi < m_lo || !known || splits < 0 || splits > 64) {
     set_error("tuned_add: kind 0..4, positive N and K, 0 <= m_lo <= m_hi, a known kernel code and 0 <= splits <= 64 expected");
     return SGLQ_EINVAL;

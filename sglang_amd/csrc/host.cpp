@@ -288,13 +288,15 @@ PyObject* block_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         char* codes = need > CODES_BYTES ? static_cast<char*>(large.data_ptr()) : ws->base;
         float* scales = reinterpret_cast<float*>(codes + round256(m * k));
         void* partial = ws->base + CODES_BYTES;
-        if (mode == BLOCK_INT8) {  // row-major activation scales
-          rc = lib.sglq_per_token_group_quant_int8(x_p, code, codes, scales, m, k, 128, kb, 1, eps, -128.0f, 127.0f, here.stream);
+        if (mode == BLOCK_INT8) {
+          // (column-major scales: the GEMM fetches a K block's scales of 64 rows with one instruction, from two cache
+          // lines instead of up to 64; 1000 x 5120 x 5120 with bias 49.8 -> 42 us together with gemm_ring_kernel)
+          rc = lib.sglq_per_token_group_quant_int8(x_p, code, codes, scales, m, k, 128, 1, m, eps, -128.0f, 127.0f, here.stream);
           if (rc == 0 && bias_p)
-            rc = lib.sglq_int8_blockwise_scaled_mm_bias(codes, k, w_p, k, scales, kb, 1, s_p, 1, sn, bias_p, out_p, n, code, m, n, k, partial,
+            rc = lib.sglq_int8_blockwise_scaled_mm_bias(codes, k, w_p, k, scales, 1, m, s_p, 1, sn, bias_p, out_p, n, code, m, n, k, partial,
                                                         SPLITK_BYTES, here.stream);
           else if (rc == 0)
-            rc = lib.sglq_int8_blockwise_scaled_mm(codes, k, w_p, k, scales, kb, 1, s_p, 1, sn, out_p, n, code, m, n, k, partial, SPLITK_BYTES,
+            rc = lib.sglq_int8_blockwise_scaled_mm(codes, k, w_p, k, scales, 1, m, s_p, 1, sn, out_p, n, code, m, n, k, partial, SPLITK_BYTES,
                                                    here.stream);
         } else if (mode == BLOCK_FP8_POW2) {
           rc = lib.sglq_per_token_group_quant_fp8_pow2(x_p, code, codes, scales, m, k, 1, m, eps, -448.0f, 448.0f, here.stream);
