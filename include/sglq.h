@@ -356,6 +356,14 @@ int sglq_per_token_group_quant_fp8_scatter(const void* input, int in_dtype, void
 int sglq_silu_and_mul_group_quant_fp8(const void* input, int in_dtype, void* output_q, float* output_s,
                                       int64_t num_tokens, int64_t d, float eps, void* stream);
 
+/* The two operators above with column-major scales, [hidden / 128][num_dst_rows] and [d / 128][num_tokens]: what the grouped
+ * GEMM fetches in whole cache lines (scale strides 1 and the number of rows). */
+int sglq_per_token_group_quant_fp8_scatter_cm(const void* input, int in_dtype, void* output_q, float* output_s,
+                                              const int32_t* slot_map, int64_t num_tokens, int64_t hidden, int64_t topk,
+                                              int64_t num_dst_rows, float eps, void* stream);
+int sglq_silu_and_mul_group_quant_fp8_cm(const void* input, int in_dtype, void* output_q, float* output_s,
+                                         int64_t num_tokens, int64_t d, float eps, void* stream);
+
 /* Replaces w8a8_block_int8_matmul, a Triton kernel in the reference
  * (python/sglang/srt/layers/quantization/int8_kernel.py:212-425; there is no
  * sgl_kernel C++ op): out[m,n] = sum_kb float(sum_{k in block kb} a[m,k] b[k,n])

@@ -79,7 +79,9 @@ SIGNATURES = {
     "sglq_tuned_add": [c_int, c_int64, c_int64, c_int64, c_int64, c_int, c_int],
     "sglq_tuned_clear": [],
     "sglq_per_token_group_quant_fp8_scatter": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_float, c_void_p],
+    "sglq_per_token_group_quant_fp8_scatter_cm": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_float, c_void_p],
     "sglq_silu_and_mul_group_quant_fp8": [c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int64, c_float, c_void_p],
+    "sglq_silu_and_mul_group_quant_fp8_cm": [c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int64, c_float, c_void_p],
     "sglq_prepare_moe_layer": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,
                                c_void_p, c_void_p],
     "sglq_fp8_blockwise_scaled_grouped_mm_planned": [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p,

@@ -22,7 +22,8 @@ CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libsglq.so"
 BENCH_LIB_PATH = PKG_DIR / "libsglq_bench.so"
 NATIVE_PATH = PKG_DIR / "_native.so"
-SOURCES = ["gemm.hip", "gemm_ring_fp8_block.hip", "gemm_ring_fp8_block_pow2.hip", "gemm_ring_fp8_rowcol.hip", "gemm_ring_i8_rowcol.hip",
+SOURCES = ["gemm.hip", "gemm_ring_fp8_block.hip", "gemm_ring_fp8_block_grouped.hip", "gemm_ring_fp8_block_pow2.hip",
+           "gemm_ring_fp8_rowcol.hip", "gemm_ring_i8_rowcol.hip",
            "gemm_ring_i8_block.hip", "common.hip", "quant.hip", "moe.hip"]
 BENCH_SOURCES = ["bench_kernels.hip"]
 

@@ -307,6 +307,12 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64, 2) void gemm_kernel(const Ge
 
   // blockIdx = split * tiles + tile; split s works on K blocks [kb_lo, kb_hi)
   GemmArgs p = p_in;
+  // (grouped: the grid covers the largest possible number of row tiles; the blocks in front are dealt over the plan's, or
+  // few tiles would all land in the first XCD's range: 2 tokens, top 3 of 62 experts of 4992 x 1280: 133 -> 58 us a layer)
+  if constexpr (GROUPED) {
+    p.tiles_m = *static_cast<const int*>(p.ws);
+    if ((int)blockIdx.x >= p.tiles_m * p.tiles_n) return;
+  }
   const int tiles = p.tiles_m * p.tiles_n;
   const int split = GROUPED ? 0 : blockIdx.x / tiles;
   int tm, tn;
@@ -315,7 +321,6 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64, 2) void gemm_kernel(const Ge
   const int n0 = tn * BN;
   if constexpr (GROUPED) {
     const int* plan = static_cast<const int*>(p.ws);
-    if (tm >= plan[0]) return;  // the grid covers the largest possible number of row tiles
     const int* entry = plan + PLAN_HEADER + PLAN_ENTRY * tm;
     const int expert = entry[0];
     m0 = entry[1];
@@ -3396,7 +3401,8 @@ extern "C" int sglq_tuned_add(int kind, int64_t N, int64_t K, int64_t m_lo, int6
 }
 
 extern "C" void sglq_debug_grouped_tile(int rows) {
-  g_grouped_tile = (rows == 32 || rows == 64 || rows == 128 || rows == 130 || rows == 256) ? rows : 0;
+  const bool ring = rows >= RING_TILE && rows < RING_TILE + RING_CONFIGS && RING_GROUPED[rows - RING_TILE];
+  g_grouped_tile = (ring || rows == 32 || rows == 64 || rows == 128 || rows == 130 || rows == 256) ? rows : 0;
 }
 extern "C" const char* sglq_debug_last_gemm_kernel(void) { return g_last_kernel; }
 extern "C" int sglq_debug_last_gemm_hw_scaled(void) { return g_last_hw_scaled ? 1 : 0; }
@@ -3502,14 +3508,31 @@ extern "C" int sglq_fp8_blockwise_scaled_mm_bias(const void* a, int64_t lda, con
 // 256-row ones 2.1-2.2 ms whatever their fill); above 128 rows per expert two 128-row tiles
 // cost what one 256-row tile costs and the 256-row tile computes faster (2.26 against
 // 2.51 ms at 256 rows, 7.7 against 8.1 ms at 1024).
-static int grouped_tile_rows(int64_t total_m, int64_t num_experts, int64_t K, bool& pipelined) {
+struct GroupedTile {
+  int rows;
+  bool pipelined;
+  int ring;  // tile shape of gemm_ring_kernel, -1 = another kernel
+};
+constexpr int RING_GROUPED_64 = 5;  // 64 x 128
+static_assert(RING_GROUPED[RING_GROUPED_64] && RING_BM[RING_GROUPED_64] == 64, "a grouped tile of 64 rows");
+static GroupedTile grouped_tile(int64_t total_m, int64_t num_experts, int64_t K) {
   const int64_t avg = total_m / num_experts;
-  if (g_grouped_tile) {  // test hook; 130 = the pipelined kernel with 128-row tiles
-    pipelined = g_grouped_tile == 256 || g_grouped_tile == 130;
-    return g_grouped_tile == 130 ? 128 : g_grouped_tile;
-  }
-  pipelined = avg >= 12 && K >= 384;
-  return pipelined ? (avg > 128 ? 256 : 128) : avg < 12 ? 64 : 128;
+  if (g_grouped_tile >= RING_TILE) return {RING_BM[g_grouped_tile - RING_TILE], false, g_grouped_tile - RING_TILE};
+  if (g_grouped_tile)  // test hook; 130 = the pipelined kernel with 128-row tiles
+    return {g_grouped_tile == 130 ? 128 : g_grouped_tile, g_grouped_tile == 256 || g_grouped_tile == 130, -1};
+  // Times of a whole layer (us), tokens x experts x top-k, hidden x intermediate:
+  //   * a few row tiles leave CUs idle whatever the tile, and the ring takes in the weights fastest: 1 x 62 x 8,
+  //     4096 x 1024: 43 on its 64 x 128 tiles, 55 with 32-row tiles of gemm_kernel, 58 with 64-row tiles;
+  //   * below 12 rows an expert the weights come from HBM once and 32-row tiles move the least besides: 16 x 32 x 8,
+  //     7168 x 2048: 247 against 265 (64 rows), 263 (ring);
+  //   * up to 40 rows the ring, 100 x 32 x 8, 7168 x 2048: 292 against 326 (32), 307 (64), 296 (pipelined 128), but on short
+  //     K gemm_kernel with the same 64-row plan (150 x 24 x 2, 3072 x 768: 61 against 66 and 73);
+  //   * above, the pipelined kernel's 128- and 256-row tiles (182 x 28 x 7, 2304 x 1920: 108 against 121 on the ring).
+  if ((total_m < num_experts + total_m / 64 ? total_m : num_experts + total_m / 64) <= 10) return {64, false, RING_GROUPED_64};
+  if (avg < 12) return {32, false, -1};
+  if (avg < 40) return {64, false, K >= 1024 ? RING_GROUPED_64 : -1};
+  if (K < 384) return {128, false, -1};
+  return {avg > 128 ? 256 : 128, true, -1};
 }
 
 // `plan_rows` > 0: `workspace` already holds the tile plan for row tiles of that height
@@ -3543,8 +3566,9 @@ static int grouped_entry(const void* a, int64_t lda, const void* b, int64_t ldb,
     set_error("%s: the experts' weights must be 16-byte aligned, fewer than 2^20 experts", name);
     return SGLQ_EINVAL;
   }
-  bool pipelined;
-  const int bm = grouped_tile_rows(total_m, num_experts, K, pipelined);
+  const GroupedTile tile = grouped_tile(total_m, num_experts, K);
+  const bool pipelined = tile.pipelined;
+  const int bm = tile.rows;
   if (plan_rows != 0 && plan_rows != bm) {
     set_error("%s: the plan is for row tiles of %lld, this call takes %d", name, (long long)plan_rows, bm);
     return SGLQ_EINVAL;
@@ -3560,7 +3584,7 @@ static int grouped_entry(const void* a, int64_t lda, const void* b, int64_t ldb,
               (long long)workspace_bytes);
     return SGLQ_EINVAL;
   }
-  if (max_tiles * ((N + 127) / 128) >= (1ll << 31)) {
+  if (max_tiles * ((N + 31) / 32) >= (1ll << 31)) {
     set_error("%s: too many tiles", name);
     return SGLQ_EUNSUPPORTED;
   }
@@ -3580,6 +3604,12 @@ static int grouped_entry(const void* a, int64_t lda, const void* b, int64_t ldb,
   if (plan_rows == 0)
     grouped_plan_kernel<<<dim3(1), dim3(256), 0, st>>>(problem_sizes, expert_offsets, (int)num_experts, (int)total_m, bm,
                                                        (int)max_tiles, static_cast<int*>(workspace));
+  if (tile.ring != -1) {
+    g_last_kernel = "grouped_plan_kernel+gemm_ring_kernel<grouped>";
+    p.tiles_m = (int)max_tiles;
+    launch_ring_fp8_block_grouped(p, tile.ring, out_dtype, st);
+    return finish(name);
+  }
   if (pipelined) {
     g_last_kernel = bm == 256 ? "grouped_plan_kernel+gemm_pipe_kernel<grouped>" : "grouped_plan_kernel+gemm_pipe_kernel<grouped, 128 rows>";
     p.tiles_m = (int)max_tiles;
@@ -3622,8 +3652,7 @@ extern "C" int sglq_fp8_blockwise_scaled_grouped_mm(const void* a, int64_t lda, 
 }
 
 extern "C" int64_t sglq_grouped_plan_rows(int64_t num_experts, int64_t total_m, int64_t K) {
-  bool pipelined;
-  return num_experts > 0 && total_m >= 0 ? grouped_tile_rows(total_m, num_experts, K, pipelined) : 0;
+  return num_experts > 0 && total_m >= 0 ? grouped_tile(total_m, num_experts, K).rows : 0;
 }
 
 extern "C" int sglq_fp8_blockwise_scaled_grouped_mm_planned(const void* a, int64_t lda, const void* b, int64_t ldb,

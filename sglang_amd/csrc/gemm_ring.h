@@ -51,9 +51,13 @@ constexpr int RING_BM[] = {SGLQ_RING_CONFIGS(SGLQ_RING_BM)};
 constexpr int RING_BN[] = {SGLQ_RING_CONFIGS(SGLQ_RING_BN)};
 constexpr int RING_KG[] = {SGLQ_RING_CONFIGS(SGLQ_RING_KG)};
 
+// ... and whether a grouped (expert) GEMM is built on it
+constexpr bool RING_GROUPED[] = {false, false, false, false, false, true, false, false, false, false, false, false, false, false, false, false};
+
 // Launches configuration `config` for the problem (tiles_m / tiles_n are set here); one function per kind, each in a
 // translation unit of its own.
 void launch_ring_fp8_block(GemmArgs& p, int config, int out_dtype, hipStream_t st);
+void launch_ring_fp8_block_grouped(GemmArgs& p, int config, int out_dtype, hipStream_t st);
 void launch_ring_fp8_block_pow2(GemmArgs& p, int config, int out_dtype, hipStream_t st);
 void launch_ring_fp8_rowcol(GemmArgs& p, int config, int out_dtype, hipStream_t st);
 void launch_ring_i8_rowcol(GemmArgs& p, int config, int out_dtype, hipStream_t st);

@@ -30,7 +30,8 @@ SGLQ_DEV void values4(const GemmArgs& p, int n, const acc_t& a, float sam, float
   }
 }
 
-template <int KIND, int OUT_DT, int WM, int WN, int KG, int MI, int NI, int NST>
+// GROUPED: the row tiles, their experts and their last rows come from the plan in the workspace (see gemm_kernel).
+template <int KIND, int OUT_DT, int WM, int WN, int KG, int MI, int NI, int NST, bool GROUPED = false>
 __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs p) {
   constexpr int NC = 8, NP = 4, NT = RING_THREADS;
   static_assert(WM * WN * KG == NC, "eight consumer waves");
@@ -57,21 +58,34 @@ __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs 
   const int r16 = lane & 15, g = lane >> 4, l8 = lane >> 3;
   // Block ids are dealt round-robin to the eight XCDs: every XCD gets one contiguous range of tiles, walked in bands of
   // up to eight tile rows, so that a band's row tiles share the weight tile they read at the same time.
+  const int tiles_m = GROUPED ? *static_cast<const int*>(p.ws) : p.tiles_m;
   int tm, tn;
   {
-    const int tiles = p.tiles_m * p.tiles_n;
+    const int tiles = tiles_m * p.tiles_n;
+    if (GROUPED && (int)blockIdx.x >= tiles) return;  // the grid covers the largest possible plan
     const int q = tiles >> 3, rem = tiles & 7;
     const int xcd = (int)blockIdx.x & 7, idx = (int)blockIdx.x >> 3;
     const int tile = xcd * q + (xcd < rem ? xcd : rem) + idx;
-    const int H = p.tiles_m <= 8 ? p.tiles_m : 4;
+    const int H = tiles_m <= 8 ? tiles_m : 4;
     const int width = H * p.tiles_n;
     const int group = tile / width, first_m = group * H;
-    const int gsz = (p.tiles_m - first_m) < H ? (p.tiles_m - first_m) : H;
+    const int gsz = (tiles_m - first_m) < H ? (tiles_m - first_m) : H;
     const int in_group = tile - group * width;
     tm = first_m + in_group % gsz;
     tn = in_group / gsz;
   }
-  const int m0 = tm * BM, n0 = tn * BN;
+  int m0 = tm * BM, m_end = p.M;
+  const int n0 = tn * BN;
+  const char* weight = p.b;
+  const float* weight_scale = p.sb;
+  if constexpr (GROUPED) {
+    const int* entry = static_cast<const int*>(p.ws) + PLAN_HEADER + PLAN_ENTRY * tm;
+    const int expert = __builtin_amdgcn_readfirstlane(entry[0]);
+    m0 = __builtin_amdgcn_readfirstlane(entry[1]);
+    m_end = __builtin_amdgcn_readfirstlane(entry[2]);
+    weight += (int64_t)expert * p.b_expert_stride;
+    weight_scale += (int64_t)expert * p.sb_expert_stride;
+  }
   const int nkb = (p.K + 127) >> 7, T = (nkb + KG - 1) / KG;
   const int k_tail = p.K & 127;  // bytes of the last K block, 0 = all of it
 
@@ -83,7 +97,7 @@ __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs 
   if (wave >= NC) {
     // ---- producers: copy c of a stage brings 8 rows of K block c / GROUPS
     const int pw = wave - NC;
-    const v4u ra = make_rsrc_sgpr(p.a, p.a_bytes), rb = make_rsrc_sgpr(p.b, p.b_bytes);
+    const v4u ra = make_rsrc_sgpr(p.a, p.a_bytes), rb = make_rsrc_sgpr(weight, p.b_bytes);
     const uint32_t chunk_even = (uint32_t)(((lane & 7) ^ l8) & 7) * 16u, chunk_odd = chunk_even ^ 16u;
     const uint32_t lane_a = (uint32_t)(m0 + l8) * p.lda, lane_b = (uint32_t)(n0 + l8) * p.ldb;
     const uint32_t base = lds_addr(smem);
@@ -92,7 +106,7 @@ __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs 
     if constexpr (BLOCK) {
       const int nblocks = (p.N + 127) >> 7;
       rsa = make_rsrc_sgpr(p.sa, (uint32_t)(((int64_t)(p.M - 1) * p.sa_stride_m + (int64_t)(nkb - 1) * p.sa_stride_k + 1) * 4));
-      rsb = make_rsrc_sgpr(p.sb, (uint32_t)(((int64_t)(nblocks - 1) * p.sb_stride_n + (int64_t)(nkb - 1) * p.sb_stride_k + 1) * 4));
+      rsb = make_rsrc_sgpr(weight_scale, (uint32_t)(((int64_t)(nblocks - 1) * p.sb_stride_n + (int64_t)(nkb - 1) * p.sb_stride_k + 1) * 4));
       const int nb = (n0 >> 7) + lane;
       off_sb = (lane < 3 && nb < nblocks) ? (uint32_t)(nb * p.sb_stride_n * 4) : OOB;
     }
@@ -331,7 +345,7 @@ __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs 
   constexpr int CH = BN / 8;
   for (int c = threadIdx.x; c < BM * CH; c += NT) {
     const int row = c / CH, cc = c % CH;
-    if (m0 + row < p.M && n0 + cc * 8 < p.N)
+    if (m0 + row < m_end && n0 + cc * 8 < p.N)
       *reinterpret_cast<v4i*>(reinterpret_cast<char*>(p.out) + ((int64_t)(m0 + row) * p.ldo + n0 + cc * 8) * 2) =
           *reinterpret_cast<const v4i*>(smem + row * IMG_PITCH + cc * 16);
   }
@@ -346,6 +360,22 @@ static void launch_ring_config(GemmArgs& p, int config, hipStream_t st) {
   switch (config) {
 #define SGLQ_RING_CASE(i, wm, wn, kg, mi, ni, nst) \
   case i: gemm_ring_kernel<KIND, OUT_DT, wm, wn, kg, mi, ni, nst><<<grid, block, 0, st>>>(p); break;
+    SGLQ_RING_CONFIGS(SGLQ_RING_CASE)
+#undef SGLQ_RING_CASE
+  }
+}
+
+// A group of problems: the grid is sized for the largest possible plan, p.tiles_m row tiles.
+template <int KIND, int OUT_DT>
+static void launch_ring_grouped_config(GemmArgs& p, int config, hipStream_t st) {
+  p.tiles_n = (p.N + RING_BN[config] - 1) / RING_BN[config];
+  p.splits = 1;
+  const dim3 grid((uint32_t)(p.tiles_m * p.tiles_n)), block(RING_THREADS);
+  switch (config) {
+#define SGLQ_RING_CASE(i, wm, wn, kg, mi, ni, nst)                                                                              \
+  case i:                                                                                                                        \
+    if constexpr (RING_GROUPED[i]) gemm_ring_kernel<KIND, OUT_DT, wm, wn, kg, mi, ni, nst, true><<<grid, block, 0, st>>>(p);       \
+    break;
     SGLQ_RING_CONFIGS(SGLQ_RING_CASE)
 #undef SGLQ_RING_CASE
   }

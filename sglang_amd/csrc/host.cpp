@@ -59,8 +59,8 @@ namespace {
   X(sglq_grouped_plan_rows)                                                                                         \
   X(sglq_fp8_blockwise_scaled_grouped_mm)                                                                           \
   X(sglq_fp8_blockwise_scaled_grouped_mm_planned)                                                                   \
-  X(sglq_per_token_group_quant_fp8_scatter)                                                                         \
-  X(sglq_silu_and_mul_group_quant_fp8)                                                                              \
+  X(sglq_per_token_group_quant_fp8_scatter_cm)                                                                      \
+  X(sglq_silu_and_mul_group_quant_fp8_cm)                                                                           \
   X(sglq_apply_shuffle_mul_sum)                                                                                     \
   X(sglq_apply_shuffle_mul_sum_f32)                                                                                 \
   X(sglq_w8a8_block_fp8_linear)                                                                                     \
@@ -616,16 +616,16 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                          int64_t width, int64_t tile_rows, bool planned) {
         const float* s_p = static_cast<const float*>(s.data_ptr());
         const int64_t ldb = w.stride(2), bs = e > 1 ? w.stride(0) : width * depth;
-        return planned ? lib.sglq_fp8_blockwise_scaled_grouped_mm_planned(q, depth, w.data_ptr(), ldb, bs, f, depth / 128, 1, s_p, s.stride(0),
+        return planned ? lib.sglq_fp8_blockwise_scaled_grouped_mm_planned(q, depth, w.data_ptr(), ldb, bs, f, 1, rows, s_p, s.stride(0),
                                                                           s.stride(1), s.stride(2), y, width, code, tile_rows, e, rows, width,
                                                                           depth, plan, plan_bytes, here.stream)
-                       : lib.sglq_fp8_blockwise_scaled_grouped_mm(q, depth, w.data_ptr(), ldb, bs, f, depth / 128, 1, s_p, s.stride(0),
+                       : lib.sglq_fp8_blockwise_scaled_grouped_mm(q, depth, w.data_ptr(), ldb, bs, f, 1, rows, s_p, s.stride(0),
                                                                   s.stride(1), s.stride(2), y, width, code, sizes, off_p, e, rows, width, depth,
                                                                   plan, plan_bytes, here.stream);
       };
-      if (rc == 0) rc = lib.sglq_per_token_group_quant_fp8_scatter(x.data_ptr(), code, q1, f1, slot_map, m, k, topk, rows, 1e-10f, here.stream);
+      if (rc == 0) rc = lib.sglq_per_token_group_quant_fp8_scatter_cm(x.data_ptr(), code, q1, f1, slot_map, m, k, topk, rows, 1e-10f, here.stream);
       if (rc == 0) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, one_block);
-      if (rc == 0) rc = lib.sglq_silu_and_mul_group_quant_fp8(y1, code, q2, f2, rows, n, 1e-10f, here.stream);
+      if (rc == 0) rc = lib.sglq_silu_and_mul_group_quant_fp8_cm(y1, code, q2, f2, rows, n, 1e-10f, here.stream);
       if (rc == 0) rc = grouped(q2, f2, w2, s2, base, ps2, n, k, plan_rows2, shared_plan);
       if (rc == 0 && float_weights)
         rc = lib.sglq_apply_shuffle_mul_sum_f32(base, out.data_ptr(), slot_map, static_cast<const float*>(weights.data_ptr()), code, m, topk, k,
