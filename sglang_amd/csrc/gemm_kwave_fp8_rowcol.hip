@@ -1,0 +1,7 @@
+#include "gemm_kwave_kernel.h"
+
+namespace sglq {
+
+void launch_kwave_fp8_rowcol(GemmArgs& p, int config, int out_dtype, hipStream_t st) { launch_kwave_kind<KIND_FP8_ROWCOL>(p, config, out_dtype, st); }
+
+}  // namespace sglq

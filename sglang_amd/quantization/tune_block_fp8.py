@@ -30,6 +30,7 @@ import time
 import torch
 
 RING_TILE, RING_CONFIGS = 300, 16  # kernel codes of gemm_ring_kernel's tile shapes
+KWAVE_TILE, KWAVE_CONFIGS = 400, (0, 1, 2, 3, 4, 6, 7, 8)  # ... and of gemm_kwave_kernel's (those of the block-scaled kinds)
 DEFAULT_M = [1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 256, 512, 1024, 1536, 2048, 3072, 4096, 8192]
 
 
@@ -49,6 +50,7 @@ def candidates(m: int, n: int, k: int):
                 out += [(68, 0), (69, 0)]
     if m > 16:
         out += [(RING_TILE + i, 0) for i in range(RING_CONFIGS)]
+        out += [(KWAVE_TILE + i, 0) for i in KWAVE_CONFIGS]
     out += [(128, s) for s in (0, 2, 4) if s == 0 or s <= nkb // 4]
     if k >= 384 and m > 64:
         out += [(130, s) for s in (0, 1, 2, 4, 8) if s <= 1 or (nkb % s == 0 and nkb // s >= 3)]
