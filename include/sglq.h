@@ -444,7 +444,7 @@ void sglq_debug_set_direct_lds(int on);
  * kernel (259 = its variant whose waves write their own outputs out and whose copies run on across tile
  * boundaries: block-scaled FP8 without bias or split-K); 130 = the same kernel with 128-row tiles; 192 / 224 / 257 = the pipelined 4x2-wave
  * kernel with tiles 192 / 224 / 256 wide; 193 = that kernel on 192 x 192 tiles (block-scaled FP8 without a bias).
- * 300 + i / 400 + i = tile shape i of gemm_ring_kernel / gemm_kwave_kernel.
+ * 270 + i / 300 + i = tile shape i of gemm_kwave_kernel / gemm_ring_kernel.
  * A kernel that does not apply to the shape falls through to the next one that does. */
 void sglq_debug_force_tile(int tile);
 /* Test hook: > 0 fixes the split-K factor of the M <= 64 kernels (0 = by shape);

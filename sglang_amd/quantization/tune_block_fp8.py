@@ -30,7 +30,7 @@ import time
 import torch
 
 RING_TILE, RING_CONFIGS = 300, 16  # kernel codes of gemm_ring_kernel's tile shapes
-KWAVE_TILE, KWAVE_CONFIGS = 400, (0, 1, 2, 3, 4, 6, 7, 8)  # ... and of gemm_kwave_kernel's (those of the block-scaled kinds)
+KWAVE_TILE, KWAVE_CONFIGS = 270, (0, 1, 2, 3, 4, 6, 7, 8)  # ... and of gemm_kwave_kernel's (those of the block-scaled kinds)
 DEFAULT_M = [1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 256, 512, 1024, 1536, 2048, 3072, 4096, 8192]
 
 

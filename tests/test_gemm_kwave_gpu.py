@@ -6,7 +6,7 @@ from oracle import w8a8_oracle as O
 from test_gemm_gpu import ATOL, RTOL, make_block_int8_case, rand_i8
 
 pytestmark = pytest.mark.gpu
-KWAVE = 400  # kernel code of configuration 0
+KWAVE = 270  # kernel code of configuration 0
 IN_PLACE_ONLY = (5, 9, 10)  # tile shapes that the block-scaled kinds do not have
 
 
