@@ -61,6 +61,30 @@ struct GemmArgs {
   float quant_eps;  // fused quantization (gemm_stream_quant_kernel): lower bound of a group's abs-max
 };
 
+// Where a tile of weight rows starts its way round K (of `steps` steps).  With weight rows a multiple of 4 KiB apart a K
+// block of every row lies in the same few memory channels, and blocks that start together walk K in step, so they are
+// bound by those channels instead of the memory; each tile starts at a place of its own instead (the golden ratio spreads
+// neighbours).  A plain copy in gemm_stream_kernel's order shows the same: 28672 x 4096 22.7 us in step, 20.5 us so.
+// On that kernel, weights rotated through more than the last-level cache, 1 and 16 rows, before and after: 28672 x 4096
+// 25.7 -> 23.2 and 27.0 -> 24.4 us, 8192 x 4096 9.9 -> 8.7 and 10.2 -> 8.9, 4096 x 4096 5.8 -> 5.2 and 6.0 -> 5.4,
+// 7168 x 16384 26.2 -> 23.9 and 28.0 -> 26.2, 57344 x 8192 80.9 -> 78.5 and 92.8 -> 90.9; nothing on rows of 1, 2, 6, 7
+// or 14 KiB, which stay in order.
+SGLQ_DEV int first_k_step(const GemmArgs& p, uint32_t tile, int steps) {
+  if (p.ldb & 4095) return 0;
+  return (int)(((tile * 40503u & 0xffffu) * (uint32_t)steps) >> 16);  // 40503 / 2^16: the golden ratio
+}
+// ... for kernels whose blocks also share an activation tile, which in step they read from their L2 together: only where
+// the weights are what is read (48 weight rows to an activation row) and the activations stay in the L2 anyway (2 MiB).
+// gemm_ring_kernel, in step and so: 24 x 28672 x 4096 30.6 -> 24.4 us, 64 x 57344 x 8192 107 -> 88, 200 x 14336 x 4096
+// 25.0 -> 22.5, 64 x 8192 x 8192 21.6 -> 19.9; gemm_kwave_kernel: 32 x 14336 x 4096 16.5 -> 14.7, 96 x 28672 x 4096
+// 33.5 -> 29.2; gemm_skinny_kernel without split-K: 64 x 14336 x 4096 18.2 -> 16.1 (with it the splits of a weight tile
+// read neighbouring K blocks already: 40 x 5120 x 8192 16.5 -> 17.7 us, left in step).  Past the bounds it loses:
+// 230 x 6144 x 8192 27.1 -> 29.6 us, 512 x 10240 x 8192 51.2 -> 54.7, 333 x 7168 x 16384 66.7 -> 84.1; another start for
+// each XCD there is no gain either (1024 x 7168 x 16384 119.8 -> 117.8, but 333 rows 66.7 -> 69.2).
+SGLQ_DEV int first_k_step_shared(const GemmArgs& p, uint32_t tile, int steps) {
+  return 48 * (int64_t)p.M <= p.N && p.a_bytes <= 2u << 20 ? first_k_step(p, tile, steps) : 0;
+}
+
 // Grouped GEMM tile plan in the workspace (int32): [0] = number of row tiles, then from [4] on
 // one entry of four per row tile: expert, first row, end row (both absolute rows of A and C).
 constexpr int PLAN_HEADER = 4, PLAN_ENTRY = 4;

@@ -157,8 +157,14 @@ SGLQ_DEV void kwave_body(const GemmArgs& p) {
       }
     }
     // copy j of unit u (both static) of wave K block t into slot `slot`; a K block past the last one is zero fill
-    auto k_offset = [&](int t) -> uint32_t {
-      const int kb = wave + NW * t;
+    const int first = __builtin_amdgcn_readfirstlane(first_k_step_shared(p, (uint32_t)tn, T));
+    const int behind = first * NW + wave, past = behind + NW * T;  // (the t-th K block, once past the last one it is `T` back)
+    auto k_block_at = [&](int t) __attribute__((always_inline)) {
+      const int kb = behind + NW * t;
+      return kb < nkb ? kb : kb < past ? kb - NW * T : nkb;
+    };
+    auto k_offset = [&](int t) __attribute__((always_inline)) -> uint32_t {
+      const int kb = k_block_at(t);
       return kb < nkb ? (uint32_t)kb * 128u : OOB;
     };
     auto copy_unit = [&](auto u_tag, auto j_tag, auto slot_tag, uint32_t k0) __attribute__((always_inline)) {
@@ -168,7 +174,7 @@ SGLQ_DEV void kwave_body(const GemmArgs& p) {
     };
     auto copy_scales = [&](int c, int t) __attribute__((always_inline)) {
       if constexpr (BLOCK) {
-        const int kb = wave + NW * t;
+        const int kb = k_block_at(t);
         const uint32_t dst = ring + NU * 4096 + (uint32_t)(t & (Plan::NSC - 1)) * Plan::SC_BYTES + (uint32_t)c * 256u;
         if (c < Plan::SA_COPIES) lds_copy4(rsa, dst, voff_sa[c], kb < nkb ? (uint32_t)(kb * p.sa_stride_k * 4) : SC_NONE);
         else lds_copy4(rsb, dst, voff_sb, kb < nkb ? (uint32_t)(kb * p.sb_stride_k * 4) : SC_NONE);

@@ -91,6 +91,8 @@ __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs 
   const bool sa_packed = HW && p.sa_packed;  // activation scales as words of four K blocks' exponent bytes
   const int sa_kshift = sa_packed ? 2 : 0;
 
+  const int first = GROUPED ? 0 : __builtin_amdgcn_readfirstlane(first_k_step_shared(p, (uint32_t)tn, T));  // stage t holds K step (t + first) % T
+
   using acc_t = typename std::conditional<float_acc(KIND), v4f, v4i>::type;
   acc_t acc[MI][NI];
   const int kg = wave / (WM * WN), wm = wave % (WM * WN) / WN, wn = wave % WN;
@@ -112,7 +114,10 @@ __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs 
       const int nb = (n0 >> 7) + lane;
       off_sb = (lane < 3 && nb < nblocks) ? (uint32_t)(nb * p.sb_stride_n * 4) : OOB;
     }
-    auto issue = [&](int t, int slot) {
+    int t_copy = first;  // the K step that the next copies bring
+    auto issue = [&](int slot) __attribute__((always_inline)) {
+      const int t = t_copy;
+      t_copy = t + 1 == T ? 0 : t + 1;
       const uint32_t st = base + (uint32_t)slot * STAGE_BYTES;
 #pragma unroll
       for (int j = 0; j < CPW; ++j) {
@@ -154,7 +159,7 @@ __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs 
     };
 #pragma unroll
     for (int t = 0; t < NST - 1; ++t)
-      if (t < T) issue(t, t);
+      if (t < T) issue(t);
     int slot = NST - 1;
     for (int t = 0; t < T; ++t) {
       const int younger = T - 1 - t < NST - 2 ? T - 1 - t : NST - 2;
@@ -165,7 +170,7 @@ __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs 
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       if (t + NST - 1 < T) {
-        issue(t + NST - 1, slot);
+        issue(slot);
         slot = slot + 1 == NST ? 0 : slot + 1;
       }
     }
@@ -212,7 +217,7 @@ __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs 
       int ea[MI], eb[NSB];  // HW: the exponent bytes of the K block's scales
       if constexpr (HW) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i) ea[i] = ue8m0_at(sfa[i], sa_packed ? 8 * ((t * KG + kg) & 3) : 23);
+        for (int i = 0; i < MI; ++i) ea[i] = ue8m0_at(sfa[i], sa_packed ? 8 * (((t + first < T ? t + first : t + first - T) * KG + kg) & 3) : 23);
 #pragma unroll
         for (int j = 0; j < NSB; ++j) eb[j] = ue8m0_of(sfb[j]);
       }
