@@ -46,6 +46,31 @@ def test_grouped_ring_tiles(gpu, rows, nk, dtype):
         torch.testing.assert_close(out[sl].float(), a @ w.t(), rtol=1e-2, atol=1e-2)
 
 
+# an expert's last two 256-row tiles share what is left in multiples of 32 rows, five to eight per half tile: a single tile of each
+# height, two of them around each change of height, whole tiles in front of them; then the same without a next expert's rows behind
+@pytest.mark.parametrize("rows", [[1, 33, 160, 161, 192, 193, 224, 225, 256], [257, 288, 320, 321, 384, 385, 448, 449, 511], [512, 513, 0, 769, 600], [150], [417]])
+@pytest.mark.parametrize("nk", [(384, 384), (512, 1152)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_grouped_256_row_tiles_share_the_last_rows(gpu, rows, nk, dtype):
+    from sglang_amd import _lib
+
+    n, k = nk
+    print("grouped 256-row tiles", rows, n, k, dtype, flush=True)
+    lib = _lib.load()
+    case, cuts, b, sb = grouped_case(gpu, rows, n, k, seed=sum(rows) + n)
+    lib.sglq_debug_grouped_tile(256)
+    try:
+        out = run_grouped(gpu, case, dtype)
+        assert lib.sglq_debug_last_gemm_kernel().decode().endswith("gemm_pipe_kernel<grouped>")
+    finally:
+        lib.sglq_debug_grouped_tile(0)
+    for x, r in enumerate(rows):
+        sl = slice(int(cuts[x]), int(cuts[x + 1]))
+        a = case["a"][sl].float() * case["scales_a"][sl].repeat_interleave(128, dim=1)
+        w = b[x].float() * sb[x].t().repeat_interleave(128, dim=0).repeat_interleave(128, dim=1)[:n]
+        torch.testing.assert_close(out[sl].float(), a @ w.t(), rtol=1e-2, atol=1e-2)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,d", [(1, 128), (15, 384), (33, 256), (100, 1152)])
 def test_column_major_scales(gpu, dtype, m, d):
