@@ -81,9 +81,10 @@ SGLQ_DEV int first_k_step(const GemmArgs& p, uint32_t tile, int steps) {
 // read neighbouring K blocks already: 40 x 5120 x 8192 16.5 -> 17.7 us, left in step).  Past the bounds it loses:
 // 230 x 6144 x 8192 27.1 -> 29.6 us, 512 x 10240 x 8192 51.2 -> 54.7, 333 x 7168 x 16384 66.7 -> 84.1; another start for
 // each XCD there is no gain either (1024 x 7168 x 16384 119.8 -> 117.8, but 333 rows 66.7 -> 69.2).
-SGLQ_DEV int first_k_step_shared(const GemmArgs& p, uint32_t tile, int steps) {
-  return 48 * (int64_t)p.M <= p.N && p.a_bytes <= 2u << 20 ? first_k_step(p, tile, steps) : 0;
+static __host__ __device__ __forceinline__ bool spreads_k_starts(const GemmArgs& p) {
+  return !(p.ldb & 4095) && 48 * (int64_t)p.M <= p.N && p.a_bytes <= 2u << 20;
 }
+SGLQ_DEV int first_k_step_shared(const GemmArgs& p, uint32_t tile, int steps) { return spreads_k_starts(p) ? first_k_step(p, tile, steps) : 0; }
 
 // Grouped GEMM tile plan in the workspace (int32): [0] = number of row tiles, then from [4] on
 // one entry of four per row tile: expert, first row, end row (both absolute rows of A and C).
