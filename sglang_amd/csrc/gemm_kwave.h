@@ -6,8 +6,8 @@
 //   * each of the block's four waves computes the whole tile on every fourth K block, from a ring of its own in LDS that it
 //     fills itself: no barrier in the loop, a wave waits for its own copies only, and every operand byte is read from LDS once
 //     (the ring's eight waves read a 64 x 128 tile's 24 KiB K block as 64 KiB);
-//   * the ring's slots are units of 32 rows (4 KiB), refilled as soon as the MFMAs that use their fragments have been issued, so
-//     that 64-80 KiB per CU are under way whatever the tile;
+//   * the ring's slots are units of 32 rows (4 KiB), refilled as soon as the MFMAs that use their fragments have been issued:
+//     behind a step's refills 80-128 KiB per CU are under way, across a wait 32-96 KiB, two of a wave's units at least;
 //   * one wave per SIMD has all of its registers: 48-192 accumulators, the K block's activations, two units of weights.
 // The partial sums meet in LDS, added in the order of the waves.
 // Bound now: what a CU takes in past the L2, 60-70 GB/s with HBM latency (a build that only copies is as fast; one whose copies

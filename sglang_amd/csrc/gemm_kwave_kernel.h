@@ -16,26 +16,36 @@ struct KwavePlan {
   static constexpr int UA = (MI + 1) / 2, UB = NI / 2, UPB = UA + UB;
   static constexpr int SA_COPIES = (BM + 63) / 64, SCP = BLOCK ? SA_COPIES + 1 : 0;  // copies of a K block's scales
   static constexpr int SC_BYTES = 256 * (SA_COPIES + 1), NSC = BLOCK ? 4 : 0;
+  // first unit (index in the K block) that step b refills, and one past its last; last unit that step b reads: the next
+  // weight unit, or with the K block's last step the next K block's activations and first weight unit
+  static constexpr int refill_from(int b) { return b == 0 ? 0 : b == 1 ? UA - 1 : UA + b - 1; }
+  static constexpr int refill_to(int b) { return b == UB - 1 ? UPB : refill_from(b + 1); }
+  static constexpr int last_read(int b) { return b == UB - 1 ? UPB + UA : UA + b + 1; }
+  // units under way across the wait of every step with a ring of `nu` slots, at least
+  static constexpr int under_way(int nu) {
+    int least = nu;
+    for (int b = 0; b < UB; ++b) least = nu + refill_from(b) - last_read(b) - 1 < least ? nu + refill_from(b) - last_read(b) - 1 : least;
+    return least;
+  }
   // Slots: the code of a K block is repeated for each of the PER positions that it can have in the ring, so that every
-  // slot is a constant; the ring is what fits, shortened by up to two slots where that needs fewer repetitions.
+  // slot is a constant; the ring is what fits, shortened by up to two slots where that needs fewer repetitions and two units
+  // stay under way across every wait.  Fewer repetitions are worth 2-3 % (block-FP8 on 64 x 64 tiles, eight slots and two of
+  // them against nine and nine); a ring that a wait drains costs more (80 x 64 and 96 x 64, seven slots: 9 % slower than nine
+  // on average of 34 shapes, 33 % at most; in place 112 x 64 and 128 x 64, one unit left: 1 %).
   static constexpr int gcd(int x, int y) { return y == 0 ? x : gcd(y, x % y); }
   static constexpr int period(int nu) { return nu / gcd(nu, UPB); }
   static constexpr int NU_MAX = (160 * 1024 / 4 - NSC * SC_BYTES) / 4096;
-  static constexpr int shorter(int x, int y) { return y >= UPB && period(y) < period(x) ? y : x; }
+  static constexpr int shorter(int x, int y) { return under_way(y) >= 2 && period(y) < period(x) ? y : x; }
   static constexpr int NU = shorter(shorter(NU_MAX, NU_MAX - 1), NU_MAX - 2), PER = period(NU);
+  static_assert(NU >= UPB && under_way(NU) >= 2, "a wait does not drain the ring");
   static constexpr int WAVE_BYTES = NU * 4096 + NSC * SC_BYTES;
   static_assert(UB >= 2 && NI % 4 == 0 && (NU + UPB - 1) / UPB <= 4, "steps, the waves' shares of the columns, slots of scales");
-  // first unit (index in the K block) that step b refills, and one past its last
-  static constexpr int refill_from(int b) { return b == 0 ? 0 : b == 1 ? UA - 1 : UA + b - 1; }
-  static constexpr int refill_to(int b) { return b == UB - 1 ? UPB : refill_from(b + 1); }
   // copies of unit u, counted on over the K blocks (a K block's scales go in front of its first unit)
   static constexpr int copies(int u) { return (u % UPB == UA - 1 && (MI & 1) ? 2 : 4) + (u % UPB == 0 ? SCP : 0); }
-  // copies under way when step b starts that are younger than the last unit it reads: the next weight unit, or with the
-  // K block's last step the next K block's activations and first weight unit
+  // copies under way when step b starts that are younger than the last unit it reads
   static constexpr int younger(int b) {
-    const int last_read = b == UB - 1 ? UPB + UA : UA + b + 1;
     int n = 0;
-    for (int u = last_read + 1; u < NU + refill_from(b); ++u) n += copies(u);
+    for (int u = last_read(b) + 1; u < NU + refill_from(b); ++u) n += copies(u);
     return n;
   }
   // refill copies of step b in the order in which they are issued: number, and for copy c its unit and its index there
