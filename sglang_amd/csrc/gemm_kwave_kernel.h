@@ -39,7 +39,7 @@ struct KwavePlan {
   static constexpr int NU = shorter(shorter(NU_MAX, NU_MAX - 1), NU_MAX - 2), PER = period(NU);
   static_assert(NU >= UPB && under_way(NU) >= 2, "a wait does not drain the ring");
   static constexpr int WAVE_BYTES = NU * 4096 + NSC * SC_BYTES;
-  static_assert(UB >= 2 && NI % 4 == 0 && (NU + UPB - 1) / UPB <= 4, "steps, the waves' shares of the columns, slots of scales");
+  static_assert(UB >= 2 && NI % 4 == 0 && (NU + UPB - 1) / UPB <= 4, "an even number of steps, the waves' shares of the columns, slots of scales");
   // copies of unit u, counted on over the K blocks (a K block's scales go in front of its first unit)
   static constexpr int copies(int u) { return (u % UPB == UA - 1 && (MI & 1) ? 2 : 4) + (u % UPB == 0 ? SCP : 0); }
   // copies under way when step b starts that are younger than the last unit it reads
@@ -109,7 +109,7 @@ SGLQ_DEV void kwave_body(const GemmArgs& p) {
   constexpr int IMG_PITCH = BN * 2 + 16;
   constexpr int LDS = 160 * 1024;  // the rings; then partial sums and the output's image
   static_assert(NW * Plan::WAVE_BYTES <= LDS && BM * IMG_PITCH <= LDS, "LDS");
-  static_assert(!BLOCK || BN == 64 || BN % 128 == 0, "a fragment's block of weight scales is known at compile time");
+  static_assert(!BLOCK || BN == 64 || BN == 128, "a tile's columns lie in one block of weight scales");
   __shared__ __attribute__((aligned(1024))) char smem[LDS];
 
   const int lane = threadIdx.x & 63;
@@ -158,8 +158,7 @@ SGLQ_DEV void kwave_body(const GemmArgs& p) {
       const int nblocks = (p.N + 127) >> 7;
       rsa = make_rsrc_sgpr(p.sa, (uint32_t)(((int64_t)(p.M - 1) * p.sa_stride_m + (int64_t)(nkb - 1) * p.sa_stride_k + 1) * 4));
       rsb = make_rsrc_sgpr(p.sb, (uint32_t)(((int64_t)(nblocks - 1) * p.sb_stride_n + (int64_t)(nkb - 1) * p.sb_stride_k + 1) * 4));
-      const int nb = (n0 >> 7) + lane;
-      if (lane < 2 && nb < nblocks) voff_sb = (uint32_t)(nb * p.sb_stride_n * 4);
+      if (lane == 0) voff_sb = (uint32_t)((n0 >> 7) * p.sb_stride_n * 4);
 #pragma unroll
       for (int c = 0; c < Plan::SA_COPIES; ++c) {
         const int row = m0 + c * 64 + lane;
@@ -200,15 +199,14 @@ SGLQ_DEV void kwave_body(const GemmArgs& p) {
       return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     };
     v8i a[MI], w[2][2];  // w[b & 1]: weight unit b
-    float sfa[MI], sfb[2];
+    float sfa[MI], sfb;
     const char* const sc_rd = smem + wave * Plan::WAVE_BYTES + NU * 4096;
     auto read_scales = [&](int t) __attribute__((always_inline)) {
       if constexpr (BLOCK) {
         const char* s = sc_rd + (t & (Plan::NSC - 1)) * Plan::SC_BYTES;
 #pragma unroll
         for (int i = 0; i < MI; ++i) sfa[i] = *reinterpret_cast<const float*>(s + (i * 16 + r16) * 4);
-        sfb[0] = *reinterpret_cast<const float*>(s + Plan::SA_COPIES * 256);
-        if constexpr (BN > 128) sfb[1] = *reinterpret_cast<const float*>(s + Plan::SA_COPIES * 256 + 4);
+        sfb = *reinterpret_cast<const float*>(s + Plan::SA_COPIES * 256);
       }
     };
 
@@ -237,7 +235,7 @@ SGLQ_DEV void kwave_body(const GemmArgs& p) {
       const uint32_t k_refill[3] = {k_offset(t + NU / UPB), k_offset(t + NU / UPB + 1), k_offset(t + NU / UPB + 2)};
       static_for<UB>([&](auto b_tag) __attribute__((always_inline)) {
         constexpr int b = decltype(b_tag)::value;
-        constexpr bool last = b == UB - 1, new_scale = (b * 32) % 128 == 0;  // (the first unit of a block of weight scales)
+        constexpr bool last = b == UB - 1;
         // the next unit has landed (with the last step: the next K block's activations too); this wave alone uses the ring
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Plan::younger(b)) : "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -250,13 +248,9 @@ SGLQ_DEV void kwave_body(const GemmArgs& p) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) d[e] = __builtin_fmaf(block_value<KIND>(part[(2 * MI * fb + q) % (LAG + 1)][e]), sc[q / 2], d[e]);
         };
-        if constexpr (FOLD && new_scale) {
-          if constexpr (b > 0) {  // (the folds that are left need the old product)
+        if constexpr (FOLD && b == 0) {
 #pragma unroll
-            for (int q = 2 * MI - LAG; q < 2 * MI; ++q) fold(q, b - 1);
-          }
-#pragma unroll
-          for (int i = 0; i < MI; ++i) sc[i] = sfa[i] * sfb[b / 4];
+          for (int i = 0; i < MI; ++i) sc[i] = sfa[i] * sfb;
         }
         __builtin_amdgcn_sched_barrier(0);
         static_for<2 * MI>([&](auto q_tag) __attribute__((always_inline)) {
@@ -286,7 +280,7 @@ SGLQ_DEV void kwave_body(const GemmArgs& p) {
           });
           if constexpr (FOLD) {
             if constexpr (q >= LAG) fold(q - LAG, b);
-            else if constexpr (b > 0 && !new_scale) fold(2 * MI + q - LAG, b - 1);
+            else if constexpr (b > 0) fold(2 * MI + q - LAG, b - 1);
           }
           __builtin_amdgcn_sched_barrier(0);
         });
@@ -298,11 +292,6 @@ SGLQ_DEV void kwave_body(const GemmArgs& p) {
           }
         }
       });
-      // (an odd number of steps: the next K block's first unit waits in the other pair of registers)
-      if constexpr (UB & 1) {
-        w[0][0] = w[1][0];
-        w[0][1] = w[1][1];
-      }
     };
     int t = 0;
     while (true) {
