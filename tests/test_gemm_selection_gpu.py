@@ -1,0 +1,61 @@
+"""Which kernel takes a GEMM, at shapes on both sides of a rule's line: the kernel is named and the result compared with the
+generic kernel's."""
+import pytest
+import torch
+
+from test_gemm_ring_gpu import pow2_operands
+
+pytestmark = pytest.mark.gpu
+STREAM_32, SPLIT_K = "gemm_stream_kernel<32 rows>", "gemm_skinny_kernel+splitk_reduce_kernel"
+
+
+def operands(gpu, kind, m, n, k):
+    """The call of the operator for `kind` on random operands."""
+    from sglang_amd.quantization.int8_kernel import w8a8_block_int8_matmul
+    from sglang_amd.sgl_kernel import fp8_blockwise_scaled_mm, fp8_scaled_mm, int8_scaled_mm
+    from sglang_amd.sgl_kernel.gemm import fp8_blockwise_scaled_mm_ue8m0
+
+    a, w, sfa, sfb = pow2_operands(gpu, m, n, k)
+    if kind == "pow2":
+        return lambda: fp8_blockwise_scaled_mm_ue8m0(a, w.t(), sfa, sfb.t(), torch.bfloat16)
+    g = torch.Generator(device=gpu).manual_seed(n)
+    if kind == "block":
+        sfa, sfb = sfa * torch.rand(sfa.shape, generator=g, device=gpu).t().contiguous().t(), sfb * torch.rand(sfb.shape, generator=g, device=gpu)
+        return lambda: fp8_blockwise_scaled_mm(a, w.t(), sfa, sfb.t(), torch.bfloat16)
+    sa, sb = torch.rand((m, 1), generator=g, device=gpu) * 0.01 + 1e-3, torch.rand((n, 1), generator=g, device=gpu) * 0.01 + 1e-3
+    if kind == "fp8":
+        return lambda: fp8_scaled_mm(a, w.t(), sa, sb, torch.bfloat16, None)
+    a8, w8 = (torch.randint(-128, 128, s, generator=g, device=gpu, dtype=torch.int8) for s in ((m, k), (n, k)))
+    if kind == "i8":
+        return lambda: int8_scaled_mm(a8, w8.t(), sa * 0.05, sb, torch.bfloat16, None)
+    return lambda: w8a8_block_int8_matmul(a8, w8, sfa * 0.05, sfb * 0.05, [128, 128], torch.bfloat16)
+
+
+CASES = [
+    # 33 to 64 rows, 7/8 of a round of 32-row blocks that start K apart: up to K = 16384, on all of these rows
+    ("block", 64, 7424, 16384, STREAM_32),
+    ("fp8", 56, 7680, 16384, STREAM_32),
+    ("block", 49, 7168, 8192, STREAM_32),
+    ("block", 48, 7424, 20480, SPLIT_K),
+    ("i8", 40, 7168, 28672, SPLIT_K),
+]
+
+
+@pytest.mark.parametrize("kind,m,n,k,kernel", CASES)
+def test_the_rules_choose(gpu, kind, m, n, k, kernel):
+    from sglang_amd import _lib
+
+    print("selection", kind, m, n, k, flush=True)
+    lib = _lib.load()
+    call = operands(gpu, kind, m, n, k)
+    out = call()
+    assert lib.sglq_debug_last_gemm_kernel().decode() == kernel
+    lib.sglq_debug_force_tile(128)
+    try:
+        ref = call()
+    finally:
+        lib.sglq_debug_force_tile(0)
+    # (two float32 sums of the same products, each rounded once to bf16: a bf16 step is 2^-8 of the value; what cancels
+    # in a sum is bounded by the size of the others)
+    assert bool(torch.isfinite(ref).all())
+    torch.testing.assert_close(out.float(), ref.float(), rtol=1e-2, atol=1e-3 * float(ref.float().std()))

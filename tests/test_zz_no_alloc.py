@@ -36,7 +36,7 @@ def test_noalloc_entry_point_matches_the_workspace_entry_point(gpu):
     workspace = torch.empty(SCRATCH_BYTES, dtype=torch.uint8, device=gpu)
     # split-K decode kernel (4 splits), then the pipelined kernel with K split over work units,
     # then a smaller split-K problem whose partial sums land on the first calls' leftovers
-    shapes = [(64, 7168, 16384), (1024, 2048, 16384), (40, 2048, 16384), (64, 7168, 16384), (8, 2112, 7168)]
+    shapes = [(64, 7168, 20480), (1024, 2048, 16384), (40, 2048, 16384), (64, 7168, 20480), (8, 2112, 7168)]
     for i, (m, n, k) in enumerate(shapes):
         print(f"noalloc case {i}: {m} x {n} x {k}", flush=True)
         xq, xs, wq, ws, dxq, dxs, dwq, dws = _case(m, n, k, 9000 + 10 * i, gpu)
@@ -65,7 +65,7 @@ def test_noalloc_entry_point_allocates_nothing_and_replays_in_a_graph(gpu):
 
     lib = _lib.load()
     assert lib.sglq_init() == 0, lib.sglq_last_error()
-    m, n, k = 64, 7168, 16384
+    m, n, k = 64, 7168, 20480
     print(f"noalloc under capture: {m} x {n} x {k}", flush=True)
     xq, xs, wq, ws, dxq, dxs, dwq, dws = _case(m, n, k, 9100, gpu)
     xq2, xs2, _, _, dxq2, dxs2, _, _ = _case(m, 128, k, 9200, gpu)
