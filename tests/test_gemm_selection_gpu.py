@@ -6,7 +6,8 @@ import torch
 from test_gemm_ring_gpu import pow2_operands
 
 pytestmark = pytest.mark.gpu
-STREAM_32, SPLIT_K = "gemm_stream_kernel<32 rows>", "gemm_skinny_kernel+splitk_reduce_kernel"
+STREAM_32 = "gemm_stream_kernel<32 rows>"
+SPLIT_K, SPLIT_K_64 = "gemm_skinny_kernel+splitk_reduce_kernel", "gemm_skinny_kernel<64 columns>+splitk_reduce_kernel"
 
 
 def operands(gpu, kind, m, n, k):
@@ -38,6 +39,16 @@ CASES = [
     ("block", 49, 7168, 8192, STREAM_32),
     ("block", 48, 7424, 20480, SPLIT_K),
     ("i8", 40, 7168, 28672, SPLIT_K),
+    # few tiles and a long K: a CU's intake bounds gemm_kwave_kernel, the split-K kernel and the ring keep what it had taken;
+    # where its tiles fill the chip, or K is short, it stays
+    ("i8block", 86, 1216, 7936, SPLIT_K_64),
+    ("i8block", 119, 1472, 6784, SPLIT_K_64),
+    ("block", 117, 2048, 8192, SPLIT_K_64),
+    ("fp8", 201, 1152, 8192, "gemm_ring_kernel"),
+    ("block", 630, 1280, 4608, "gemm_kwave_kernel"),
+    ("block", 333, 4096, 7040, "gemm_kwave_kernel"),
+    ("fp8", 277, 2112, 6400, "gemm_kwave_kernel"),
+    ("i8", 506, 1920, 8576, "gemm_kwave_kernel"),
 ]
 
 
