@@ -1,5 +1,7 @@
 """Which kernel takes a GEMM, at shapes on both sides of a rule's line: the kernel is named and the result compared with the
 generic kernel's."""
+import ctypes
+
 import pytest
 import torch
 
@@ -50,6 +52,43 @@ CASES = [
     ("fp8", 277, 2112, 6400, "gemm_kwave_kernel"),
     ("i8", 506, 1920, 8576, "gemm_kwave_kernel"),
 ]
+
+PIPE_128 = "gemm_pipe_kernel<128 rows>+splitk_reduce_kernel"
+# Power-of-two scales on up to 128 rows: the pipelined 128-row kernel applies them in the MFMA and reads packed words as they are,
+# gemm_kwave_kernel and the ring fold them and take packed words expanded by a launch in front
+SCALED = [
+    (112, 11264, 8192, PIPE_128, PIPE_128),
+    (92, 8704, 8192, "gemm_kwave_kernel", PIPE_128),
+    (128, 16384, 4096, "gemm_ring_kernel", "gemm_ring_kernel"),
+    (96, 11648, 5504, "gemm_kwave_kernel", "gemm_kwave_kernel"),
+]
+
+
+@pytest.mark.parametrize("m,n,k,kernel,packed_kernel", SCALED)
+def test_power_of_two_scales_up_to_128_rows(gpu, m, n, k, kernel, packed_kernel):
+    """Same kernel for scales as fp32 and as packed words, unless the expansion costs more than the kernel gains."""
+    from sglang_amd import _lib
+    from sglang_amd.sgl_kernel import fp8_blockwise_scaled_mm
+    from sglang_amd.sgl_kernel.gemm import fp8_blockwise_scaled_mm_ue8m0
+
+    print("selection, power-of-two scales", m, n, k, flush=True)
+    lib = _lib.load()
+    a, w, sfa, sfb = pow2_operands(gpu, m, n, k)
+    plain = fp8_blockwise_scaled_mm(a, w.t(), sfa, sfb.t(), torch.bfloat16)
+    out = fp8_blockwise_scaled_mm_ue8m0(a, w.t(), sfa, sfb.t(), torch.bfloat16)
+    assert lib.sglq_debug_last_gemm_kernel().decode() == kernel
+    assert bool(lib.sglq_debug_last_gemm_hw_scaled()) == (kernel == PIPE_128)
+    kb = k // 128
+    codes = torch.zeros((m, (kb + 3) // 4 * 4), dtype=torch.uint8, device=gpu)
+    codes[:, :kb] = (sfa.contiguous().view(torch.int32) >> 23).to(torch.uint8)
+    words = codes.view(torch.int32).t().contiguous()
+    scratch, packed_out = torch.empty(64 << 20, dtype=torch.uint8, device=gpu), torch.empty_like(out)
+    rc = lib.sglq_fp8_blockwise_scaled_mm_ue8m0_packed(a.data_ptr(), k, w.data_ptr(), k, words.data_ptr(), 1, m, sfb.data_ptr(), 1, kb, packed_out.data_ptr(), n, 0, m, n, k,
+                                                       scratch.data_ptr(), scratch.numel(), ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream))
+    assert rc == 0 and lib.sglq_debug_last_gemm_kernel().decode() == packed_kernel
+    assert bool(lib.sglq_debug_last_gemm_hw_scaled()) == (packed_kernel == PIPE_128)
+    for got in (out, packed_out):
+        torch.testing.assert_close(got.float(), plain.float(), rtol=1e-2, atol=1e-3 * float(plain.float().std()))
 
 
 @pytest.mark.parametrize("kind,m,n,k,kernel", CASES)
