@@ -59,6 +59,7 @@ struct GemmArgs {
   int sa_packed;
   float* sa_expanded;  // room for [M, K / 128] fp32 scales (sa_packed only)
   float quant_eps;  // fused quantization (gemm_stream_quant_kernel): lower bound of a group's abs-max
+  int cus;          // compute units of the call's device (host: the choice of a kernel and its grid)
 };
 
 // Where a tile of weight rows starts its way round K (of `steps` steps).  With weight rows a multiple of 4 KiB apart a K
