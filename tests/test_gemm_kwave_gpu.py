@@ -78,3 +78,39 @@ def test_kwave_kernel_reads_strided_operands(gpu):
     assert rc == 0 and lib.sglq_debug_last_gemm_kernel().decode() == "gemm_kwave_kernel"
     torch.testing.assert_close(out[:, :n].cpu().float(), ref, rtol=RTOL, atol=ATOL)
     assert bool((out[:, n:] == 7.0).all())
+
+
+# the entry points that only the tile's epilogue or a launch in front sets apart; both output types, M and N cut
+@pytest.mark.parametrize("config", [c for c in range(11) if c not in IN_PLACE_ONLY])
+def test_kwave_kernel_block_int8_bias_and_packed_scales(gpu, config):
+    import ctypes
+
+    from sglang_amd import _lib
+    from sglang_amd.quantization.int8_kernel import w8a8_block_int8_matmul
+    from test_gemm_ring_gpu import pow2_operands
+
+    m, n, k = 130, 264, 1408
+    print("kwave kernel, block-INT8 bias, packed scales", config, flush=True)
+    lib = _lib.load()
+    x8, s8, wq8, ws8 = make_block_int8_case(m, n, k, seed=config)
+    a, w, sfa, sfb = pow2_operands(gpu, m, n, k)
+    kb = k // 128
+    codes = torch.zeros((m, (kb + 3) // 4 * 4), dtype=torch.uint8)
+    codes[:, :kb] = (sfa.cpu().contiguous().view(torch.int32) >> 23).to(torch.uint8)
+    words, scratch = codes.view(torch.int32).t().contiguous().to(gpu), torch.empty(4 * m * kb + 4096, dtype=torch.uint8, device=gpu)
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=gpu)
+    lib.sglq_debug_force_tile(KWAVE + config)
+    try:
+        for dtype in (torch.bfloat16, torch.float16):
+            bias = (torch.randn(n, generator=torch.Generator().manual_seed(config)) * 0.1).to(dtype)
+            ref = O.w8a8_block_int8_matmul(x8, wq8, s8, ws8, torch.float32, acc_dtype=torch.float64) + bias.float()
+            got = w8a8_block_int8_matmul(x8.to(gpu), wq8.to(gpu), s8.to(gpu), ws8.to(gpu), [128, 128], dtype, bias=bias.to(gpu))
+            assert lib.sglq_debug_last_gemm_kernel().decode() == "gemm_kwave_kernel"
+            torch.testing.assert_close(got.cpu().float(), ref, rtol=RTOL, atol=2 * ATOL)  # (rounded twice: the product, then with the bias)
+        rc = lib.sglq_fp8_blockwise_scaled_mm_ue8m0_packed(a.data_ptr(), k, w.data_ptr(), k, words.data_ptr(), 1, m, sfb.data_ptr(), 1, kb, out.data_ptr(), n, 0, m, n, k,
+                                                           scratch.data_ptr(), scratch.numel(), ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream))
+        assert rc == 0 and lib.sglq_debug_last_gemm_kernel().decode() == "gemm_kwave_kernel" and not lib.sglq_debug_last_gemm_hw_scaled()
+    finally:
+        lib.sglq_debug_force_tile(0)
+    ref = O.fp8_blockwise_scaled_mm(a.cpu(), w.cpu().t(), sfa.cpu(), sfb.cpu().t(), torch.float32, acc_dtype=torch.float64)
+    torch.testing.assert_close(out.cpu().float(), ref, rtol=RTOL, atol=ATOL)
