@@ -47,6 +47,8 @@ CASES = [
     ("i8block", 119, 1472, 6784, SPLIT_K_64),
     ("block", 117, 2048, 8192, SPLIT_K_64),
     ("fp8", 201, 1152, 8192, "gemm_ring_kernel"),
+    ("fp8", 512, 512, 7168, "gemm_ring_kernel"),
+    ("fp8", 128, 2112, 7168, SPLIT_K_64),
     ("block", 630, 1280, 4608, "gemm_kwave_kernel"),
     ("block", 333, 4096, 7040, "gemm_kwave_kernel"),
     ("fp8", 277, 2112, 6400, "gemm_kwave_kernel"),
