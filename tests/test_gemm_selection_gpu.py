@@ -63,6 +63,7 @@ SCALED = [
     (92, 8704, 8192, "gemm_kwave_kernel", PIPE_128),
     (128, 16384, 4096, "gemm_ring_kernel", "gemm_ring_kernel"),
     (96, 11648, 5504, "gemm_kwave_kernel", "gemm_kwave_kernel"),
+    (128, 13824, 5120, "gemm_kwave_kernel", "gemm_kwave_kernel"),
 ]
 
 
