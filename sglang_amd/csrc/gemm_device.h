@@ -65,7 +65,8 @@ struct GemmArgs {
 // Where a tile of weight rows starts its way round K (of `steps` steps).  With weight rows a multiple of 4 KiB apart a K
 // block of every row lies in the same few memory channels, and blocks that start together walk K in step, so they are
 // bound by those channels instead of the memory; each tile starts at a place of its own instead (the golden ratio spreads
-// neighbours).  A plain copy in gemm_stream_kernel's order shows the same: 28672 x 4096 22.7 us in step, 20.5 us so.
+// neighbours).  A plain copy in gemm_stream_kernel's order shows the same: 28672 x 4096 in blocks of 16 rows 22.0 us in step, 20.5 us so,
+// of 32 rows 23.2 and 20.8.
 // On that kernel, weights rotated through more than the last-level cache, 1 and 16 rows, before and after: 28672 x 4096
 // 25.7 -> 23.2 and 27.0 -> 24.4 us, 8192 x 4096 9.9 -> 8.7 and 10.2 -> 8.9, 4096 x 4096 5.8 -> 5.2 and 6.0 -> 5.4,
 // 7168 x 16384 26.2 -> 23.9 and 28.0 -> 26.2, 57344 x 8192 80.9 -> 78.5 and 92.8 -> 90.9; nothing on rows of 1, 2, 6, 7
