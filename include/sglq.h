@@ -194,8 +194,8 @@ int sglq_fp8_blockwise_scaled_mm_bias(const void* a, int64_t lda, const void* b,
  *   b, sfb, bias (may be NULL), out: as sglq_fp8_blockwise_scaled_mm_bias
  *   eps  lower bound of a group's abs-max (the callers' 1e-10)
  * Where it was measured faster (16-bit activations, shapes that the decode kernel without split-K
- * takes: up to 4 rows with one to 2.5 blocks per compute unit, or with K <= 4096 and N >= 1024; up to 8 rows
- * with K <= 4096, N >= 1024 and M * K <= 8192 or N <= 4096), one
+ * takes: one row; up to 4 rows with N >= 1024 and K <= 4096 or a block for every compute unit; up to 8 rows
+ * with K <= 4096, N >= 1024 and K >= 3072, M * K <= 8192 or N <= 4096), one
  * kernel quantizes each K block's activations in LDS right before multiplying them: no
  * quantization launch, no round trip of codes and scales through memory, no workspace.  Other
  * shapes run the quantization kernel and the GEMM one after the other; their codes and
@@ -216,8 +216,8 @@ int sglq_w8a8_block_fp8_linear(const void* x, int in_dtype, const void* b, int64
  * (sgl-kernel/csrc/cpu/gemm_int8.cpp:423-489).
  *   x    [M, K] contiguous activations, in_dtype in {BF16, FP16, FP32}, 16-byte aligned
  *   b, scales_b, bias (may be NULL), out: as sglq_int8_scaled_mm / sglq_fp8_scaled_mm
- * For M <= 2, and M <= 4 with M * K <= 8192 and N <= 4096 (16-bit activations, K % 128 == 0), on the shapes
- * that the decode kernel without split-K takes, one kernel forms the rows' scales in its prologue and quantizes each K block's
+ * For M <= 2, M <= 4 with K >= 2304 or with M * K <= 8192 and N <= 4096, and M <= 8 with 2304 <= K <= 4096 (FP8: 8192)
+ * (16-bit activations, K % 128 == 0), on the shapes that the decode kernel without split-K takes, one kernel forms the rows' scales in its prologue and quantizes each K block's
  * activations in LDS right before multiplying them: no quantization launch, no round trip of codes
  * and scales through memory, no workspace.  Other shapes run the quantization kernel and the GEMM
  * one after the other; their codes and row scales need M * K + 4 * M bytes (each rounded up to

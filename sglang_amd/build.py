@@ -25,7 +25,8 @@ NATIVE_PATH = PKG_DIR / "_native.so"
 SOURCES = ["gemm.hip", "gemm_ring_fp8_block.hip", "gemm_ring_fp8_block_grouped.hip", "gemm_ring_fp8_block_pow2.hip",
            "gemm_ring_fp8_rowcol.hip", "gemm_ring_i8_rowcol.hip",
            "gemm_ring_i8_block.hip",
-           *(f"gemm_kwave_{kind}.hip" for kind in ("fp8_block", "fp8_rowcol", "i8_rowcol", "i8_block")), "common.hip", "quant.hip", "moe.hip"]
+           *(f"gemm_kwave_{kind}.hip" for kind in ("fp8_block", "fp8_rowcol", "i8_rowcol", "i8_block")),
+           *(f"gemm_stream_linear_{kind}.hip" for kind in ("fp8_block", "fp8_token", "i8_token")), "common.hip", "quant.hip", "moe.hip"]
 BENCH_SOURCES = ["bench_kernels.hip"]
 
 HIPCC_FLAGS = [

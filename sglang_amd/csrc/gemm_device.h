@@ -3,10 +3,21 @@
 // head of gemm.hip).
 #pragma once
 #include <type_traits>
+#include <utility>
 
 #include "sglq_common.h"
 
 namespace sglq {
+
+// f(0), f(1) ... f(N - 1), each with its index as a constant
+template <int... I, typename F>
+SGLQ_DEV void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+SGLQ_DEV void static_for(F&& f) {
+  static_for_impl(std::make_integer_sequence<int, N>{}, f);
+}
 
 constexpr int KIND_FP8_BLOCK = 0;   // a4: sum_kb P_kb * sfa[m,kb] * sfb[kb,n/128]
 constexpr int KIND_FP8_ROWCOL = 1;  // a6: sa[m] * (sb[n] * acc) + bias[n]

@@ -1,7 +1,5 @@
 // gemm_kwave_kernel (see gemm_kwave.h) and its launcher for one kind.
 #pragma once
-#include <utility>
-
 #include "gemm_kwave.h"
 
 namespace sglq {
@@ -87,15 +85,6 @@ struct KwavePlan {
 template <int DST>
 SGLQ_DEV void lds_copy16_at(v4u rsrc, uint32_t base, uint32_t voff, uint32_t soff) {
   asm volatile("s_add_u32 m0, %0, %4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" : : "s"(base), "v"(voff), "s"(rsrc), "s"(soff), "n"(DST) : "memory", "scc");
-}
-
-template <int... I, typename F>
-SGLQ_DEV void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-SGLQ_DEV void static_for(F&& f) {
-  static_for_impl(std::make_integer_sequence<int, N>{}, f);
 }
 
 template <int KIND, int OUT_DT, int MI, int NI>
