@@ -173,51 +173,81 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_place_kernel(const int* __res
 }
 
 // ---------------------------------------------------------------------------
-// The same tables, the -1 default of output_permutation and the grouped GEMMs' tile plan from one block,
+// The same tables, the -1 default of output_permutation and the grouped GEMMs' tile plan in one launch,
 // for up to 32768 slots and 512 experts.  A decode step's layer is a chain of short dependent launches,
 // each of 2-5 us whatever it does (16 tokens, 32 experts: the fill of c_map, the three launches above and
-// two plan launches were 28 of the layer's 273 us); one block does their work in one of them.
-// Sixteen waves take consecutive ranges of slots and keep their ids in registers; counts per (wave, expert)
-// through LDS atomics (sums: the order does not matter), a running sum over waves and experts, then every
+// two plan launches were 28 of the layer's 273 us).
+// A block places the slots of one segment.  Sixteen waves take consecutive ranges of it and keep their ids in registers; counts per
+// (wave, expert) through LDS atomics (sums: the order does not matter), a running sum over waves and experts, then every
 // wave walks its slots again in order: lanes that name the same expert find each other with one ballot per
-// id bit, so positions follow slot order as above.
+// id bit, so positions follow slot order as above.  That walk is a chain of LDS round trips, 64 slots of a wave at a time, and what a long
+// prompt's tables spent their time on; so above 2048 slots there are several segments, and each block counts all slots
+// for itself, which needs no exchange between blocks: a slot adds 1 to its expert's word, and 65536 more where it lies in front
+// of the block's segment.  One block -> segments of 1024 slots (us): 5600 slots of 64 experts 9.7 -> 7.3, 20000 of 32 17.5 -> 9.3, 32768 of 32
+// 24.7 -> 11.3 (of 2048 slots 11.8, of 4096 12.9); 128 slots, where no step that there are no slots for is walked any more, 6.5 -> 5.7.
 // ---------------------------------------------------------------------------
 constexpr int TABLE_THREADS = 1024, TABLE_WAVES = TABLE_THREADS / 64, TABLE_STEPS = 32;
 constexpr int TABLE_MAX_SLOTS = TABLE_THREADS * TABLE_STEPS, TABLE_MAX_EXPERTS = 512;
+// (several segments double the LDS: 32 KiB at 256 experts, from there on one)
+constexpr int TABLE_ONE_SEGMENT = 2048, TABLE_SEGMENT = TABLE_THREADS, TABLE_SEGMENTS_EXPERTS = 256;
 
 __global__ __launch_bounds__(TABLE_THREADS) void moe_tables_kernel(const int* __restrict__ topk_ids, int* __restrict__ expert_offsets,
                                                                    int* __restrict__ ps1, int* __restrict__ ps2,
                                                                    int* __restrict__ output_permutation, int topk_length,
                                                                    int num_experts, int id_bits, int n, int k, int* __restrict__ plan,
-                                                                   int plan_rows, int plan_max_tiles) {
-  extern __shared__ int counts[];  // [TABLE_WAVES][num_experts]: first the counts, then the next position of each
+                                                                   int plan_rows, int plan_max_tiles, int segment) {
+  // [TABLE_WAVES][num_experts]: first the segment's counts, then the next position of each; of several segments, all slots' behind them
+  extern __shared__ int counts[];
   __shared__ int wave_rows[TABLE_WAVES], wave_tiles[TABLE_WAVES];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int steps = (topk_length + TABLE_THREADS - 1) / TABLE_THREADS;  // 64 slots each, per wave
-  const int first = wave * steps * 64;
+  const int begin_slot = (int)blockIdx.x * segment, end_slot = begin_slot + segment < topk_length ? begin_slot + segment : topk_length;
+  const bool alone = gridDim.x == 1;
+  const int steps = segment / TABLE_THREADS;  // 64 slots each, per wave
+  const int first = begin_slot + wave * steps * 64;
   int id[TABLE_STEPS];
 #pragma unroll
   for (int s = 0; s < TABLE_STEPS; ++s) {
     const int i = first + s * 64 + lane;
-    id[s] = s < steps && i < topk_length ? topk_ids[i] : -1;
+    id[s] = s < steps && i < end_slot ? topk_ids[i] : -1;
   }
-  for (int i = tid; i < TABLE_WAVES * num_experts; i += TABLE_THREADS) counts[i] = 0;
+  int* const all = counts + TABLE_WAVES * num_experts;
+  for (int i = tid; i < (alone ? 1 : 2) * TABLE_WAVES * num_experts; i += TABLE_THREADS) counts[i] = 0;
   __syncthreads();
   int* mine = counts + wave * num_experts;
 #pragma unroll
-  for (int s = 0; s < TABLE_STEPS; ++s)
+  for (int s = 0; s < TABLE_STEPS; ++s) {
+    if (s >= steps) break;
     if ((uint32_t)id[s] < (uint32_t)num_experts) atomicAdd(mine + id[s], 1);
+  }
+  if (!alone) {
+    int* const mine_all = all + wave * num_experts;
+#pragma unroll 8
+    for (int i = tid; i < topk_length; i += TABLE_THREADS) {
+      const int e = topk_ids[i];
+      if ((uint32_t)e < (uint32_t)num_experts) atomicAdd(mine_all + e, i < begin_slot ? 65537 : 1);
+    }
+  }
   __syncthreads();
   // one thread per expert (num_experts <= 512): rows and tiles, then their running sums over the block
   int rows = 0, tiles = 0;
   if (tid < num_experts) {
+    int before = 0;  // this expert's slots in earlier segments, then in earlier waves too
+    if (!alone) {
+#pragma unroll
+      for (int w = 0; w < TABLE_WAVES; ++w) {
+        const int c = all[w * num_experts + tid];
+        rows += c & 0xffff;
+        before += c >> 16;
+      }
+    }
 #pragma unroll
     for (int w = 0; w < TABLE_WAVES; ++w) {
       const int c = counts[w * num_experts + tid];
-      counts[w * num_experts + tid] = rows;  // this expert's slots in earlier waves
-      rows += c;
+      counts[w * num_experts + tid] = before;
+      before += c;
     }
+    if (alone) rows = before;
     tiles = (rows + plan_rows - 1) / plan_rows;
   }
   int row_sum = rows, tile_sum = tiles;
@@ -239,20 +269,22 @@ __global__ __launch_bounds__(TABLE_THREADS) void moe_tables_kernel(const int* __
   }
   if (tid < num_experts) {
     const int begin = row_sum - rows;
-    if (tid == 0) expert_offsets[0] = 0;
-    expert_offsets[tid + 1] = row_sum;
-    ps1[3 * tid] = rows;
-    ps1[3 * tid + 1] = 2 * n;
-    ps1[3 * tid + 2] = k;
-    ps2[3 * tid] = rows;
-    ps2[3 * tid + 1] = k;
-    ps2[3 * tid + 2] = n;
 #pragma unroll
     for (int w = 0; w < TABLE_WAVES; ++w) counts[w * num_experts + tid] += begin;
-    // (the layout grouped_plan_kernel writes: expert, first row, end row)
-    for (int i = 0, slot = tile_sum - tiles; i < tiles && slot < plan_max_tiles; ++i, ++slot)
-      reinterpret_cast<v4i*>(plan)[1 + slot] = v4i{tid, begin + i * plan_rows, row_sum, 0};
-    if (tid == num_experts - 1) plan[0] = tile_sum < plan_max_tiles ? tile_sum : plan_max_tiles;
+    if (blockIdx.x == 0) {
+      if (tid == 0) expert_offsets[0] = 0;
+      expert_offsets[tid + 1] = row_sum;
+      ps1[3 * tid] = rows;
+      ps1[3 * tid + 1] = 2 * n;
+      ps1[3 * tid + 2] = k;
+      ps2[3 * tid] = rows;
+      ps2[3 * tid + 1] = k;
+      ps2[3 * tid + 2] = n;
+      // (the layout grouped_plan_kernel writes: expert, first row, end row)
+      for (int i = 0, slot = tile_sum - tiles; i < tiles && slot < plan_max_tiles; ++i, ++slot)
+        reinterpret_cast<v4i*>(plan)[1 + slot] = v4i{tid, begin + i * plan_rows, row_sum, 0};
+      if (tid == num_experts - 1) plan[0] = tile_sum < plan_max_tiles ? tile_sum : plan_max_tiles;
+    }
   }
   __syncthreads();
   const uint64_t below = (1ull << lane) - 1ull;
@@ -275,7 +307,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void moe_tables_kernel(const int* __
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     if (live && (same & below) == 0) mine[e] += __popcll(same);  // (the wave's LDS operations run in this order)
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    if (i < topk_length) output_permutation[i] = pos;
+    if (i < end_slot) output_permutation[i] = pos;
   }
 }
 
@@ -457,8 +489,13 @@ extern "C" int sglq_prepare_moe_layer(const int32_t* topk_ids, int32_t* expert_o
   }
   int id_bits = 0;
   while ((1 << id_bits) < num_experts) ++id_bits;
-  moe_tables_kernel<<<dim3(1), dim3(TABLE_THREADS), (size_t)TABLE_WAVES * num_experts * sizeof(int), static_cast<hipStream_t>(stream)>>>(
-      topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, (int)topk_length, (int)num_experts, id_bits, (int)n, (int)k, static_cast<int*>(plan), (int)plan_rows, (int)plan_max_tiles);
+  int64_t segments = 1;
+  if (topk_length > TABLE_ONE_SEGMENT && num_experts <= TABLE_SEGMENTS_EXPERTS) segments = (topk_length + TABLE_SEGMENT - 1) / TABLE_SEGMENT;
+  const int64_t segment = ((topk_length + segments - 1) / segments + TABLE_THREADS - 1) / TABLE_THREADS * TABLE_THREADS;
+  segments = (topk_length + segment - 1) / segment;
+  const size_t lds = (size_t)(segments > 1 ? 2 : 1) * TABLE_WAVES * num_experts * sizeof(int);
+  moe_tables_kernel<<<dim3((uint32_t)segments), dim3(TABLE_THREADS), lds, static_cast<hipStream_t>(stream)>>>(
+      topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, (int)topk_length, (int)num_experts, id_bits, (int)n, (int)k, static_cast<int*>(plan), (int)plan_rows, (int)plan_max_tiles, (int)segment);
   return check_moe_launch(name);
 }
 

@@ -1,5 +1,5 @@
-"""The expert layer's one-block tables (sglq_prepare_moe_layer) against the oracle's at the edges of what one
-block takes, its tile plan against the definition, and the layer's host path against the same layer called
+"""The expert layer's tables in one launch (sglq_prepare_moe_layer) against the oracle's at the edges of what it
+takes, its tile plan against the definition, and the layer's host path against the same layer called
 operator by operator, bit for bit."""
 import pytest
 import torch
@@ -38,6 +38,12 @@ def test_tables_and_plan(gpu, slots, experts, tile):
     plan = plan.cpu()
     assert int(plan[0]) == len(tiles)
     assert torch.equal(plan[4:4 + 4 * len(tiles)].view(-1, 4), torch.tensor(tiles, dtype=torch.int32).view(-1, 4))
+
+
+@pytest.mark.parametrize("slots,experts,tile", [(2048, 7, 64), (2049, 7, 64), (3073, 256, 16), (3100, 257, 256), (5000, 1, 256), (32767, 256, 256), (32768, 31, 64)])
+def test_several_segments(gpu, slots, experts, tile):
+    """Both sides of the lines for several segments (2048 slots, 256 experts), short last segments, one expert with nearly all slots."""
+    test_tables_and_plan(gpu, slots, experts, tile)
 
 
 def test_limits_of_one_block(gpu):
