@@ -287,6 +287,19 @@ int sglq_fp8_blockwise_scaled_grouped_mm_planned(const void* a, int64_t lda, con
                                                  int out_dtype, int64_t plan_rows, int64_t num_experts, int64_t total_m,
                                                  int64_t N, int64_t K, void* plan, int64_t plan_bytes, void* stream);
 
+/* sglq_fp8_blockwise_scaled_grouped_mm, or with plan_rows > 0 ..._planned, with the activation rows gathered by the GEMM: row m of the
+ * groups (scales and outputs lie there) multiplies row row_map[m] of a [num_a_rows, K].  row_map is [total_m] int32 on the
+ * device, 0 <= row_map[m] < num_a_rows for every row of every group, anything for others (sglq_prepare_moe_layer_rows and
+ * sglq_prepare_moe_input write it).  For sizes for which sglq_grouped_gathers is 1 (SGLQ_EINVAL otherwise). */
+int64_t sglq_grouped_gathers(int64_t num_experts, int64_t total_m, int64_t K);
+int sglq_fp8_blockwise_scaled_grouped_mm_gathered(const void* a, int64_t lda, int64_t num_a_rows, const int32_t* row_map,
+                                                  const void* b, int64_t ldb, int64_t b_expert_stride, const float* sfa,
+                                                  int64_t sfa_stride_m, int64_t sfa_stride_k, const float* sfb,
+                                                  int64_t sfb_expert_stride, int64_t sfb_stride_k, int64_t sfb_stride_n, void* out,
+                                                  int64_t ldo, int out_dtype, const int32_t* problem_sizes,
+                                                  const int32_t* expert_offsets, int64_t plan_rows, int64_t num_experts,
+                                                  int64_t total_m, int64_t N, int64_t K, void* plan, int64_t plan_bytes, void* stream);
+
 /* The data movement around the grouped GEMM in an MoE layer
  * (python/sglang/srt/layers/moe/cutlass_moe.py:140-222).
  *
@@ -326,6 +339,11 @@ int sglq_prepare_moe_layer(const int32_t* topk_ids, int32_t* expert_offsets, int
                            int32_t* problem_sizes2, int32_t* output_permutation, int64_t topk_length,
                            int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows, int64_t plan_max_tiles,
                            void* plan, void* stream);
+/* ... and input_permutation [topk_length] (expert-major position -> token, slot i being token i / topk's). */
+int sglq_prepare_moe_layer_rows(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1,
+                                int32_t* problem_sizes2, int32_t* output_permutation, int32_t* input_permutation, int64_t topk,
+                                int64_t topk_length, int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows,
+                                int64_t plan_max_tiles, void* plan, void* stream);
 int sglq_shuffle_rows(const void* input, const int32_t* dst2src_map, void* output, int64_t num_src_rows,
                       int64_t num_dst_rows, int64_t row_bytes, void* stream);
 int sglq_silu_and_mul(const void* input, int dtype, void* output, int64_t num_tokens, int64_t d, void* stream);
@@ -362,6 +380,10 @@ int sglq_silu_and_mul_group_quant_fp8(const void* input, int in_dtype, void* out
 int sglq_per_token_group_quant_fp8_scatter_cm(const void* input, int in_dtype, void* output_q, float* output_s,
                                               const int32_t* slot_map, int64_t num_tokens, int64_t hidden, int64_t topk,
                                               int64_t num_dst_rows, float eps, void* stream);
+/* ... with the codes written once, output_q [num_tokens, hidden] in token order (for a GEMM that gathers its rows). */
+int sglq_per_token_group_quant_fp8_scatter_scales_cm(const void* input, int in_dtype, void* output_q, float* output_s,
+                                                     const int32_t* slot_map, int64_t num_tokens, int64_t hidden, int64_t topk,
+                                                     int64_t num_dst_rows, float eps, void* stream);
 int sglq_silu_and_mul_group_quant_fp8_cm(const void* input, int in_dtype, void* output_q, float* output_s,
                                          int64_t num_tokens, int64_t d, float eps, void* stream);
 

@@ -61,6 +61,8 @@ struct GemmArgs {
   int splits;
   int64_t b_expert_stride, sb_expert_stride;  // grouped GEMM: bytes / floats between experts' weights / weight scales
   int num_experts;
+  const int* row_map;  // grouped GEMM: row m of A is row row_map[m] of `a`, which has map_rows rows (nullptr: row m)
+  int map_rows;
   int stream_out;  // the output is larger than the last-level cache: store it with the non-temporal hint
   int pow2_scales;  // block-scaled FP8: every scale is a power of two (KIND_FP8_BLOCK_POW2 where it is built)
   // ... and the activation scales come as UE8M0 codes, four K blocks to an int32 word: word (m, kb / 4) sits at

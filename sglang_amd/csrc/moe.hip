@@ -3,6 +3,7 @@
 // between the two GEMMs, and the weighted combine back to token order.  All HBM-bound.
 #include <type_traits>
 
+#include "quant_device.h"
 #include "sglq_common.h"
 
 namespace sglq {
@@ -193,8 +194,8 @@ constexpr int TABLE_ONE_SEGMENT = 2048, TABLE_SEGMENT = TABLE_THREADS, TABLE_SEG
 
 __global__ __launch_bounds__(TABLE_THREADS) void moe_tables_kernel(const int* __restrict__ topk_ids, int* __restrict__ expert_offsets,
                                                                    int* __restrict__ ps1, int* __restrict__ ps2,
-                                                                   int* __restrict__ output_permutation, int topk_length,
-                                                                   int num_experts, int id_bits, int n, int k, int* __restrict__ plan,
+                                                                   int* __restrict__ output_permutation, int* __restrict__ input_permutation,
+                                                                   FastDiv topk, int topk_length, int num_experts, int id_bits, int n, int k, int* __restrict__ plan,
                                                                    int plan_rows, int plan_max_tiles, int segment) {
   // [TABLE_WAVES][num_experts]: first the segment's counts, then the next position of each; of several segments, all slots' behind them
   extern __shared__ int counts[];
@@ -308,6 +309,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void moe_tables_kernel(const int* __
     if (live && (same & below) == 0) mine[e] += __popcll(same);  // (the wave's LDS operations run in this order)
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     if (i < end_slot) output_permutation[i] = pos;
+    if (input_permutation && live) input_permutation[pos] = (int)topk.div((uint32_t)i);
   }
 }
 
@@ -468,13 +470,12 @@ extern "C" int sglq_prepare_moe_input(const int32_t* topk_ids, int32_t* expert_o
   return check_moe_launch(name);
 }
 
-extern "C" int sglq_prepare_moe_layer(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1,
-                                      int32_t* problem_sizes2, int32_t* output_permutation, int64_t topk_length,
-                                      int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows, int64_t plan_max_tiles,
-                                      void* plan, void* stream) {
+static int prepare_layer_entry(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1, int32_t* problem_sizes2,
+                               int32_t* output_permutation, int32_t* input_permutation, int64_t topk, int64_t topk_length,
+                               int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows, int64_t plan_max_tiles, void* plan, void* stream) {
   const char* name = "prepare_moe_layer";
   if (topk_length <= 0 || num_experts <= 0 || n < 0 || k < 0 || n >= (1ll << 30) || k >= (1ll << 31) || plan_rows <= 0 ||
-      plan_max_tiles <= 0 || plan_max_tiles >= (1ll << 27)) {
+      plan_max_tiles <= 0 || plan_max_tiles >= (1ll << 27) || topk <= 0 || topk >= (1 << 20)) {
     set_error("%s: bad sizes", name);
     return SGLQ_EINVAL;
   }
@@ -489,14 +490,36 @@ extern "C" int sglq_prepare_moe_layer(const int32_t* topk_ids, int32_t* expert_o
   }
   int id_bits = 0;
   while ((1 << id_bits) < num_experts) ++id_bits;
+  FastDiv per_token;
+  per_token.init((uint32_t)topk);
   int64_t segments = 1;
   if (topk_length > TABLE_ONE_SEGMENT && num_experts <= TABLE_SEGMENTS_EXPERTS) segments = (topk_length + TABLE_SEGMENT - 1) / TABLE_SEGMENT;
   const int64_t segment = ((topk_length + segments - 1) / segments + TABLE_THREADS - 1) / TABLE_THREADS * TABLE_THREADS;
   segments = (topk_length + segment - 1) / segment;
   const size_t lds = (size_t)(segments > 1 ? 2 : 1) * TABLE_WAVES * num_experts * sizeof(int);
   moe_tables_kernel<<<dim3((uint32_t)segments), dim3(TABLE_THREADS), lds, static_cast<hipStream_t>(stream)>>>(
-      topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, (int)topk_length, (int)num_experts, id_bits, (int)n, (int)k, static_cast<int*>(plan), (int)plan_rows, (int)plan_max_tiles, (int)segment);
+      topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, input_permutation, per_token, (int)topk_length, (int)num_experts, id_bits, (int)n, (int)k, static_cast<int*>(plan), (int)plan_rows, (int)plan_max_tiles, (int)segment);
   return check_moe_launch(name);
+}
+
+extern "C" int sglq_prepare_moe_layer(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1,
+                                      int32_t* problem_sizes2, int32_t* output_permutation, int64_t topk_length,
+                                      int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows, int64_t plan_max_tiles,
+                                      void* plan, void* stream) {
+  return prepare_layer_entry(topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, nullptr, 1, topk_length, num_experts, n, k,
+                             plan_rows, plan_max_tiles, plan, stream);
+}
+
+extern "C" int sglq_prepare_moe_layer_rows(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1,
+                                           int32_t* problem_sizes2, int32_t* output_permutation, int32_t* input_permutation,
+                                           int64_t topk, int64_t topk_length, int64_t num_experts, int64_t n, int64_t k,
+                                           int64_t plan_rows, int64_t plan_max_tiles, void* plan, void* stream) {
+  if (!input_permutation) {
+    set_error("prepare_moe_layer_rows: null pointer");
+    return SGLQ_EINVAL;
+  }
+  return prepare_layer_entry(topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, input_permutation, topk, topk_length,
+                             num_experts, n, k, plan_rows, plan_max_tiles, plan, stream);
 }
 
 extern "C" int sglq_shuffle_rows(const void* input, const int32_t* dst2src_map, void* output, int64_t num_src_rows,

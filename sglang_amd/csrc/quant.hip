@@ -110,8 +110,9 @@ __global__ __launch_bounds__(256) void group_quant_kernel(const char* __restrict
 // [0, num_dst_rows); other entries (slots routed to nobody) are skipped.  Same arithmetic as
 // group_quant_kernel; each token is read once and written topk times instead of being
 // written once, read topk times and written topk times.
+// ONCE: only the scales go to the slots' rows, the codes are written once, in token order (for a GEMM that gathers the rows itself).
 // ---------------------------------------------------------------------------
-template <int DT, bool CM>
+template <int DT, bool CM, bool ONCE = false>
 __global__ __launch_bounds__(256) void group_quant_scatter_kernel(const char* __restrict__ x, char* __restrict__ q,
                                                                   float* __restrict__ s, const int* __restrict__ slot_map,
                                                                   uint32_t num_rows, uint32_t groups_per_row, FastDiv walk, int topk,
@@ -151,6 +152,16 @@ __global__ __launch_bounds__(256) void group_quant_scatter_kernel(const char* __
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = quantize_elem<false>(ch[c].get(i), y_s, r, -qmax, qmax);
     o[c] = Fp8Pack::pack(v);
+  }
+  if constexpr (ONCE) {
+    char* qp = q + (int64_t)row * hidden + (int64_t)col * GROUP + sub * 8;
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) *reinterpret_cast<v2u*>(qp + c * (GROUP / NCH)) = o[c];
+    for (int j = sub; j < topk; j += LPG) {
+      const int64_t dst = slot_map[(int64_t)row * topk + j];
+      if (dst >= 0 && dst < num_dst_rows) s[CM ? col * num_dst_rows + dst : dst * groups_per_row + col] = y_s;
+    }
+    return;
   }
   for (int j = 0; j < topk; ++j) {
     const int64_t dst = slot_map[(int64_t)row * topk + j];
@@ -858,7 +869,7 @@ static int static_quant_entry(const void* input, int in_dtype, void* output_q, c
 namespace sglq {
 
 static int scatter_entry(const void* input, int in_dtype, void* output_q, float* output_s, const int32_t* slot_map, int64_t num_tokens,
-                         int64_t hidden, int64_t topk, int64_t num_dst_rows, float eps, bool column_major, void* stream) {
+                         int64_t hidden, int64_t topk, int64_t num_dst_rows, float eps, bool column_major, bool once, void* stream) {
   const char* name = "per_token_group_quant_fp8_scatter";
   if (num_tokens < 0 || hidden <= 0 || hidden % 128 != 0 || topk <= 0 || topk >= (1 << 20) || num_dst_rows < 0) {
     set_error("%s: hidden (%lld) must be a positive multiple of 128, topk positive", name, (long long)hidden);
@@ -890,7 +901,9 @@ static int scatter_entry(const void* input, int in_dtype, void* output_q, float*
   const char* xi = static_cast<const char*>(input);
   char* qo = static_cast<char*>(output_q);
 #define SGLQ_SCATTER(DT)                                                                                                            \
-  column_major ? group_quant_scatter_kernel<DT, true><<<grid, block, 0, st>>>(xi, qo, output_s, slot_map, (uint32_t)num_tokens, (uint32_t)gpr, \
+  once ? group_quant_scatter_kernel<DT, true, true><<<grid, block, 0, st>>>(xi, qo, output_s, slot_map, (uint32_t)num_tokens, (uint32_t)gpr, walk,    \
+                                                                            (int)topk, num_dst_rows, eps, qmax, 1.0f / qmax)                       \
+  : column_major ? group_quant_scatter_kernel<DT, true><<<grid, block, 0, st>>>(xi, qo, output_s, slot_map, (uint32_t)num_tokens, (uint32_t)gpr, \
                                                                               walk, (int)topk, num_dst_rows, eps, qmax, 1.0f / qmax)   \
                : group_quant_scatter_kernel<DT, false><<<grid, block, 0, st>>>(xi, qo, output_s, slot_map, (uint32_t)num_tokens, (uint32_t)gpr, \
                                                                                walk, (int)topk, num_dst_rows, eps, qmax, 1.0f / qmax)
@@ -959,12 +972,18 @@ static int silu_quant_entry(const void* input, int in_dtype, void* output_q, flo
 extern "C" int sglq_per_token_group_quant_fp8_scatter(const void* input, int in_dtype, void* output_q, float* output_s,
                                                       const int32_t* slot_map, int64_t num_tokens, int64_t hidden,
                                                       int64_t topk, int64_t num_dst_rows, float eps, void* stream) {
-  return sglq::scatter_entry(input, in_dtype, output_q, output_s, slot_map, num_tokens, hidden, topk, num_dst_rows, eps, false, stream);
+  return sglq::scatter_entry(input, in_dtype, output_q, output_s, slot_map, num_tokens, hidden, topk, num_dst_rows, eps, false, false, stream);
 }
 extern "C" int sglq_per_token_group_quant_fp8_scatter_cm(const void* input, int in_dtype, void* output_q, float* output_s,
                                                          const int32_t* slot_map, int64_t num_tokens, int64_t hidden,
                                                          int64_t topk, int64_t num_dst_rows, float eps, void* stream) {
-  return sglq::scatter_entry(input, in_dtype, output_q, output_s, slot_map, num_tokens, hidden, topk, num_dst_rows, eps, true, stream);
+  return sglq::scatter_entry(input, in_dtype, output_q, output_s, slot_map, num_tokens, hidden, topk, num_dst_rows, eps, true, false, stream);
+}
+
+extern "C" int sglq_per_token_group_quant_fp8_scatter_scales_cm(const void* input, int in_dtype, void* output_q, float* output_s,
+                                                                const int32_t* slot_map, int64_t num_tokens, int64_t hidden, int64_t topk,
+                                                                int64_t num_dst_rows, float eps, void* stream) {
+  return sglq::scatter_entry(input, in_dtype, output_q, output_s, slot_map, num_tokens, hidden, topk, num_dst_rows, eps, true, true, stream);
 }
 extern "C" int sglq_silu_and_mul_group_quant_fp8(const void* input, int in_dtype, void* output_q, float* output_s,
                                                  int64_t num_tokens, int64_t d, float eps, void* stream) {
