@@ -44,7 +44,7 @@ def cutlass_fused_experts_fp8(
     scales) to their expert-major rows; grouped GEMM 1; SiLU-and-multiply fused with the second
     quantization; grouped GEMM 2; weighted sum back into token order.  No per-expert transpose pass is needed: the
     C++ host path writes the activation scales column-major over all rows (a K block's scales of 64 rows are then one
-    load), the steps below keep them K-major, the branch the reference takes for SM100 (:160-162,194-196)."""
+    load; with many rows an expert it writes the codes once, in token order, and GEMM 1 gathers them), the steps below keep them K-major, the branch the reference takes for SM100 (:160-162,194-196)."""
     assert use_fp8_blockscale, "Only support fp8 blockscale for now"
     assert topk_weights.shape == topk_ids.shape, "topk shape mismatch"
     assert w1_q.dtype == torch.float8_e4m3fn
