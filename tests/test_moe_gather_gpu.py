@@ -64,6 +64,16 @@ def test_gathered_rows(gpu, m, topk, e, n, k, dtype, empty, planned):
     assert torch.equal(y, z)
 
 
+# Blocks that walk three to five tiles each: the next tiles' row maps, K blocks of theirs read in the steps before, stores left in flight, tiles of
+# other heights behind each other (150 rows an expert) and columns that end inside a tile; three K blocks leave no step between the first and the last but one.
+@pytest.mark.parametrize("m,topk,e,n,dtype,empty", [(4000, 8, 8, 768, torch.bfloat16, False), (4001, 8, 9, 1088, torch.float16, True), (3000, 4, 80, 1152, torch.bfloat16, True)])
+@pytest.mark.parametrize("k", [384, 512, 640, 1024])
+@pytest.mark.parametrize("planned", [True, False])
+def test_gathered_blocks_walk_several_tiles(gpu, m, topk, e, n, k, dtype, empty, planned):
+    assert max(m * topk // 256, e - 1) * (2 * n // 256) > 2 * torch.cuda.get_device_properties(gpu).multi_processor_count
+    test_gathered_rows(gpu, m, topk, e, n, k, dtype, empty, planned)
+
+
 def test_sizes_that_do_not_gather(gpu):
     from sglang_amd import _lib
 
