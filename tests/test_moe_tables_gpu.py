@@ -94,3 +94,15 @@ def test_layer_host_path(gpu, monkeypatch, m, topk, e, n, k, dtype, weights):
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
     for a, b in zip(got_t, want_t):
         assert torch.equal(a, b)
+
+
+# (in one launch: blocks of the gathered GEMM walk several tiles of three K blocks; beyond it: GEMM 2 takes the plan that GEMM 1 left, or forms its own)
+@pytest.mark.parametrize("m,topk,e,n,k,one_launch,gathers,shared", [(4000, 8, 8, 768, 384, True, 1, True), (5000, 8, 6, 512, 640, False, 1, True),
+                                                                    (12000, 3, 5, 256, 512, False, 1, False), (11000, 3, 5, 512, 256, False, 0, False)])
+def test_layer_host_path_of_long_prompts(gpu, monkeypatch, m, topk, e, n, k, one_launch, gathers, shared):
+    from sglang_amd import _lib
+
+    lib, rows = _lib.load(), m * topk
+    assert (rows <= 32768) == one_launch and topk > 2 and lib.sglq_grouped_gathers(e, rows, k) == gathers
+    assert (lib.sglq_grouped_plan_rows(e, rows, k) == lib.sglq_grouped_plan_rows(e, rows, n)) == shared
+    test_layer_host_path(gpu, monkeypatch, m, topk, e, n, k, torch.bfloat16, torch.float32)
