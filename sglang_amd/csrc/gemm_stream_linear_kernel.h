@@ -5,7 +5,9 @@
 
 namespace sglq {
 
-// (arrives in `dst` unseen by the compiler's wait counts, see wait_x)
+// (arrives in `dst` unseen by the compiler's wait counts, see wait_x.  To the compiler `dst` is written here: a copy or a spill of it in front of
+// wait_x would take what was there before.  None of the instantiations has one, and nothing but a look at the code built shows it:
+// tests/test_waits_in_code.py follows every way through each, for another compiler, another register budget, another order of these loads.)
 SGLQ_DEV void load16(v4u& dst, v4u rsrc, uint32_t voff) {
   asm volatile("buffer_load_dwordx4 %0, %1, %2, 0 offen" : "=v"(dst) : "v"(voff), "s"(rsrc) : "memory");
 }

@@ -97,6 +97,37 @@ def walk(code, start, step, meet):
                 todo.append(s)
 
 
+def registers(operands):
+    out = set()
+    for a, b in re.findall(r"\bv(?:\[(\d+):(\d+)\])", operands):
+        out |= set(range(int(a), int(b) + 1))
+    return out | {int(r) for r in re.findall(r"\bv(\d+)\b", operands)}
+
+
+def test_linears_touch_no_activation_before_it_has_arrived(tmp_path):
+    """gemm_stream_quant_kernel and gemm_stream_tokenquant_kernel load their activations into registers behind the compiler's back."""
+    found = kernels(tmp_path, r"gemm_stream_(token)?quant_kernel")
+    assert len(found) == 96
+    for name, code in found.items():
+        loads = [0]
+
+        def step(state, op, operands):  # state: register -> the fewest vector-memory operations younger than its load
+            count = vmcnt(op, operands)
+            if count is not None:
+                return {r: c for r, c in state.items() if c < count}
+            touched = registers(operands)
+            load = op == "buffer_load_dwordx4" and not operands.endswith("lds")
+            fresh = registers(operands.split(",")[0]) if load else set()
+            assert not touched & set(state) - fresh, f"{name}: {op} {operands}"
+            if VMEM.match(op):
+                state = {r: min(c + 1, 64) for r, c in state.items()}
+            loads[0] += load
+            return {**state, **{r: 0 for r in fresh}}
+
+        walk(code, {}, step, lambda old, new: new if old is None else {r: min(old.get(r, 64), new.get(r, 64)) for r in old.keys() | new.keys()})
+        assert loads[0] >= 16
+
+
 def test_gathered_rows_are_named_before_they_are_read(tmp_path):
     """PIPE_GATHERED's row maps, copied into LDS by waves 0 to 3 and read by all: the copy is waited for, then a barrier.  Two places in turn: a read with
     no barrier since the copy is one of the place that is not being written.  A tile has sixteen stores and then steps with
