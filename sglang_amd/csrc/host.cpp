@@ -669,7 +669,7 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int code = dtype_code(x.scalar_type());
     const int64_t plan_rows = lib.sglq_grouped_plan_rows(e, rows, k), plan_rows2 = lib.sglq_grouped_plan_rows(e, rows, n);
     const bool one_block = rows <= 32768 && e <= 512;
-    const bool shared_plan = plan_rows == plan_rows2;  // (written by the tables, or by the first GEMM: 5 us less on 48000 slots)
+    const bool shared_plan = plan_rows == plan_rows2;  // (written by the tables, or by the first GEMM: a launch of 5 us less on 48000 slots, 2210 us a layer)
     // GEMM 1 gathers its rows from the tokens' codes, written once.  Quantization + GEMM 1, without and with (us), tokens x experts x
     // top-k, hidden x intermediate: 2500 x 32 x 8, 7168 x 2048 664 -> 626; 600 x 32 x 8 239 -> 223; 2500 x 16 x 3 266 -> 255;
     // 3000 x 16 x 4, 4096 x 1408 194.5 -> 187.8; on 6000 x 16, 2048 x 768 top-8 186 -> 173, top-3 78.5 and 78.4, top-2 68.0 -> 71.4:
