@@ -195,7 +195,8 @@ int sglq_fp8_blockwise_scaled_mm_bias(const void* a, int64_t lda, const void* b,
  *   eps  lower bound of a group's abs-max (the callers' 1e-10)
  * Where it was measured faster (16-bit activations, shapes that the decode kernel without split-K
  * takes: one row; up to 4 rows with N >= 1024 and K <= 4096 or a block for every compute unit; up to 8 rows
- * with K <= 4096, N >= 1024 and K >= 3072, M * K <= 8192 or N <= 4096), one
+ * with K <= 4096, N >= 1024 and K >= 3072, M * K <= 8192 or N <= 4096, but not, where the workspace holds the
+ * codes, with more than 4.5 blocks a compute unit on K >= 3072), one
  * kernel loads the activations into registers and quantizes them beside the stream of weights, codes and
  * scales pass through LDS of the wave that multiplies them: no
  * quantization launch, no round trip through memory, no workspace.  Other
@@ -218,7 +219,8 @@ int sglq_w8a8_block_fp8_linear(const void* x, int in_dtype, const void* b, int64
  *   x    [M, K] contiguous activations, in_dtype in {BF16, FP16, FP32}, 16-byte aligned
  *   b, scales_b, bias (may be NULL), out: as sglq_int8_scaled_mm / sglq_fp8_scaled_mm
  * For M <= 2, M <= 4 with K >= 2304 or with M * K <= 8192 and N <= 4096, and M <= 8 with 2304 <= K <= 4096 (FP8: 8192)
- * (16-bit activations, K % 128 == 0), on the shapes that the decode kernel without split-K takes, one kernel loads the activations into registers, forms the
+ * (16-bit activations, K % 128 == 0), on the shapes that the decode kernel without split-K takes, but not, where the workspace holds the codes, for M > 4 with
+ * many blocks a compute unit or, INT8, K > 3584 and N < 4096, one kernel loads the activations into registers, forms the
  * rows' scales (rows longer than the registers hold are read twice) and quantizes beside the stream of weights, the codes pass through LDS of the wave
  * that multiplies them: no quantization launch, no round trip through memory, no workspace.  Other shapes run the quantization kernel and the GEMM
  * one after the other; their codes and row scales need M * K + 4 * M bytes (each rounded up to
