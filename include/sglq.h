@@ -303,6 +303,17 @@ int sglq_fp8_blockwise_scaled_grouped_mm_gathered(const void* a, int64_t lda, in
                                                   const int32_t* expert_offsets, int64_t plan_rows, int64_t num_experts,
                                                   int64_t total_m, int64_t N, int64_t K, void* plan, int64_t plan_bytes, void* stream);
 
+/* ..._planned, or with a row map ..._gathered, on 256-row tiles in the order of a walk that sglq_prepare_moe_layer_walks has written: the experts' weights are
+ * read from memory once.  sglq_grouped_walk_bytes: what the walks of a layer's two GEMMs take (n: intermediate, k: hidden size) and where the second one
+ * begins; 0 where a layer has none. */
+int64_t sglq_grouped_walk_bytes(int64_t num_experts, int64_t total_m, int64_t n, int64_t k, int64_t* second);
+int sglq_fp8_blockwise_scaled_grouped_mm_walked(const void* a, int64_t lda, int64_t num_a_rows, const int32_t* row_map, const void* b,
+                                                int64_t ldb, int64_t b_expert_stride, const float* sfa, int64_t sfa_stride_m,
+                                                int64_t sfa_stride_k, const float* sfb, int64_t sfb_expert_stride,
+                                                int64_t sfb_stride_k, int64_t sfb_stride_n, void* out, int64_t ldo, int out_dtype,
+                                                int64_t num_experts, int64_t total_m, int64_t N, int64_t K, void* plan,
+                                                int64_t plan_bytes, const void* walk, void* stream);
+
 /* The data movement around the grouped GEMM in an MoE layer
  * (python/sglang/srt/layers/moe/cutlass_moe.py:140-222).
  *
@@ -347,6 +358,11 @@ int sglq_prepare_moe_layer_rows(const int32_t* topk_ids, int32_t* expert_offsets
                                 int32_t* problem_sizes2, int32_t* output_permutation, int32_t* input_permutation, int64_t topk,
                                 int64_t topk_length, int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows,
                                 int64_t plan_max_tiles, void* plan, void* stream);
+/* ... with a plan for 256-row tiles, and the walks of both GEMMs (2 n x k and k x n): walks_bytes, 16-byte aligned. */
+int sglq_prepare_moe_layer_walks(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1,
+                                 int32_t* problem_sizes2, int32_t* output_permutation, int32_t* input_permutation, int64_t topk,
+                                 int64_t topk_length, int64_t num_experts, int64_t n, int64_t k, void* plan, void* walks,
+                                 int64_t walks_bytes, void* stream);
 int sglq_shuffle_rows(const void* input, const int32_t* dst2src_map, void* output, int64_t num_src_rows,
                       int64_t num_dst_rows, int64_t row_bytes, void* stream);
 int sglq_silu_and_mul(const void* input, int dtype, void* output, int64_t num_tokens, int64_t d, void* stream);

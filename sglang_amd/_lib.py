@@ -90,6 +90,11 @@ SIGNATURES = {
     "sglq_per_token_group_quant_fp8_scatter_scales_cm": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_float, c_void_p],
     "sglq_prepare_moe_layer_rows": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64,
                                     c_int64, c_int64, c_void_p, c_void_p],
+    "sglq_fp8_blockwise_scaled_grouped_mm_walked": [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p,
+                                                    c_int64, c_int64, c_int64, c_void_p, c_int64, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p,
+                                                    c_int64, c_void_p, c_void_p],
+    "sglq_prepare_moe_layer_walks": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p,
+                                     c_void_p, c_int64, c_void_p],
     "sglq_fp8_blockwise_scaled_grouped_mm_gathered": [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int64,
                                                       c_int64, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_int, c_void_p,
                                                       c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p],
@@ -128,6 +133,8 @@ def load() -> ctypes.CDLL:
     lib.sglq_grouped_plan_rows.restype = c_int64
     lib.sglq_grouped_gathers.argtypes = [c_int64, c_int64, c_int64]
     lib.sglq_grouped_gathers.restype = c_int64
+    lib.sglq_grouped_walk_bytes.argtypes = [c_int64, c_int64, c_int64, c_int64, c_void_p]
+    lib.sglq_grouped_walk_bytes.restype = c_int64
     lib.sglq_abi_version.restype = c_int
     lib.sglq_abi_version.argtypes = []
     lib.sglq_debug_set_direct_lds.argtypes = [c_int]

@@ -61,6 +61,7 @@ struct GemmArgs {
   int splits;
   int64_t b_expert_stride, sb_expert_stride;  // grouped GEMM: bytes / floats between experts' weights / weight scales
   int num_experts;
+  const int* walk;     // grouped GEMM on 256-row tiles: its walk (nullptr: in the order of the plan)
   const int* row_map;  // grouped GEMM: row m of A is row row_map[m] of `a`, which has map_rows rows (nullptr: row m)
   int map_rows;
   int stream_out;  // the output is larger than the last-level cache: store it with the non-temporal hint
@@ -104,6 +105,10 @@ SGLQ_DEV int first_k_step_shared(const GemmArgs& p, uint32_t tile, int steps) { 
 // Grouped GEMM tile plan in the workspace (int32): [0] = number of row tiles, then from [4] on
 // one entry of four per row tile: expert, first row, end row (both absolute rows of A and C).
 constexpr int PLAN_HEADER = 4, PLAN_ENTRY = 4;
+
+// Walk of a grouped GEMM on 256-row tiles (int32, sglq_prepare_moe_layer_walks): [0] = number of tiles, then from [WALK_HEADER] on one entry of four per
+// tile, in the order in which they are taken: first row, end row (at most 256 rows on; where it is fewer, the tile computes only these), expert, column tile.
+constexpr int WALK_HEADER = 16;
 
 // s_waitcnt immediate: wait until at most `vm` vector-memory loads are outstanding
 // and all LDS / scalar-memory operations are done (vmcnt is split over bits 3:0 and 15:14).

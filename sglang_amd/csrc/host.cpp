@@ -64,7 +64,10 @@ namespace {
   X(sglq_prepare_moe_input)                                                                                         \
   X(sglq_prepare_moe_layer)                                                                                         \
   X(sglq_prepare_moe_layer_rows)                                                                                    \
+  X(sglq_prepare_moe_layer_walks)                                                                                   \
   X(sglq_grouped_gathers)                                                                                           \
+  X(sglq_grouped_walk_bytes)                                                                                        \
+  X(sglq_fp8_blockwise_scaled_grouped_mm_walked)                                                                    \
   X(sglq_fp8_blockwise_scaled_grouped_mm_gathered)                                                                  \
   X(sglq_grouped_plan_rows)                                                                                         \
   X(sglq_fp8_blockwise_scaled_grouped_mm)                                                                           \
@@ -676,6 +679,10 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     // two copies of the codes cost less than the gathering.
     const bool gathers = topk > 2 && lib.sglq_grouped_gathers(e, rows, k) != 0;
     const int64_t plan_bytes = round256(16 * (rows / 16 + e + 1));
+    // On 256-row tiles the tables come with both GEMMs' walks.
+    int64_t walk2_at = 0;
+    const int64_t walk_bytes = one_block ? lib.sglq_grouped_walk_bytes(e, rows, n, k, &walk2_at) : 0;
+    const bool walked = walk_bytes > 0, maps_rows = walked || gathers || !one_block;
     // expert-major rows: quantized activations (dead once GEMM 1 has run) under GEMM 2's output, GEMM 1's
     // output, the quantized intermediate
     const int64_t codes1 = round256(rows * k), scales1 = round256(rows * (k / 128) * 4), c2 = round256(rows * k * 2);
@@ -687,7 +694,7 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       ReleaseGil unlocked;
       Launch here(x.device());
       out = empty({m, k}, x.scalar_type(), here.device);
-      Tensor arena = empty({head + c1 + codes2 + scales2 + plan_bytes + map + (one_block && !gathers ? 0 : map)}, at::kByte, here.device);
+      Tensor arena = empty({head + c1 + codes2 + scales2 + plan_bytes + map + (maps_rows ? map : 0) + walk_bytes}, at::kByte, here.device);
       char* base = static_cast<char*>(arena.data_ptr());
       char *q1 = base, *y1 = base + head, *q2 = y1 + c1, *plan = q2 + codes2 + scales2;
       float *f1 = reinterpret_cast<float*>(q1 + codes1), *f2 = reinterpret_cast<float*>(q2 + codes2);
@@ -695,7 +702,11 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       const int32_t* ids_p = static_cast<const int32_t*>(ids.data_ptr());
       int32_t *off_p = static_cast<int32_t*>(offsets.data_ptr()), *ps1 = static_cast<int32_t*>(sizes1.data_ptr()),
               *ps2 = static_cast<int32_t*>(sizes2.data_ptr());
-      if (one_block && gathers) {
+      char* const walk1 = reinterpret_cast<char*>(row_map) + map;
+      char* const walk2 = walk1 + walk2_at;
+      if (walked) {
+        rc = lib.sglq_prepare_moe_layer_walks(ids_p, off_p, ps1, ps2, slot_map, row_map, topk, rows, e, n, k, plan, walk1, walk_bytes, here.stream);
+      } else if (one_block && gathers) {
         rc = lib.sglq_prepare_moe_layer_rows(ids_p, off_p, ps1, ps2, slot_map, row_map, topk, rows, e, n, k, plan_rows, rows / plan_rows + e, plan,
                                              here.stream);
       } else if (one_block) {
@@ -706,9 +717,13 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         rc = lib.sglq_prepare_moe_input(ids_p, off_p, nullptr, ps1, ps2, row_map, slot_map, rows, topk, e, n, k, here.stream);
       }
       auto grouped = [&](const void* q, const float* f, const Tensor& w, const Tensor& s, void* y, const int32_t* sizes, int64_t depth,
-                         int64_t width, int64_t tile_rows, bool planned) {
+                         int64_t width, int64_t tile_rows, bool planned, const char* walk, const int32_t* map_p) {
         const float* s_p = static_cast<const float*>(s.data_ptr());
         const int64_t ldb = w.stride(2), bs = e > 1 ? w.stride(0) : width * depth;
+        if (walked)
+          return lib.sglq_fp8_blockwise_scaled_grouped_mm_walked(q, depth, m, map_p, w.data_ptr(), ldb, bs, f, 1, rows, s_p, s.stride(0), s.stride(1),
+                                                                 s.stride(2), y, width, code, e, rows, width, depth, plan, plan_bytes, walk,
+                                                                 here.stream);
         return planned ? lib.sglq_fp8_blockwise_scaled_grouped_mm_planned(q, depth, w.data_ptr(), ldb, bs, f, 1, rows, s_p, s.stride(0),
                                                                           s.stride(1), s.stride(2), y, width, code, tile_rows, e, rows, width,
                                                                           depth, plan, plan_bytes, here.stream)
@@ -719,17 +734,18 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       if (gathers) {
         if (rc == 0)
           rc = lib.sglq_per_token_group_quant_fp8_scatter_scales_cm(x.data_ptr(), code, q1, f1, slot_map, m, k, topk, rows, 1e-10f, here.stream);
-        if (rc == 0)
+        if (rc == 0 && walked) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, true, walk1, row_map);
+        else if (rc == 0)
           rc = lib.sglq_fp8_blockwise_scaled_grouped_mm_gathered(q1, k, m, row_map, w1.data_ptr(), w1.stride(2), e > 1 ? w1.stride(0) : 2 * n * k, f1,
                                                                  1, rows, static_cast<const float*>(s1.data_ptr()), s1.stride(0), s1.stride(1),
                                                                  s1.stride(2), y1, 2 * n, code, ps1, off_p, one_block ? plan_rows : 0, e, rows,
                                                                  2 * n, k, plan, plan_bytes, here.stream);
       } else {
         if (rc == 0) rc = lib.sglq_per_token_group_quant_fp8_scatter_cm(x.data_ptr(), code, q1, f1, slot_map, m, k, topk, rows, 1e-10f, here.stream);
-        if (rc == 0) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, one_block);
+        if (rc == 0) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, one_block, walk1, nullptr);
       }
       if (rc == 0) rc = lib.sglq_silu_and_mul_group_quant_fp8_cm(y1, code, q2, f2, rows, n, 1e-10f, here.stream);
-      if (rc == 0) rc = grouped(q2, f2, w2, s2, base, ps2, n, k, plan_rows2, shared_plan);
+      if (rc == 0) rc = grouped(q2, f2, w2, s2, base, ps2, n, k, plan_rows2, shared_plan, walk2, nullptr);
       if (rc == 0 && float_weights)
         rc = lib.sglq_apply_shuffle_mul_sum_f32(base, out.data_ptr(), slot_map, static_cast<const float*>(weights.data_ptr()), code, m, topk, k,
                                                 rows, here.stream);

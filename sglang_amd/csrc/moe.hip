@@ -3,6 +3,7 @@
 // between the two GEMMs, and the weighted combine back to token order.  All HBM-bound.
 #include <type_traits>
 
+#include "gemm_device.h"
 #include "quant_device.h"
 #include "sglq_common.h"
 
@@ -192,14 +193,25 @@ constexpr int TABLE_MAX_SLOTS = TABLE_THREADS * TABLE_STEPS, TABLE_MAX_EXPERTS =
 // (several segments double the LDS: 32 KiB at 256 experts, from there on one)
 constexpr int TABLE_ONE_SEGMENT = 2048, TABLE_SEGMENT = TABLE_THREADS, TABLE_SEGMENTS_EXPERTS = 256;
 
+// The walks of the layer's two GEMMs on 256-row tiles (gemm_device.h), written by blocks of their own, which count the slots as the others do and place
+// none: a band is an expert's row tiles, up to WALK_BAND of them (of more than that bands of like size), column by column, so that the blocks of an XCD share the
+// weights that they read at the same time and every weight is read by one band only.
+struct LayerWalks {
+  int* walk[2];
+  FastDiv columns[2];  // column tiles
+  int first_block;     // blocks from here on write them (none: the grid ends there)
+};
+constexpr int WALK_BAND = 8, WALK_ROWS = 256;
+
 __global__ __launch_bounds__(TABLE_THREADS) void moe_tables_kernel(const int* __restrict__ topk_ids, int* __restrict__ expert_offsets,
                                                                    int* __restrict__ ps1, int* __restrict__ ps2,
                                                                    int* __restrict__ output_permutation, int* __restrict__ input_permutation,
                                                                    FastDiv topk, int topk_length, int num_experts, int id_bits, int n, int k, int* __restrict__ plan,
-                                                                   int plan_rows, int plan_max_tiles, int segment) {
+                                                                   int plan_rows, int plan_max_tiles, int segment, const LayerWalks walks) {
   // [TABLE_WAVES][num_experts]: first the segment's counts, then the next position of each; of several segments, all slots' behind them
   extern __shared__ int counts[];
   __shared__ int wave_rows[TABLE_WAVES], wave_tiles[TABLE_WAVES];
+  __shared__ int expert_rows[TABLE_MAX_EXPERTS], expert_end[TABLE_MAX_EXPERTS], expert_tiles[TABLE_MAX_EXPERTS];  // (walks only)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int begin_slot = (int)blockIdx.x * segment, end_slot = begin_slot + segment < topk_length ? begin_slot + segment : topk_length;
@@ -286,8 +298,43 @@ __global__ __launch_bounds__(TABLE_THREADS) void moe_tables_kernel(const int* __
         reinterpret_cast<v4i*>(plan)[1 + slot] = v4i{tid, begin + i * plan_rows, row_sum, 0};
       if (tid == num_experts - 1) plan[0] = tile_sum < plan_max_tiles ? tile_sum : plan_max_tiles;
     }
+    if ((int)blockIdx.x >= walks.first_block) {
+      expert_rows[tid] = rows;
+      expert_end[tid] = row_sum;
+      expert_tiles[tid] = tile_sum;
+    }
   }
   __syncthreads();
+  if ((int)blockIdx.x >= walks.first_block) {
+    const uint32_t all_tiles = (uint32_t)expert_tiles[num_experts - 1], units1 = all_tiles * walks.columns[0].d;
+    const uint32_t units = units1 + all_tiles * walks.columns[1].d;
+    if ((int)blockIdx.x == walks.first_block && tid < 2) walks.walk[tid][0] = (int)(tid == 0 ? units1 : units - units1);
+    for (uint32_t i = (blockIdx.x - walks.first_block) * TABLE_THREADS + tid; i < units; i += (gridDim.x - walks.first_block) * TABLE_THREADS) {
+      const bool one = i < units1;
+      const int columns = (int)(one ? walks.columns[0].d : walks.columns[1].d);
+      const uint32_t u = one ? i : i - units1;
+      const int any = (int)(one ? walks.columns[0].div(u) : walks.columns[1].div(u));  // a row tile of the unit's expert: their units follow each other
+      int e = 0;  // ... the first expert whose tiles end behind it
+      for (int step = 1 << (id_bits > 0 ? id_bits - 1 : 0); step > 0; step >>= 1)
+        if (e + step <= num_experts && expert_tiles[e + step - 1] <= any) e += step;
+      const int rows_e = expert_rows[e], end = expert_end[e];
+      const int count = (rows_e + WALK_ROWS - 1) / WALK_ROWS, first = expert_tiles[e] - count;
+      const int bands = (count + WALK_BAND - 1) / WALK_BAND, height = bands == 1 ? count : (count + bands - 1) / bands;
+      const int unit = (int)u - first * columns, band = bands == 1 ? 0 : (any - first) / height;
+      const int left = count - band * height, rows_b = left < height ? left : height;
+      const int in_band = unit - band * height * columns, column = in_band / rows_b;
+      const int t = band * height + in_band - column * rows_b;
+      // an expert's last two tiles share the rows that are left: the first half of them, rounded up to 32, and the rest
+      int row = end - rows_e + t * WALK_ROWS, to = end;
+      const int rest = to - row;
+      const bool second = rest <= WALK_ROWS && t > 0;
+      const int both = second ? rest + WALK_ROWS : rest, share = ((both + 1) / 2 + 31) & ~31;
+      if (second) row += share - WALK_ROWS;
+      else if (rest > WALK_ROWS) to = row + (rest < 2 * WALK_ROWS ? share : WALK_ROWS);
+      reinterpret_cast<v4i*>((one ? walks.walk[0] : walks.walk[1]) + WALK_HEADER)[u] = v4i{row, to, e, column};
+    }
+    return;
+  }
   const uint64_t below = (1ull << lane) - 1ull;
 #pragma unroll
   for (int s = 0; s < TABLE_STEPS; ++s) {
@@ -472,7 +519,8 @@ extern "C" int sglq_prepare_moe_input(const int32_t* topk_ids, int32_t* expert_o
 
 static int prepare_layer_entry(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1, int32_t* problem_sizes2,
                                int32_t* output_permutation, int32_t* input_permutation, int64_t topk, int64_t topk_length,
-                               int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows, int64_t plan_max_tiles, void* plan, void* stream) {
+                               int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows, int64_t plan_max_tiles, void* plan, void* stream,
+                               void* walk1 = nullptr, void* walk2 = nullptr) {
   const char* name = "prepare_moe_layer";
   if (topk_length <= 0 || num_experts <= 0 || n < 0 || k < 0 || n >= (1ll << 30) || k >= (1ll << 31) || plan_rows <= 0 ||
       plan_max_tiles <= 0 || plan_max_tiles >= (1ll << 27) || topk <= 0 || topk >= (1 << 20)) {
@@ -496,9 +544,20 @@ static int prepare_layer_entry(const int32_t* topk_ids, int32_t* expert_offsets,
   if (topk_length > TABLE_ONE_SEGMENT && num_experts <= TABLE_SEGMENTS_EXPERTS) segments = (topk_length + TABLE_SEGMENT - 1) / TABLE_SEGMENT;
   const int64_t segment = ((topk_length + segments - 1) / segments + TABLE_THREADS - 1) / TABLE_THREADS * TABLE_THREADS;
   segments = (topk_length + segment - 1) / segment;
-  const size_t lds = (size_t)(segments > 1 ? 2 : 1) * TABLE_WAVES * num_experts * sizeof(int);
-  moe_tables_kernel<<<dim3((uint32_t)segments), dim3(TABLE_THREADS), lds, static_cast<hipStream_t>(stream)>>>(
-      topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, input_permutation, per_token, (int)topk_length, (int)num_experts, id_bits, (int)n, (int)k, static_cast<int*>(plan), (int)plan_rows, (int)plan_max_tiles, (int)segment);
+  LayerWalks walks{};
+  walks.first_block = (int)segments;
+  int64_t walk_blocks = 0;
+  if (walk1) {
+    walks.walk[0] = static_cast<int*>(walk1);
+    walks.walk[1] = static_cast<int*>(walk2);
+    walks.columns[0].init((uint32_t)((2 * n + 255) / 256));
+    walks.columns[1].init((uint32_t)((k + 255) / 256));
+    walk_blocks = (plan_max_tiles * (walks.columns[0].d + walks.columns[1].d) + TABLE_THREADS - 1) / TABLE_THREADS;
+    if (walk_blocks > 32) walk_blocks = 32;
+  }
+  const size_t lds = (size_t)(segments + walk_blocks > 1 ? 2 : 1) * TABLE_WAVES * num_experts * sizeof(int);
+  moe_tables_kernel<<<dim3((uint32_t)(segments + walk_blocks)), dim3(TABLE_THREADS), lds, static_cast<hipStream_t>(stream)>>>(
+      topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, input_permutation, per_token, (int)topk_length, (int)num_experts, id_bits, (int)n, (int)k, static_cast<int*>(plan), (int)plan_rows, (int)plan_max_tiles, (int)segment, walks);
   return check_moe_launch(name);
 }
 
@@ -520,6 +579,19 @@ extern "C" int sglq_prepare_moe_layer_rows(const int32_t* topk_ids, int32_t* exp
   }
   return prepare_layer_entry(topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, input_permutation, topk, topk_length,
                              num_experts, n, k, plan_rows, plan_max_tiles, plan, stream);
+}
+
+extern "C" int sglq_prepare_moe_layer_walks(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1, int32_t* problem_sizes2,
+                                            int32_t* output_permutation, int32_t* input_permutation, int64_t topk, int64_t topk_length,
+                                            int64_t num_experts, int64_t n, int64_t k, void* plan, void* walks, int64_t walks_bytes, void* stream) {
+  int64_t second = 0;
+  const int64_t need = sglq_grouped_walk_bytes(num_experts, topk_length, n, k, &second);
+  if (!input_permutation || !walks || (reinterpret_cast<uintptr_t>(walks) & 15) || need == 0 || walks_bytes < need) {
+    set_error("prepare_moe_layer_walks: a row map and 16-byte aligned walks of %lld bytes are needed, for sizes that sglq_grouped_walk_bytes names", (long long)need);
+    return SGLQ_EINVAL;
+  }
+  return prepare_layer_entry(topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, input_permutation, topk, topk_length,
+                             num_experts, n, k, WALK_ROWS, topk_length / WALK_ROWS + num_experts, plan, stream, walks, static_cast<char*>(walks) + second);
 }
 
 extern "C" int sglq_shuffle_rows(const void* input, const int32_t* dst2src_map, void* output, int64_t num_src_rows,
