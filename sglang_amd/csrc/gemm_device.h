@@ -61,6 +61,7 @@ struct GemmArgs {
   int splits;
   int64_t b_expert_stride, sb_expert_stride;  // grouped GEMM: bytes / floats between experts' weights / weight scales
   int num_experts;
+  float* out_scales;   // grouped GEMM with the activation behind it (PIPE_SILU): scales of its FP8 outputs, [N / 256][M]
   const int* walk;     // grouped GEMM on 256-row tiles: its walk (nullptr: in the order of the plan)
   const int* row_map;  // grouped GEMM: row m of A is row row_map[m] of `a`, which has map_rows rows (nullptr: row m)
   int map_rows;

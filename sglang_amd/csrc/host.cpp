@@ -68,6 +68,7 @@ namespace {
   X(sglq_grouped_gathers)                                                                                           \
   X(sglq_grouped_walk_bytes)                                                                                        \
   X(sglq_fp8_blockwise_scaled_grouped_mm_walked)                                                                    \
+  X(sglq_fp8_blockwise_scaled_grouped_mm_silu)                                                                      \
   X(sglq_fp8_blockwise_scaled_grouped_mm_gathered)                                                                  \
   X(sglq_grouped_plan_rows)                                                                                         \
   X(sglq_fp8_blockwise_scaled_grouped_mm)                                                                           \
@@ -679,14 +680,18 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     // two copies of the codes cost less than the gathering.
     const bool gathers = topk > 2 && lib.sglq_grouped_gathers(e, rows, k) != 0;
     const int64_t plan_bytes = round256(16 * (rows / 16 + e + 1));
-    // On 256-row tiles the tables come with both GEMMs' walks.
+    // On 256-row tiles the tables come with both GEMMs' walks, and GEMM 1 with the activation and its quantization behind it, from 2^21 activations on
+    // (us, GEMM 1 and the activation's launch -> one launch): 2500 tokens x 32 experts x 8, 7168 x 2048 599.1 -> 584.7, 777 tokens 270.2 -> 260.9; 2048 x 64 x 8,
+    // 4096 x 1024 210.5 -> 198.8; 1870 x 8 x 8, 1152 x 512 32.6 -> 24.4; at 2.4 million 452 x 6 x 6, 5248 x 896 56.8 -> 57.1, 3767 x 8 x 1, 1920 x 640 28.8 -> 27.7.
+    // The activation takes the last tile of a block 5 us more than the stores that it saves, a launch of its own 2.5 us and its bytes: at 1.7 million 523 x 20 x 5,
+    // 7168 x 640 72.0 -> 74.3, at 1.4 million 442 x 16 x 5, 3456 x 640 39.7 -> 41.0.
     int64_t walk2_at = 0;
     const int64_t walk_bytes = one_block ? lib.sglq_grouped_walk_bytes(e, rows, n, k, &walk2_at) : 0;
-    const bool walked = walk_bytes > 0, maps_rows = walked || gathers || !one_block;
+    const bool walked = walk_bytes > 0, activates = walked && rows * n >= (2 << 20), maps_rows = walked || gathers || !one_block;
     // expert-major rows: quantized activations (dead once GEMM 1 has run) under GEMM 2's output, GEMM 1's
     // output, the quantized intermediate
     const int64_t codes1 = round256(rows * k), scales1 = round256(rows * (k / 128) * 4), c2 = round256(rows * k * 2);
-    const int64_t c1 = round256(rows * 2 * n * 2), codes2 = round256(rows * n), scales2 = round256(rows * (n / 128) * 4);
+    const int64_t c1 = activates ? 0 : round256(rows * 2 * n * 2), codes2 = round256(rows * n), scales2 = round256(rows * (n / 128) * 4);
     const int64_t head = codes1 + scales1 > c2 ? codes1 + scales1 : c2, map = round256(rows * 4);
     Tensor out;
     int rc;
@@ -721,9 +726,9 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         const float* s_p = static_cast<const float*>(s.data_ptr());
         const int64_t ldb = w.stride(2), bs = e > 1 ? w.stride(0) : width * depth;
         if (walked)
-          return lib.sglq_fp8_blockwise_scaled_grouped_mm_walked(q, depth, m, map_p, w.data_ptr(), ldb, bs, f, 1, rows, s_p, s.stride(0), s.stride(1),
-                                                                 s.stride(2), y, width, code, e, rows, width, depth, plan, plan_bytes, walk,
-                                                                 here.stream);
+          return lib.sglq_fp8_blockwise_scaled_grouped_mm_walked(q, depth, map_p ? m : rows, map_p, w.data_ptr(), ldb, bs, f, 1, rows, s_p, s.stride(0),
+                                                                 s.stride(1), s.stride(2), y, width, code, e, rows, width, depth, plan, plan_bytes,
+                                                                 walk, here.stream);
         return planned ? lib.sglq_fp8_blockwise_scaled_grouped_mm_planned(q, depth, w.data_ptr(), ldb, bs, f, 1, rows, s_p, s.stride(0),
                                                                           s.stride(1), s.stride(2), y, width, code, tile_rows, e, rows, width,
                                                                           depth, plan, plan_bytes, here.stream)
@@ -734,17 +739,22 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       if (gathers) {
         if (rc == 0)
           rc = lib.sglq_per_token_group_quant_fp8_scatter_scales_cm(x.data_ptr(), code, q1, f1, slot_map, m, k, topk, rows, 1e-10f, here.stream);
-        if (rc == 0 && walked) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, true, walk1, row_map);
-        else if (rc == 0)
+        if (rc == 0 && walked && !activates) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, true, walk1, row_map);
+        else if (rc == 0 && !walked)
           rc = lib.sglq_fp8_blockwise_scaled_grouped_mm_gathered(q1, k, m, row_map, w1.data_ptr(), w1.stride(2), e > 1 ? w1.stride(0) : 2 * n * k, f1,
                                                                  1, rows, static_cast<const float*>(s1.data_ptr()), s1.stride(0), s1.stride(1),
                                                                  s1.stride(2), y1, 2 * n, code, ps1, off_p, one_block ? plan_rows : 0, e, rows,
                                                                  2 * n, k, plan, plan_bytes, here.stream);
       } else {
         if (rc == 0) rc = lib.sglq_per_token_group_quant_fp8_scatter_cm(x.data_ptr(), code, q1, f1, slot_map, m, k, topk, rows, 1e-10f, here.stream);
-        if (rc == 0) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, one_block, walk1, nullptr);
+        if (rc == 0 && !activates) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, one_block, walk1, nullptr);
       }
-      if (rc == 0) rc = lib.sglq_silu_and_mul_group_quant_fp8_cm(y1, code, q2, f2, rows, n, 1e-10f, here.stream);
+      if (rc == 0 && activates)
+        rc = lib.sglq_fp8_blockwise_scaled_grouped_mm_silu(q1, k, gathers ? m : rows, gathers ? row_map : nullptr, w1.data_ptr(), w1.stride(2),
+                                                           e > 1 ? w1.stride(0) : 2 * n * k, f1, 1, rows, static_cast<const float*>(s1.data_ptr()),
+                                                           s1.stride(0), s1.stride(1), s1.stride(2), q2, f2, code, 1e-10f, e, rows, 2 * n, k, plan,
+                                                           plan_bytes, walk1, here.stream);
+      else if (rc == 0) rc = lib.sglq_silu_and_mul_group_quant_fp8_cm(y1, code, q2, f2, rows, n, 1e-10f, here.stream);
       if (rc == 0) rc = grouped(q2, f2, w2, s2, base, ps2, n, k, plan_rows2, shared_plan, walk2, nullptr);
       if (rc == 0 && float_weights)
         rc = lib.sglq_apply_shuffle_mul_sum_f32(base, out.data_ptr(), slot_map, static_cast<const float*>(weights.data_ptr()), code, m, topk, k,

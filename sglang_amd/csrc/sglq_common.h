@@ -92,6 +92,19 @@ SGLQ_DEV uint16_t from_f32_16(float v) {
   else return __builtin_bit_cast(uint16_t, (_Float16)v);
 }
 
+// ... two of them in a word, the first in its low half: one conversion instruction for both.
+template <int DT>
+SGLQ_DEV uint32_t from_f32_2x16(float lo, float hi) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  if constexpr (DT == SGLQ_BF16) {
+    typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{lo, hi}), bf2));
+  } else {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{lo, hi}), h2));
+  }
+}
+
 // silu(v) = v / (1 + exp(-v)) in fp32 with the hardware's exp2 and reciprocal (each within one
 // unit in the last place; the reference writes v / (1 + expf(-v)),
 // sgl-kernel/csrc/elementwise/activation.cu:57-60, and builds with -use_fast_math,
@@ -111,6 +124,18 @@ SGLQ_DEV uint16_t silu_mul_16(uint16_t xb, uint16_t yb) {
   asm volatile("" : "+v"(s));
   const float act = to_f32_16<DT>(from_f32_16<DT>(s));
   return from_f32_16<DT>(act * to_f32_16<DT>(yb));
+}
+// ... of two pairs, as from_f32_2x16 holds them.
+template <int DT>
+SGLQ_DEV uint32_t silu_mul_2x16(uint32_t x, uint32_t y) {
+  float s[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    s[e] = silu_f32(to_f32_16<DT>((uint16_t)(x >> (16 * e))));
+    asm volatile("" : "+v"(s[e]));
+  }
+  const uint32_t act = from_f32_2x16<DT>(s[0], s[1]);
+  return from_f32_2x16<DT>(to_f32_16<DT>((uint16_t)act) * to_f32_16<DT>((uint16_t)y), to_f32_16<DT>((uint16_t)(act >> 16)) * to_f32_16<DT>((uint16_t)(y >> 16)));
 }
 
 }  // namespace sglq

@@ -76,6 +76,18 @@ def test_walks(gpu, m, topk, e, n, k, empty, dtype):
         _lib.check(rc, "in the plan's order")
         assert torch.isfinite(y.float()).all() and torch.equal(y, z)
         assert bool((y[routed:] == 3.0).all())
+        if row_map_p is not None:
+            # ... and with the activation behind it: GEMM, activation and quantization one after the other
+            want_q, q = (torch.full((rows, n), 1, dtype=torch.uint8, device=gpu) for _ in range(2))
+            want_s, s = (torch.full((n // 128, rows), 5.0, device=gpu) for _ in range(2))
+            _lib.check(lib.sglq_silu_and_mul_group_quant_fp8_cm(p(y), out_code, p(want_q), p(want_s), rows, n, 1e-10, st), "activation")
+            for name, once in (("gathered", True), ("in place", False)):
+                src = a if once else torch.cat([a[row_map[:routed].long()], a[:1].expand(rows - routed, -1)])
+                head = (p(src), depth, src.shape[0], p(row_map) if once else None, *tail(q)[:-3])
+                _lib.check(lib.sglq_fp8_blockwise_scaled_grouped_mm_silu(*head, p(q), p(s), out_code, 1e-10, *sizes, p(walks) + at, st), name)
+                assert torch.equal(q[:routed], want_q[:routed]) and torch.equal(s[:, :routed], want_s[:, :routed]), name
+                assert bool((q[routed:] == 1).all()) and bool((s[:, routed:] == 5.0).all())
+                q.fill_(1), s.fill_(5.0)
 
 
 def test_layers_without_walks(gpu):
@@ -85,3 +97,46 @@ def test_layers_without_walks(gpu):
     assert lib.sglq_grouped_walk_bytes(32, 32 * 128, 2048, 7168, None) == 0  # 128-row tiles
     assert lib.sglq_grouped_walk_bytes(4, 4096, 256, 7168, None) == 0        # two K blocks
     assert lib.sglq_grouped_walk_bytes(0, 4096, 2048, 7168, None) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_activation_of_extremes(gpu, dtype):
+    """Rows of infinities, NaN, zeros and values that the 16-bit type cannot hold through GEMM, activation and quantization: what the three give."""
+    from sglang_amd import _lib
+
+    print("extremes", dtype, flush=True)
+    lib = _lib.load()
+    m, e, n, k = 700, 3, 384, 512
+    g = torch.Generator(device="cuda").manual_seed(5)
+    ids = torch.randint(0, e, (m, 1), generator=g, device=gpu, dtype=torch.int32)
+    second = ctypes.c_int64(0)
+    bytes_ = lib.sglq_grouped_walk_bytes(e, m, n, k, ctypes.byref(second))
+    i32 = lambda *shape: torch.zeros(shape, dtype=torch.int32, device=gpu)
+    offsets, ps1, ps2, slot_map, row_map, plan = i32(e + 1), i32(e, 3), i32(e, 3), i32(m), i32(m), i32(4 * (m // 256 + e + 1))
+    walks = torch.zeros(bytes_, dtype=torch.uint8, device=gpu)
+    p, st, code = (lambda t: t.data_ptr()), _lib.stream_ptr(gpu), 0 if dtype == torch.bfloat16 else 1
+    _lib.check(lib.sglq_prepare_moe_layer_walks(p(ids), p(offsets), p(ps1), p(ps2), p(slot_map), p(row_map), 1, m, e, n, k, p(plan), p(walks), bytes_, st), "walks")
+    w = torch.randn((e, 2 * n, k), generator=g, device=gpu).to(torch.float8_e4m3fn)
+    sw = torch.rand((e, 2 * n // 128, k // 128), generator=g, device=gpu) * 1e-2 + 1e-3
+    a = torch.randn((m, k), generator=g, device=gpu).to(torch.float8_e4m3fn)
+    sa = torch.rand((k // 128, m), generator=g, device=gpu) + 0.5
+    for i, v in enumerate((float("inf"), float("-inf"), float("nan"), 0.0, -0.0, 1e38, 1e4, 1e-20, 1e-38, -1.0)):
+        sa[:, i::13] = v
+    y = torch.zeros((m, 2 * n), dtype=dtype, device=gpu)
+    tail = (p(w), k, 2 * n * k, p(sa), 1, m, p(sw), sw.stride(0), 1, sw.stride(1))
+    sizes = (e, m, 2 * n, k, p(plan), plan.numel() * 4)
+    _lib.check(lib.sglq_fp8_blockwise_scaled_grouped_mm_walked(p(a), k, m, None, *tail, p(y), 2 * n, code, *sizes, p(walks), st), "walked")
+    (want_q, q), (want_s, s) = torch.zeros((2, m, n), dtype=torch.uint8, device=gpu), torch.zeros((2, n // 128, m), device=gpu)
+    _lib.check(lib.sglq_silu_and_mul_group_quant_fp8_cm(p(y), code, p(want_q), p(want_s), m, n, 1e-10, st), "activation")
+    _lib.check(lib.sglq_fp8_blockwise_scaled_grouped_mm_silu(p(a), k, m, None, *tail, p(q), p(s), code, 1e-10, *sizes, p(walks), st), "in one launch")
+    assert not torch.isfinite(y.float()).all()
+    assert torch.equal(q, want_q)
+    torch.testing.assert_close(s, want_s, rtol=0, atol=0, equal_nan=True)  # (a NaN has no sign to keep)
+
+
+# (rows x intermediate on both sides of 2^21, where the activation joins GEMM 1; slots gathered and not; intermediate sizes without a walk)
+@pytest.mark.parametrize("m,topk,e,n,k", [(911, 6, 6, 384, 512), (910, 6, 6, 384, 512), (2731, 2, 5, 384, 1024), (2730, 2, 5, 384, 1024), (900, 6, 6, 256, 512)])
+def test_layer(gpu, monkeypatch, m, topk, e, n, k):
+    import test_moe_tables_gpu as layers
+
+    layers.test_layer_host_path(gpu, monkeypatch, m, topk, e, n, k, torch.bfloat16, torch.float32)

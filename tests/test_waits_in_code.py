@@ -164,3 +164,45 @@ def test_gathered_rows_are_named_before_they_are_read(tmp_path):
         step = lambda states, op, operands: frozenset(filter(None, (one(s, op, operands) for s in states)))
         walk(code, frozenset([(None, False, False, 0, False)]), step, lambda old, new: new if old is None else old | new)
         assert seen["copy"] >= 2 and seen["read"] >= 18  # (two reads a map: in front of the walk, and at two steps of each of the four heights)
+
+
+@pytest.mark.parametrize("mode,tile_stores,inner_barriers", [(7, 16, 0), (9, 5, 1)])
+def test_walked_rows_are_named_before_they_are_read(tmp_path, mode, tile_stores, inner_barriers):
+    """The same of PIPE_WALKED_GATHERED and of PIPE_SILU_GATHERED, whose tiles have five stores, and a barrier between the copy of the row map and these."""
+    found = kernels(tmp_path, rf"gemm_pipe_kernelILi0ELi[01]ELi{mode}ELi256E")
+    assert len(found) == 2
+    for name, code in found.items():
+        seen = {"copy": 0, "read": 0, "handed over": 0}
+        header = min(((t - a, t) for a, (_, succ) in code.items() for t in succ if t < a))[1]  # of the walk over tiles, the longest loop
+        code[header][0].insert(0, ("next tile", ""))
+
+        def one(state, op, operands):  # operations younger than the copy (None: handed over); it has landed; barriers since (behind the tile's stores); stores; barriers in front of these; another tile
+            younger, landed, barrier, stores, inner, tile = state
+            count = vmcnt(op, operands)
+            if count is not None:
+                return (younger, landed or (younger is not None and count <= younger), barrier, stores, inner, tile)
+            if op == "buffer_load_dword" and operands.endswith("lds") and ", 0 offen" in operands:
+                seen["copy"] += 1
+                return (0, False, False, 0, 0, tile)
+            if op.startswith("ds_read2st64_b32"):
+                seen["read"] += 1
+                assert younger is None or not barrier, f"{name}: {op} {operands} behind a barrier, the copy and {younger} younger operations in flight"
+            if op.startswith("v_exp_f32") and tile:
+                return None  # (the activation's epilogue with none of the tile's heights in front of it)
+            if op == "next tile":
+                return None if tile else (younger, landed, barrier, stores, inner, True)
+            if op == "s_barrier":
+                if younger is None or landed:
+                    seen["handed over"] += younger is not None
+                    return (None, False, False, 0, 0, False)
+                if not barrier and stores == 0 and inner < inner_barriers:
+                    return (younger, False, False, 0, inner + 1, tile)
+                # (ways with another number of stores are none: they mix branches on the same condition)
+                return (younger, False, True, 0, inner, False) if barrier or (stores == tile_stores and inner == inner_barriers) else None
+            if VMEM.match(op):
+                return (younger if younger is None else min(younger + 1, 64), landed, barrier, min(stores + op.startswith("buffer_store"), 17), inner, tile)
+            return state
+
+        step = lambda states, op, operands: frozenset(filter(None, (one(s, op, operands) for s in states)))
+        walk(code, frozenset([(None, False, False, 0, 0, False)]), step, lambda old, new: new if old is None else old | new)
+        assert seen["copy"] >= 2 and seen["read"] >= 18 and seen["handed over"] >= 2
