@@ -303,9 +303,19 @@ int sglq_fp8_blockwise_scaled_grouped_mm_gathered(const void* a, int64_t lda, in
                                                   const int32_t* expert_offsets, int64_t plan_rows, int64_t num_experts,
                                                   int64_t total_m, int64_t N, int64_t K, void* plan, int64_t plan_bytes, void* stream);
 
+/* The row tile height for both GEMMs of an expert layer (n: intermediate, k: hidden size, each at least 384) from its expected tiles: 32, 64 or 128, for
+ * sglq_prepare_moe_layer and ..._tiled; 256, for sglq_prepare_moe_layer_walks, ..._walked and ..._silu; 0 where every GEMM's own choice stands. */
+int64_t sglq_grouped_layer_rows(int64_t num_experts, int64_t tokens, int64_t topk, int64_t n, int64_t k);
+int sglq_fp8_blockwise_scaled_grouped_mm_tiled(const void* a, int64_t lda, const void* b, int64_t ldb,
+                                               int64_t b_expert_stride, const float* sfa, int64_t sfa_stride_m,
+                                               int64_t sfa_stride_k, const float* sfb, int64_t sfb_expert_stride,
+                                               int64_t sfb_stride_k, int64_t sfb_stride_n, void* out, int64_t ldo,
+                                               int out_dtype, int64_t tile_rows, int64_t num_experts, int64_t total_m,
+                                               int64_t N, int64_t K, void* plan, int64_t plan_bytes, void* stream);
+
 /* ..._planned, or with a row map ..._gathered, on 256-row tiles in the order of a walk that sglq_prepare_moe_layer_walks has written: the experts' weights are
- * read from memory once.  sglq_grouped_walk_bytes: what the walks of a layer's two GEMMs take (n: intermediate, k: hidden size) and where the second one
- * begins; 0 where a layer has none. */
+ * read from memory once.  K of at least 384.  sglq_grouped_walk_bytes: what the walks of a layer's two GEMMs take (n: intermediate, k: hidden size) and where the
+ * second one begins; 0 where a layer cannot have them (n or k below 384, more than 256 experts). */
 int64_t sglq_grouped_walk_bytes(int64_t num_experts, int64_t total_m, int64_t n, int64_t k, int64_t* second);
 int sglq_fp8_blockwise_scaled_grouped_mm_walked(const void* a, int64_t lda, int64_t num_a_rows, const int32_t* row_map, const void* b,
                                                 int64_t ldb, int64_t b_expert_stride, const float* sfa, int64_t sfa_stride_m,

@@ -98,6 +98,9 @@ SIGNATURES = {
     "sglq_fp8_blockwise_scaled_grouped_mm_silu": [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p,
                                                   c_int64, c_int64, c_int64, c_void_p, c_void_p, c_int, c_float, c_int64, c_int64, c_int64, c_int64,
                                                   c_void_p, c_int64, c_void_p, c_void_p],
+    "sglq_fp8_blockwise_scaled_grouped_mm_tiled": [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p,
+                                                     c_int64, c_int64, c_int64, c_void_p, c_int64, c_int, c_int64, c_int64, c_int64, c_int64,
+                                                     c_int64, c_void_p, c_int64, c_void_p],
     "sglq_fp8_blockwise_scaled_grouped_mm_gathered": [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int64,
                                                       c_int64, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_int64, c_int, c_void_p,
                                                       c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p],
@@ -136,6 +139,8 @@ def load() -> ctypes.CDLL:
     lib.sglq_grouped_plan_rows.restype = c_int64
     lib.sglq_grouped_gathers.argtypes = [c_int64, c_int64, c_int64]
     lib.sglq_grouped_gathers.restype = c_int64
+    lib.sglq_grouped_layer_rows.argtypes = [c_int64, c_int64, c_int64, c_int64, c_int64]
+    lib.sglq_grouped_layer_rows.restype = c_int64
     lib.sglq_grouped_walk_bytes.argtypes = [c_int64, c_int64, c_int64, c_int64, c_void_p]
     lib.sglq_grouped_walk_bytes.restype = c_int64
     lib.sglq_abi_version.restype = c_int

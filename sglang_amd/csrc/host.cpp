@@ -67,6 +67,8 @@ namespace {
   X(sglq_prepare_moe_layer_walks)                                                                                   \
   X(sglq_grouped_gathers)                                                                                           \
   X(sglq_grouped_walk_bytes)                                                                                        \
+  X(sglq_grouped_layer_rows)                                                                                        \
+  X(sglq_fp8_blockwise_scaled_grouped_mm_tiled)                                                                     \
   X(sglq_fp8_blockwise_scaled_grouped_mm_walked)                                                                    \
   X(sglq_fp8_blockwise_scaled_grouped_mm_silu)                                                                      \
   X(sglq_fp8_blockwise_scaled_grouped_mm_gathered)                                                                  \
@@ -671,23 +673,25 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (!int32_buffer(ids, rows, x) || !int32_buffer(offsets, e + 1, x) || !int32_buffer(sizes1, 3 * e, x) || !int32_buffer(sizes2, 3 * e, x))
       return none();
     const int code = dtype_code(x.scalar_type());
-    const int64_t plan_rows = lib.sglq_grouped_plan_rows(e, rows, k), plan_rows2 = lib.sglq_grouped_plan_rows(e, rows, n);
     const bool one_block = rows <= 32768 && e <= 512;
+    const int64_t layer_rows = one_block ? lib.sglq_grouped_layer_rows(e, m, topk, n, k) : 0;
+    const bool walked = layer_rows == 256, tiled = layer_rows != 0 && !walked;
+    const int64_t plan_rows = layer_rows ? layer_rows : lib.sglq_grouped_plan_rows(e, rows, k);
+    const int64_t plan_rows2 = layer_rows ? layer_rows : lib.sglq_grouped_plan_rows(e, rows, n);
     const bool shared_plan = plan_rows == plan_rows2;  // (written by the tables, or by the first GEMM: a launch of 5 us less on 48000 slots, 2210 us a layer)
     // GEMM 1 gathers its rows from the tokens' codes, written once.  Quantization + GEMM 1, without and with (us), tokens x experts x
     // top-k, hidden x intermediate: 2500 x 32 x 8, 7168 x 2048 664 -> 626; 600 x 32 x 8 239 -> 223; 2500 x 16 x 3 266 -> 255;
     // 3000 x 16 x 4, 4096 x 1408 194.5 -> 187.8; on 6000 x 16, 2048 x 768 top-8 186 -> 173, top-3 78.5 and 78.4, top-2 68.0 -> 71.4:
     // two copies of the codes cost less than the gathering.
-    const bool gathers = topk > 2 && lib.sglq_grouped_gathers(e, rows, k) != 0;
+    const bool gathers = topk > 2 && (walked || (!tiled && lib.sglq_grouped_gathers(e, rows, k) != 0));
     const int64_t plan_bytes = round256(16 * (rows / 16 + e + 1));
-    // On 256-row tiles the tables come with both GEMMs' walks, and GEMM 1 with the activation and its quantization behind it, from 2^21 activations on
-    // (us, GEMM 1 and the activation's launch -> one launch): 2500 tokens x 32 experts x 8, 7168 x 2048 599.1 -> 584.7, 777 tokens 270.2 -> 260.9; 2048 x 64 x 8,
-    // 4096 x 1024 210.5 -> 198.8; 1870 x 8 x 8, 1152 x 512 32.6 -> 24.4; at 2.4 million 452 x 6 x 6, 5248 x 896 56.8 -> 57.1, 3767 x 8 x 1, 1920 x 640 28.8 -> 27.7.
-    // The activation takes the last tile of a block 5 us more than the stores that it saves, a launch of its own 2.5 us and its bytes: at 1.7 million 523 x 20 x 5,
-    // 7168 x 640 72.0 -> 74.3, at 1.4 million 442 x 16 x 5, 3456 x 640 39.7 -> 41.0.
+    // On 256-row tiles the tables come with both GEMMs' walks, and GEMM 1 with the activation and its quantization behind it.  Up to 128 rows an expert
+    // always, above where tiles fill 3/8 of the CUs: a tile's rows take it up to 8 us, a launch of its own 2.5 us and its bytes (GEMM 1 and the activation's launch -> one launch, us:
+    // 2500 tokens x 32 experts x 8, 7168 x 2048 582 -> 570; 777 tokens 267 -> 252; 2048 x 64 x 8, 4096 x 1024 211 -> 191; 1500 x 8 x 3, 1024 x 640 24.2 -> 20.0; of 40 layers of 20 to 128 rows
+    // an expert 0.944 on average, 1.013 at most; on few tiles of more rows 881 x 5 x 2, 3200 x 384 37.1 -> 38.5, 606 x 8 x 3, 3072 x 1024 37.2 -> 38.4).
     int64_t walk2_at = 0;
-    const int64_t walk_bytes = one_block ? lib.sglq_grouped_walk_bytes(e, rows, n, k, &walk2_at) : 0;
-    const bool walked = walk_bytes > 0, activates = walked && rows * n >= (2 << 20), maps_rows = walked || gathers || !one_block;
+    const int64_t walk_bytes = walked ? lib.sglq_grouped_walk_bytes(e, rows, n, k, &walk2_at) : 0;
+    const bool activates = walked && (rows < 129 * e || (rows / 256 + e / 2) * (n / 128) >= 96), maps_rows = walked || gathers || !one_block;
     // expert-major rows: quantized activations (dead once GEMM 1 has run) under GEMM 2's output, GEMM 1's
     // output, the quantized intermediate
     const int64_t codes1 = round256(rows * k), scales1 = round256(rows * (k / 128) * 4), c2 = round256(rows * k * 2);
@@ -729,6 +733,9 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
           return lib.sglq_fp8_blockwise_scaled_grouped_mm_walked(q, depth, map_p ? m : rows, map_p, w.data_ptr(), ldb, bs, f, 1, rows, s_p, s.stride(0),
                                                                  s.stride(1), s.stride(2), y, width, code, e, rows, width, depth, plan, plan_bytes,
                                                                  walk, here.stream);
+        if (tiled)
+          return lib.sglq_fp8_blockwise_scaled_grouped_mm_tiled(q, depth, w.data_ptr(), ldb, bs, f, 1, rows, s_p, s.stride(0), s.stride(1), s.stride(2), y,
+                                                                width, code, tile_rows, e, rows, width, depth, plan, plan_bytes, here.stream);
         return planned ? lib.sglq_fp8_blockwise_scaled_grouped_mm_planned(q, depth, w.data_ptr(), ldb, bs, f, 1, rows, s_p, s.stride(0),
                                                                           s.stride(1), s.stride(2), y, width, code, tile_rows, e, rows, width,
                                                                           depth, plan, plan_bytes, here.stream)

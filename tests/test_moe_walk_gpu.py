@@ -94,7 +94,7 @@ def test_layers_without_walks(gpu):
     from sglang_amd import _lib
 
     lib = _lib.load()
-    assert lib.sglq_grouped_walk_bytes(32, 32 * 128, 2048, 7168, None) == 0  # 128-row tiles
+    assert lib.sglq_grouped_walk_bytes(257, 65536, 2048, 7168, None) == 0  # more experts than the tables' blocks hold
     assert lib.sglq_grouped_walk_bytes(4, 4096, 256, 7168, None) == 0        # two K blocks
     assert lib.sglq_grouped_walk_bytes(0, 4096, 2048, 7168, None) == 0
 
@@ -134,9 +134,15 @@ def test_activation_of_extremes(gpu, dtype):
     torch.testing.assert_close(s, want_s, rtol=0, atol=0, equal_nan=True)  # (a NaN has no sign to keep)
 
 
-# (rows x intermediate on both sides of 2^21, where the activation joins GEMM 1; slots gathered and not; intermediate sizes without a walk)
-@pytest.mark.parametrize("m,topk,e,n,k", [(911, 6, 6, 384, 512), (910, 6, 6, 384, 512), (2731, 2, 5, 384, 1024), (2730, 2, 5, 384, 1024), (900, 6, 6, 256, 512)])
-def test_layer(gpu, monkeypatch, m, topk, e, n, k):
+# (the row tiles that the layer's sizes choose; on 256 rows the activation in GEMM 1 up to 128 rows an expert and from 96 tiles' worth, 24 x 3 and 35 x 3 here;
+# 0: each GEMM's own, below 12 rows an expert and on intermediate sizes without a walk)
+@pytest.mark.parametrize("m,topk,e,n,k,tile", [(900, 6, 6, 384, 512, 256), (1400, 6, 6, 384, 512, 256), (1400, 2, 5, 384, 1024, 256), (300, 8, 32, 1024, 1024, 256),
+                                               (121, 3, 24, 384, 1152, 32), (1326, 1, 9, 384, 2048, 64), (600, 2, 5, 2048, 1024, 128), (95, 4, 32, 384, 1664, 0),
+                                               (900, 6, 6, 256, 512, 0)])
+def test_layer(gpu, monkeypatch, m, topk, e, n, k, tile):
     import test_moe_tables_gpu as layers
 
+    from sglang_amd import _lib
+
+    assert _lib.load().sglq_grouped_layer_rows(e, m, topk, n, k) == tile
     layers.test_layer_host_path(gpu, monkeypatch, m, topk, e, n, k, torch.bfloat16, torch.float32)
