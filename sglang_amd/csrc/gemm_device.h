@@ -86,6 +86,10 @@ struct GemmArgs {
 // 25.7 -> 23.2 and 27.0 -> 24.4 us, 8192 x 4096 9.9 -> 8.7 and 10.2 -> 8.9, 4096 x 4096 5.8 -> 5.2 and 6.0 -> 5.4,
 // 7168 x 16384 26.2 -> 23.9 and 28.0 -> 26.2, 57344 x 8192 80.9 -> 78.5 and 92.8 -> 90.9; nothing on rows of 1, 2, 6, 7
 // or 14 KiB, which stay in order.
+// Grouped (gemm_kernel, gemm_ring_kernel): the tile is one of all experts' weights, and row tiles of one expert start together; whatever the rows, since an
+// expert's are few where these kernels run.  Layers in step and so, us: 64 x 8, 4096 x 1024 8 / 64 / 256 tokens 122 / 185 / 231 -> 105 / 161 / 212; 16 x 4, 4096 x 2048
+// 16 / 64 / 128 tokens 102 / 118 / 148 -> 85 / 102 / 100; 32 x 8, 8192 x 2048 32 / 64 / 256 tokens 308 / 392 / 384 -> 303 / 320 / 366; 32 x 4, 4096 x 4096 8 / 176
+// tokens 169 / 362 -> 148 / 315.  Weights that the last-level cache holds: even (8 x 2, 4096 x 2048 50.1 -> 51.1 at worst).
 SGLQ_DEV int first_k_step(const GemmArgs& p, uint32_t tile, int steps) {
   if (p.ldb & 4095) return 0;
   return (int)(((tile * 40503u & 0xffffu) * (uint32_t)steps) >> 16);  // 40503 / 2^16: the golden ratio

@@ -78,6 +78,7 @@ __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs 
   const int n0 = tn * BN;
   const char* weight = p.b;
   const float* weight_scale = p.sb;
+  uint32_t weight_tile = (uint32_t)tn;
   if constexpr (GROUPED) {
     const int* entry = static_cast<const int*>(p.ws) + PLAN_HEADER + PLAN_ENTRY * tm;
     const int expert = __builtin_amdgcn_readfirstlane(entry[0]);
@@ -85,13 +86,14 @@ __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs 
     m_end = __builtin_amdgcn_readfirstlane(entry[2]);
     weight += (int64_t)expert * p.b_expert_stride;
     weight_scale += (int64_t)expert * p.sb_expert_stride;
+    weight_tile = (uint32_t)(expert * p.tiles_n + tn);  // of all experts'
   }
   const int nkb = (p.K + 127) >> 7, T = (nkb + KG - 1) / KG;
   const int k_tail = p.K & 127;  // bytes of the last K block, 0 = all of it
   const bool sa_packed = HW && p.sa_packed;  // activation scales as words of four K blocks' exponent bytes
   const int sa_kshift = sa_packed ? 2 : 0;
 
-  const int first = GROUPED ? 0 : __builtin_amdgcn_readfirstlane(first_k_step_shared(p, (uint32_t)tn, T));  // stage t holds K step (t + first) % T
+  const int first = __builtin_amdgcn_readfirstlane(GROUPED ? first_k_step(p, weight_tile, T) : first_k_step_shared(p, weight_tile, T));  // stage t holds K step (t + first) % T
 
   using acc_t = typename std::conditional<float_acc(KIND), v4f, v4i>::type;
   acc_t acc[MI][NI];
