@@ -383,6 +383,13 @@ int sglq_prepare_moe_layer_walks(const int32_t* topk_ids, int32_t* expert_offset
                                  int32_t* problem_sizes2, int32_t* output_permutation, int32_t* input_permutation, int64_t topk,
                                  int64_t topk_length, int64_t num_experts, int64_t n, int64_t k, void* plan, void* walks,
                                  int64_t walks_bytes, void* stream);
+/* ... in one launch with sglq_per_token_group_quant_fp8_scatter_cm or, `once`, ..._scatter_scales_cm of the layer's activations [topk_length / topk, k] (16-bit types):
+ * any of the three tables, by whether input_permutation and walks are given.  Up to 1024 slots, 64 a token, k a multiple of 128. */
+int sglq_prepare_moe_layer_quant(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1,
+                                 int32_t* problem_sizes2, int32_t* output_permutation, int32_t* input_permutation, int64_t topk,
+                                 int64_t topk_length, int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows,
+                                 int64_t plan_max_tiles, void* plan, void* walks, int64_t walks_bytes, const void* input,
+                                 int in_dtype, void* output_q, float* output_s, int once, float eps, void* stream);
 int sglq_shuffle_rows(const void* input, const int32_t* dst2src_map, void* output, int64_t num_src_rows,
                       int64_t num_dst_rows, int64_t row_bytes, void* stream);
 int sglq_silu_and_mul(const void* input, int dtype, void* output, int64_t num_tokens, int64_t d, void* stream);

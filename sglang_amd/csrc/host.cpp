@@ -65,6 +65,7 @@ namespace {
   X(sglq_prepare_moe_layer)                                                                                         \
   X(sglq_prepare_moe_layer_rows)                                                                                    \
   X(sglq_prepare_moe_layer_walks)                                                                                   \
+  X(sglq_prepare_moe_layer_quant)                                                                                   \
   X(sglq_grouped_gathers)                                                                                           \
   X(sglq_grouped_walk_bytes)                                                                                        \
   X(sglq_grouped_layer_rows)                                                                                        \
@@ -636,8 +637,8 @@ PyObject* token_quant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 
 // ---------------------------------------------------------------------------
 // experts(a, w1_q, w2_q, w1_scale, w2_scale, topk_weights, topk_ids, expert_offsets, problem_sizes1,
-// problem_sizes2) -> [m, k]: cutlass_fused_experts_fp8 (moe/cutlass_moe.py) as six launches where the tables
-// fit one launch (prepare, quantize, GEMM, SiLU and quantize, GEMM, combine) from twelve, and
+// problem_sizes2) -> [m, k]: cutlass_fused_experts_fp8 (moe/cutlass_moe.py) as four to six launches where the tables
+// fit one launch (prepare and quantize, together on few slots; GEMM, SiLU and quantize, one launch on 256-row tiles; GEMM; combine) from twelve, and
 // one allocation beside the result's from eleven: a layer of a few tokens was bound by about 95 us of host
 // time around 30-50 us of GPU work.
 // ---------------------------------------------------------------------------
@@ -684,6 +685,10 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     // 3000 x 16 x 4, 4096 x 1408 194.5 -> 187.8; on 6000 x 16, 2048 x 768 top-8 186 -> 173, top-3 78.5 and 78.4, top-2 68.0 -> 71.4:
     // two copies of the codes cost less than the gathering.
     const bool gathers = topk > 2 && (walked || (!tiled && lib.sglq_grouped_gathers(e, rows, k) != 0));
+    // Few slots: the quantization runs beside the tables, in their launch (a launch of 5 us less; its blocks find their rows from all the ids).  Layers without and with
+    // (us), tokens x experts x top-k, hidden x intermediate: 1 x 64 x 6, 2048 x 1408 32.3 -> 28.7; 8 x 128 x 8, 2048 x 768 46.9 -> 43.1; 8 x 32 x 8, 7168 x 2048 223.8 -> 220.5; at 2048 slots
+    // 256 x 128 x 8 144.0 -> 140.0, 512 x 16 x 4, 5120 x 1536 136.6 -> 134.7, but 1024 x 8 x 2, 6144 x 2048, two blocks a CU, 158.3 -> 159.4.
+    const bool joins = rows <= 2048 && m <= 512 && e <= 512 && topk <= 64;
     const int64_t plan_bytes = round256(16 * (rows / 16 + e + 1));
     // On 256-row tiles the tables come with both GEMMs' walks, and GEMM 1 with the activation and its quantization behind it.  Up to 128 rows an expert
     // always, above where tiles fill 3/8 of the CUs: a tile's rows take it up to 8 us, a launch of its own 2.5 us and its bytes (GEMM 1 and the activation's launch -> one launch, us:
@@ -713,7 +718,11 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
               *ps2 = static_cast<int32_t*>(sizes2.data_ptr());
       char* const walk1 = reinterpret_cast<char*>(row_map) + map;
       char* const walk2 = walk1 + walk2_at;
-      if (walked) {
+      if (joins) {
+        rc = lib.sglq_prepare_moe_layer_quant(ids_p, off_p, ps1, ps2, slot_map, walked || gathers ? row_map : nullptr, topk, rows, e, n, k, plan_rows,
+                                              rows / plan_rows + e, plan, walked ? walk1 : nullptr, walk_bytes, x.data_ptr(), code, q1, f1, gathers, 1e-10f,
+                                              here.stream);
+      } else if (walked) {
         rc = lib.sglq_prepare_moe_layer_walks(ids_p, off_p, ps1, ps2, slot_map, row_map, topk, rows, e, n, k, plan, walk1, walk_bytes, here.stream);
       } else if (one_block && gathers) {
         rc = lib.sglq_prepare_moe_layer_rows(ids_p, off_p, ps1, ps2, slot_map, row_map, topk, rows, e, n, k, plan_rows, rows / plan_rows + e, plan,
@@ -744,7 +753,7 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                                                                   plan, plan_bytes, here.stream);
       };
       if (gathers) {
-        if (rc == 0)
+        if (rc == 0 && !joins)
           rc = lib.sglq_per_token_group_quant_fp8_scatter_scales_cm(x.data_ptr(), code, q1, f1, slot_map, m, k, topk, rows, 1e-10f, here.stream);
         if (rc == 0 && walked && !activates) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, true, walk1, row_map);
         else if (rc == 0 && !walked)
@@ -753,7 +762,7 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                                                                  s1.stride(2), y1, 2 * n, code, ps1, off_p, one_block ? plan_rows : 0, e, rows,
                                                                  2 * n, k, plan, plan_bytes, here.stream);
       } else {
-        if (rc == 0) rc = lib.sglq_per_token_group_quant_fp8_scatter_cm(x.data_ptr(), code, q1, f1, slot_map, m, k, topk, rows, 1e-10f, here.stream);
+        if (rc == 0 && !joins) rc = lib.sglq_per_token_group_quant_fp8_scatter_cm(x.data_ptr(), code, q1, f1, slot_map, m, k, topk, rows, 1e-10f, here.stream);
         if (rc == 0 && !activates) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, one_block, walk1, nullptr);
       }
       if (rc == 0 && activates)

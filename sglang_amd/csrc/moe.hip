@@ -203,11 +203,106 @@ struct LayerWalks {
 };
 constexpr int WALK_BAND = 8, WALK_ROWS = 256;
 
+// The activations of a layer of few slots, quantized beside its tables by blocks of their own; codes and scales are group_quant_scatter_kernel's (quant.hip; CM, ONCE).
+// Both launches are latency (tables 5.4 us, quantization 4.1-5.0 behind each other, whatever they hold), and the blocks depend on the ids alone.
+struct LayerQuant {
+  const char* x;
+  char* q;
+  float* s;
+  FastDiv walk;  // blocks to a band of tokens
+  uint32_t num_tokens, groups_per_row;
+  int first_block;  // blocks from here on (none: the grid ends there)
+  float eps, qmax, rqmax;
+};
+constexpr int QUANT_STEPS = 32, QUANT_MAX_SLOTS = 64 * QUANT_STEPS, QUANT_MAX_TOPK = 64;
+constexpr int QUANT_TOKENS = 2, QUANT_WAVES = TABLE_WAVES / QUANT_TOKENS;  // tokens to a block, waves to a token
+
+// A wave takes eight groups of 128 of one token.  Where the token's slots go its waves find for themselves, since the tables are being written: slots ordered by
+// (expert, slot) lie where their rank says, so a lane keeps such keys of every 64th slot and a ballot a step counts those in front.  Eight waves share a token's
+// slots (of a layer of 512 and of 1024 slots of 8 x 2, 6144 x 2048, us without / so: 106.8 / 102.7, 123.9 / 121.7; every wave for itself 16 tokens a block 109.4 / 105.7 and
+// 128.3 / 124.1, but 128 tokens x 128 x 8, 2048 x 768 125.9 -> 128.0 instead of 120.5; a band of 16 tokens placed by the tables' own code 0 to 2 us of the 4 won).
+template <int DT, bool ONCE>
+SGLQ_DEV void quantize_beside_tables(const int* __restrict__ topk_ids, int topk, int topk_length, int num_experts, const LayerQuant& quant,
+                                     int (&slot_row)[QUANT_TOKENS][QUANT_MAX_TOPK]) {
+  constexpr uint32_t NOBODY = ~0u;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t t = wave / QUANT_WAVES, of_token = wave % QUANT_WAVES, sub = lane & 7;
+  const uint32_t b = blockIdx.x - (uint32_t)quant.first_block, band = quant.walk.div(b);
+  const uint32_t token = band * QUANT_TOKENS + t, group = ((b - band * quant.walk.d) * QUANT_WAVES + of_token) * 8 + (lane >> 3);
+  const bool there = token < quant.num_tokens, live = there && group < quant.groups_per_row;
+  const int64_t hidden = (int64_t)quant.groups_per_row * 128, at = (int64_t)group * 128 + sub * 8;
+  Chunk8<DT> ch[2];
+  if (live) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) ch[c].load(quant.x + (token * hidden + at + c * 64) * elem_bytes<DT>());
+  }
+  const int steps = (topk_length + 63) >> 6;
+  auto key_of = [&](int i, bool any) {
+    const uint32_t e = any ? (uint32_t)topk_ids[i] : NOBODY;
+    return e < (uint32_t)num_experts ? e * QUANT_MAX_SLOTS + (uint32_t)i : NOBODY;
+  };
+  const uint32_t own = key_of((int)token * topk + lane, there && lane < topk);
+  uint32_t keys[QUANT_STEPS];
+#pragma unroll
+  for (int s = 0; s < QUANT_STEPS; ++s) keys[s] = key_of(s * 64 + lane, s * 64 + lane < topk_length);
+  for (int j = (int)of_token; j < topk; j += QUANT_WAVES) {
+    const uint32_t key = (uint32_t)__builtin_amdgcn_readlane((int)own, j);
+    int row = 0;
+#pragma unroll
+    for (int s = 0; s < QUANT_STEPS; ++s) {
+      if (s >= steps) break;
+      row += __popcll(__ballot(keys[s] < key));
+    }
+    slot_row[t][j] = key == NOBODY ? -1 : row;
+  }
+  v2u o[2];
+  float y_s = 0.f;
+  if (live) {
+    const uint32_t mb = group_umax<8>(umax(ch[0].amax_bits(), ch[1].amax_bits()));
+    const float amax = u2f(umax(mb, f2u(quant.eps)));
+    y_s = div_by(amax, quant.qmax, quant.rqmax);
+    const float r = 1.0f / y_s;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = quantize_elem<false>(ch[c].get(i), y_s, r, -quant.qmax, quant.qmax);
+      o[c] = Fp8Pack::pack(v);
+    }
+  }
+  __syncthreads();
+  if (!live) return;
+  if constexpr (ONCE) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) *reinterpret_cast<v2u*>(quant.q + token * hidden + at + c * 64) = o[c];
+  }
+  for (int j = ONCE ? (int)sub : 0; j < topk; j += ONCE ? 8 : 1) {
+    const int row = slot_row[t][j];
+    if (row < 0) continue;
+    if constexpr (!ONCE) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c) *reinterpret_cast<v2u*>(quant.q + row * hidden + at + c * 64) = o[c];
+    }
+    if (ONCE || sub == 0) quant.s[(int64_t)group * topk_length + row] = y_s;
+  }
+}
+
+// QUANT_DT: the activations' type, -1: tables only
+template <int QUANT_DT, bool ONCE>
 __global__ __launch_bounds__(TABLE_THREADS) void moe_tables_kernel(const int* __restrict__ topk_ids, int* __restrict__ expert_offsets,
                                                                    int* __restrict__ ps1, int* __restrict__ ps2,
                                                                    int* __restrict__ output_permutation, int* __restrict__ input_permutation,
                                                                    FastDiv topk, int topk_length, int num_experts, int id_bits, int n, int k, int* __restrict__ plan,
-                                                                   int plan_rows, int plan_max_tiles, int segment, const LayerWalks walks) {
+                                                                   int plan_rows, int plan_max_tiles, int segment, const LayerWalks walks,
+                                                                   const LayerQuant quant) {
+  if constexpr (QUANT_DT >= 0) {
+    if ((int)blockIdx.x >= quant.first_block) {
+      __shared__ int slot_row[QUANT_TOKENS][QUANT_MAX_TOPK];
+      quantize_beside_tables<QUANT_DT, ONCE>(topk_ids, (int)topk.d, topk_length, num_experts, quant, slot_row);
+      return;
+    }
+  }
   // [TABLE_WAVES][num_experts]: first the segment's counts, then the next position of each; of several segments, all slots' behind them
   extern __shared__ int counts[];
   __shared__ int wave_rows[TABLE_WAVES], wave_tiles[TABLE_WAVES];
@@ -215,7 +310,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void moe_tables_kernel(const int* __
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int begin_slot = (int)blockIdx.x * segment, end_slot = begin_slot + segment < topk_length ? begin_slot + segment : topk_length;
-  const bool alone = gridDim.x == 1;
+  const bool alone = quant.first_block == 1;
   const int steps = segment / TABLE_THREADS;  // 64 slots each, per wave
   const int first = begin_slot + wave * steps * 64;
   int id[TABLE_STEPS];
@@ -309,7 +404,7 @@ __global__ __launch_bounds__(TABLE_THREADS) void moe_tables_kernel(const int* __
     const uint32_t all_tiles = (uint32_t)expert_tiles[num_experts - 1], units1 = all_tiles * walks.columns[0].d;
     const uint32_t units = units1 + all_tiles * walks.columns[1].d;
     if ((int)blockIdx.x == walks.first_block && tid < 2) walks.walk[tid][0] = (int)(tid == 0 ? units1 : units - units1);
-    for (uint32_t i = (blockIdx.x - walks.first_block) * TABLE_THREADS + tid; i < units; i += (gridDim.x - walks.first_block) * TABLE_THREADS) {
+    for (uint32_t i = (blockIdx.x - walks.first_block) * TABLE_THREADS + tid; i < units; i += (uint32_t)(quant.first_block - walks.first_block) * TABLE_THREADS) {
       const bool one = i < units1;
       const int columns = (int)(one ? walks.columns[0].d : walks.columns[1].d);
       const uint32_t u = one ? i : i - units1;
@@ -520,7 +615,7 @@ extern "C" int sglq_prepare_moe_input(const int32_t* topk_ids, int32_t* expert_o
 static int prepare_layer_entry(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1, int32_t* problem_sizes2,
                                int32_t* output_permutation, int32_t* input_permutation, int64_t topk, int64_t topk_length,
                                int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows, int64_t plan_max_tiles, void* plan, void* stream,
-                               void* walk1 = nullptr, void* walk2 = nullptr) {
+                               void* walk1 = nullptr, void* walk2 = nullptr, LayerQuant quant = LayerQuant{}, int quant_dtype = -1, bool once = false) {
   const char* name = "prepare_moe_layer";
   if (topk_length <= 0 || num_experts <= 0 || n < 0 || k < 0 || n >= (1ll << 30) || k >= (1ll << 31) || plan_rows <= 0 ||
       plan_max_tiles <= 0 || plan_max_tiles >= (1ll << 27) || topk <= 0 || topk >= (1 << 20)) {
@@ -556,8 +651,24 @@ static int prepare_layer_entry(const int32_t* topk_ids, int32_t* expert_offsets,
     if (walk_blocks > 32) walk_blocks = 32;
   }
   const size_t lds = (size_t)(segments + walk_blocks > 1 ? 2 : 1) * TABLE_WAVES * num_experts * sizeof(int);
-  moe_tables_kernel<<<dim3((uint32_t)(segments + walk_blocks)), dim3(TABLE_THREADS), lds, static_cast<hipStream_t>(stream)>>>(
-      topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, input_permutation, per_token, (int)topk_length, (int)num_experts, id_bits, (int)n, (int)k, static_cast<int*>(plan), (int)plan_rows, (int)plan_max_tiles, (int)segment, walks);
+  quant.first_block = (int)(segments + walk_blocks);
+  int64_t quant_blocks = 0;
+  if (quant_dtype >= 0) {
+    quant.walk.init((quant.groups_per_row + 8 * QUANT_WAVES - 1) / (8 * QUANT_WAVES));
+    quant_blocks = (int64_t)((quant.num_tokens + QUANT_TOKENS - 1) / QUANT_TOKENS) * quant.walk.d;
+  }
+  const dim3 grid((uint32_t)(segments + walk_blocks + quant_blocks)), block(TABLE_THREADS);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+#define SGLQ_TABLES(DT, ONCE)                                                                                                                          \
+  moe_tables_kernel<DT, ONCE><<<grid, block, lds, st>>>(topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation,                 \
+                                                        input_permutation, per_token, (int)topk_length, (int)num_experts, id_bits, (int)n, (int)k,    \
+                                                        static_cast<int*>(plan), (int)plan_rows, (int)plan_max_tiles, (int)segment, walks, quant)
+  if (quant_dtype == SGLQ_BF16 && once) SGLQ_TABLES(SGLQ_BF16, true);
+  else if (quant_dtype == SGLQ_BF16) SGLQ_TABLES(SGLQ_BF16, false);
+  else if (quant_dtype == SGLQ_FP16 && once) SGLQ_TABLES(SGLQ_FP16, true);
+  else if (quant_dtype == SGLQ_FP16) SGLQ_TABLES(SGLQ_FP16, false);
+  else SGLQ_TABLES(-1, false);
+#undef SGLQ_TABLES
   return check_moe_launch(name);
 }
 
@@ -592,6 +703,44 @@ extern "C" int sglq_prepare_moe_layer_walks(const int32_t* topk_ids, int32_t* ex
   }
   return prepare_layer_entry(topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, input_permutation, topk, topk_length,
                              num_experts, n, k, WALK_ROWS, topk_length / WALK_ROWS + num_experts, plan, stream, walks, static_cast<char*>(walks) + second);
+}
+
+extern "C" int sglq_prepare_moe_layer_quant(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1, int32_t* problem_sizes2,
+                                            int32_t* output_permutation, int32_t* input_permutation, int64_t topk, int64_t topk_length,
+                                            int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows, int64_t plan_max_tiles, void* plan,
+                                            void* walks, int64_t walks_bytes, const void* input, int in_dtype, void* output_q, float* output_s,
+                                            int once, float eps, void* stream) {
+  const char* name = "prepare_moe_layer_quant";
+  if (topk <= 0 || topk > QUANT_MAX_TOPK || topk_length <= 0 || topk_length > QUANT_MAX_SLOTS || topk_length % topk != 0 || k <= 0 || k % 128 != 0) {
+    set_error("%s: up to %d slots, %d a token, k (%lld) a multiple of 128", name, QUANT_MAX_SLOTS, QUANT_MAX_TOPK, (long long)k);
+    return SGLQ_EINVAL;
+  }
+  if (in_dtype != SGLQ_BF16 && in_dtype != SGLQ_FP16) {
+    set_error("%s: unsupported in_dtype %d", name, in_dtype);
+    return SGLQ_EUNSUPPORTED;
+  }
+  if (!input || !output_q || !output_s || (reinterpret_cast<uintptr_t>(input) & 15) || (reinterpret_cast<uintptr_t>(output_q) & 7) || !(eps > 0.f)) {
+    set_error("%s: input must be 16-byte and output_q 8-byte aligned, eps positive", name);
+    return SGLQ_EINVAL;
+  }
+  int64_t second = 0;
+  if (walks && (plan_rows != WALK_ROWS || plan_max_tiles != topk_length / WALK_ROWS + num_experts || !input_permutation || (reinterpret_cast<uintptr_t>(walks) & 15) ||
+                sglq_grouped_walk_bytes(num_experts, topk_length, n, k, &second) == 0 ||
+                walks_bytes < sglq_grouped_walk_bytes(num_experts, topk_length, n, k, &second))) {
+    set_error("%s: walks need 256-row tiles, a row map and sglq_grouped_walk_bytes bytes, 16-byte aligned", name);
+    return SGLQ_EINVAL;
+  }
+  LayerQuant quant{};
+  quant.x = static_cast<const char*>(input);
+  quant.q = static_cast<char*>(output_q);
+  quant.s = output_s;
+  quant.num_tokens = (uint32_t)(topk_length / topk);
+  quant.groups_per_row = (uint32_t)(k / 128);
+  quant.eps = eps;
+  quant.qmax = 448.0f;
+  quant.rqmax = 1.0f / 448.0f;
+  return prepare_layer_entry(topk_ids, expert_offsets, problem_sizes1, problem_sizes2, output_permutation, input_permutation, topk, topk_length, num_experts, n, k,
+                             plan_rows, plan_max_tiles, plan, stream, walks, walks ? static_cast<char*>(walks) + second : nullptr, quant, in_dtype, once != 0);
 }
 
 extern "C" int sglq_shuffle_rows(const void* input, const int32_t* dst2src_map, void* output, int64_t num_src_rows,
