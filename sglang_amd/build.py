@@ -22,7 +22,7 @@ CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libsglq.so"
 BENCH_LIB_PATH = PKG_DIR / "libsglq_bench.so"
 NATIVE_PATH = PKG_DIR / "_native.so"
-SOURCES = ["gemm.hip", "gemm_ring_fp8_block.hip", "gemm_ring_fp8_block_grouped.hip", "gemm_ring_fp8_block_pow2.hip",
+SOURCES = ["gemm.hip", "gemm_ring_fp8_block.hip", "gemm_ring_fp8_block_grouped.hip", "gemm_ring_fp8_block_pow2.hip", "gemm_few_rows.hip",
            "gemm_ring_fp8_rowcol.hip", "gemm_ring_i8_rowcol.hip",
            "gemm_ring_i8_block.hip",
            *(f"gemm_kwave_{kind}.hip" for kind in ("fp8_block", "fp8_rowcol", "i8_rowcol", "i8_block")),
