@@ -333,15 +333,15 @@ int sglq_fp8_blockwise_scaled_grouped_mm_silu(const void* a, int64_t lda, int64_
                                               int64_t sfb_stride_k, int64_t sfb_stride_n, void* out_q, float* out_s,
                                               int act_dtype, float eps, int64_t num_experts, int64_t total_m, int64_t N,
                                               int64_t K, void* plan, int64_t plan_bytes, const void* walk, void* stream);
-/* The same on 32-row tiles (expert-major rows, a plan for 32-row tiles; no walk).  sglq_grouped_few_rows_activates: 1 where it is faster than GEMM and
+/* The same on tiles of `rows` rows, 32 or 64 (expert-major rows, a plan for such tiles; no walk).  sglq_grouped_few_rows_activates: 1 where it is faster than GEMM and
  * activation one after the other. */
-int sglq_grouped_few_rows_activates(int64_t num_experts, int64_t tokens, int64_t topk, int64_t n, int64_t k);
-int sglq_fp8_blockwise_scaled_grouped_mm_silu_32(const void* a, int64_t lda, const void* b, int64_t ldb,
+int sglq_grouped_few_rows_activates(int64_t num_experts, int64_t tokens, int64_t topk, int64_t n, int64_t k, int64_t rows);
+int sglq_fp8_blockwise_scaled_grouped_mm_silu_few_rows(const void* a, int64_t lda, const void* b, int64_t ldb,
                                                  int64_t b_expert_stride, const float* sfa, int64_t sfa_stride_m,
                                                  int64_t sfa_stride_k, const float* sfb, int64_t sfb_expert_stride,
                                                  int64_t sfb_stride_k, int64_t sfb_stride_n, void* out_q, float* out_s,
                                                  int act_dtype, float eps, int64_t num_experts, int64_t total_m, int64_t N,
-                                                 int64_t K, void* plan, int64_t plan_bytes, void* stream);
+                                                 int64_t K, void* plan, int64_t plan_bytes, int64_t rows, void* stream);
 
 /* The data movement around the grouped GEMM in an MoE layer
  * (python/sglang/srt/layers/moe/cutlass_moe.py:140-222).

@@ -95,9 +95,9 @@ SIGNATURES = {
                                                     c_int64, c_void_p, c_void_p],
     "sglq_prepare_moe_layer_walks": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p,
                                      c_void_p, c_int64, c_void_p],
-    "sglq_grouped_few_rows_activates": [c_int64, c_int64, c_int64, c_int64, c_int64],
-    "sglq_fp8_blockwise_scaled_grouped_mm_silu_32": [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64,
-                                                     c_void_p, c_void_p, c_int, c_float, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_void_p],
+    "sglq_grouped_few_rows_activates": [c_int64, c_int64, c_int64, c_int64, c_int64, c_int64],
+    "sglq_fp8_blockwise_scaled_grouped_mm_silu_few_rows": [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_int64,
+                                                     c_void_p, c_void_p, c_int, c_float, c_int64, c_int64, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p],
     "sglq_prepare_moe_layer_quant": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,
                                      c_int64, c_void_p, c_void_p, c_int64, c_void_p, c_int, c_void_p, c_void_p, c_int, c_float, c_void_p],
     "sglq_fp8_blockwise_scaled_grouped_mm_silu": [c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p,

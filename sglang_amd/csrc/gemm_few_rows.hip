@@ -1,12 +1,13 @@
-// gemm_few_rows_kernel: GEMM 1 of an expert layer of few rows an expert (decode) on 32-row tiles, with the activation and its quantization behind it.
+// gemm_few_rows_kernel: GEMM 1 of an expert layer of few rows an expert (decode) on 32- or 64-row tiles, with the activation and its quantization behind it.
 //
-// Bound by the weights' bytes from HBM.  A tile is 32 rows x 128 gates and their 128 partners, so that it holds whole groups of the activation; half as many tiles as
-// gemm_kernel<32 x 128> has.  Two blocks of two stages a CU, as that kernel has four, drain at every K block and lose on few tiles what the launch saves (16 experts, 5120 x 1536, 192
-// tiles: 86.6 -> 97.4 us a layer); so one block a CU keeps four stages of 37 KiB, three of them in flight, and walks its tiles without a break: the copies run on into the next
-// tile while one is finished.  Eight waves copy, five operations a stage each, and multiply, 16 gates and 16 partners each.
-// Layers without and with it, us (tokens x experts x top-k, hidden x intermediate): 16 x 32 x 8, 7168 x 2048 242.7 -> 231.8; 32 x 64 x 8, 4096 x 1024 148.5 -> 137.8;
-// 16 x 16 x 4, 5120 x 1536 86.4 -> 80.3; 42 x 64 x 6, 2048 x 1408 112.0 -> 106.5; 128 x 128 x 8, 2048 x 768 121.2 -> 114.2.  GEMM 2 on the same loop (256 columns and four stages,
-// or 128 and seven) is 1 to 3 % slower than on gemm_kernel and stays there.
+// Bound by the weights' bytes from HBM.  A tile is 32 or 64 rows x 128 gates and their 128 partners, so that it holds whole groups of the activation; half as many tiles as
+// gemm_kernel<32 x 128> and the ring's 64 x 128 have.  Two blocks of two stages a CU, as gemm_kernel has four, drain at every K block and lose on few tiles what the launch saves
+// (16 experts, 5120 x 1536, 192 tiles: 86.6 -> 97.4 us a layer); so one block a CU keeps four stages of 37 KiB, three of them in flight (64 rows: three of 41, two), and walks its tiles without a
+// break: the copies run on into the next tile while one is finished.  Eight waves copy, five or six operations a stage each, and multiply, 16 gates and 16 partners each.
+// Layers without and with it, us (tokens x experts x top-k, hidden x intermediate), on 32 rows: 16 x 32 x 8, 7168 x 2048 242.7 -> 231.2; 32 x 64 x 8, 4096 x 1024 147.3 -> 138.4;
+// 16 x 16 x 4, 5120 x 1536 86.9 -> 81.2; 42 x 64 x 6, 2048 x 1408 112.3 -> 106.4; 128 x 128 x 8, 2048 x 768 121.3 -> 114.3; on 64 rows: 480 x 60 x 4, 2048 x 1408 146.8 -> 129.3; 100 x 16 x 4,
+// 5120 x 1536 109.6 -> 97.8; 512 x 128 x 8, 2048 x 768 173.1 -> 156.5.  GEMM 2 on the same loop (256 columns and four stages, or 128 and seven) is 1 to 3 % slower than on gemm_kernel
+// and stays there.
 #include "gemm_device.h"
 #include "gemm_few_rows.h"
 #include "quant_device.h"
@@ -14,12 +15,14 @@
 
 namespace sglq {
 
-constexpr int FEW_ROWS = 32, FEW_WAVES = 8;
+constexpr int FEW_WAVES = 8;
 
-template <int OUT_DT>
+template <int OUT_DT, int BM>
 __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_rows_kernel(const GemmArgs p) {
-  constexpr int NW = FEW_WAVES, BM = FEW_ROWS, BN = 256, NST = 4, MI = 2, NI = 2, BCOPIES = BN / 8 / NW;
-  constexpr int CPS = BCOPIES + 1;  // copies of a wave and stage: its part of the weights, and one of the rest
+  static_assert(BM == 32 || BM == 64, "four or eight copies of activations a stage");
+  constexpr int NW = FEW_WAVES, BN = 256, NST = BM == 32 ? 4 : 3, MI = BM / 16, NI = 2, BCOPIES = BN / 8 / NW;
+  constexpr int CPS = BCOPIES + BM / 32;  // copies of a wave and stage: its part of the weights, and one of the rest (64 rows: one of the activations and one of the rest)
+  constexpr int W_SCALES = BM == 32 ? 4 : 0;  // the wave that copies the activations' scales; the next one copies the weights'
   constexpr int STAGE_BYTES = (BM + BN) * 128 + 512, SCALES = (BM + BN) * 128;
   constexpr int DUMP = NST * STAGE_BYTES, CODES = DUMP + 256, MAXIMA = CODES + BM * 128;
   static_assert((NST - 2) * CPS < 64, "vmcnt holds six bits");
@@ -58,7 +61,7 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_rows_kernel(const 
     // ---- copies: the stage of a step holds its K block's activations, weights and scales
     int c_tile = -1, c_left = 0, c_kb = 0;
     v4u rb = ra, rsb = ra;
-    uint32_t off_b[BCOPIES], off_rest = OOB;
+    uint32_t off_b[BCOPIES], off_a = OOB, off_s = OOB;
 #pragma unroll
     for (int j = 0; j < BCOPIES; ++j) off_b[j] = OOB;
     auto next_tile = [&]() {
@@ -66,7 +69,7 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_rows_kernel(const 
       c_left = nkb;
       if (c_tile >= here) {
         c_left = 1 << 30;
-        off_rest = OOB;
+        off_a = off_s = OOB;
 #pragma unroll
         for (int j = 0; j < BCOPIES; ++j) off_b[j] = OOB;
         return;
@@ -82,14 +85,13 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_rows_kernel(const 
         const int col = tn * (BN / 2) + (c >> 2) * 16 + (c & 1) * 8 + l8 + (c & 2 ? half : 0);  // 16 gates of a wave, 16 partners
         off_b[j] = (uint32_t)col * p.ldb + chunk;
       }
-      off_rest = OOB;
-      if (wave < 4) {
-        const int row = m0 + wave * 8 + l8;
-        if (row < end) off_rest = (uint32_t)row * p.lda + chunk;
-      } else if (wave == 4) {
-        if (lane < BM && m0 + lane < end) off_rest = (uint32_t)((m0 + lane) * p.sa_stride_m * 4);
-      } else if (wave == 5) {
-        if (lane < 2) off_rest = (uint32_t)((tn + (lane ? half >> 7 : 0)) * p.sb_stride_n * 4);
+      const int row = m0 + wave * 8 + l8;
+      off_a = (BM == 64 || wave < 4) && row < end ? (uint32_t)row * p.lda + chunk : OOB;
+      off_s = OOB;
+      if (wave == W_SCALES) {
+        if (lane < BM && m0 + lane < end) off_s = (uint32_t)((m0 + lane) * p.sa_stride_m * 4);
+      } else if (wave == W_SCALES + 1) {
+        if (lane < 2) off_s = (uint32_t)((tn + (lane ? half >> 7 : 0)) * p.sb_stride_n * 4);
       }
     };
     auto issue = [&](int slot) {
@@ -98,10 +100,12 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_rows_kernel(const 
       const bool live = c_tile < here;
 #pragma unroll
       for (int j = 0; j < BCOPIES; ++j) lds_copy16(rb, st + BM * 128 + (uint32_t)(wave + NW * j) * 1024u, off_b[j], live ? kb * 128u : 0u);
-      if (wave < 4) lds_copy16(ra, st + (uint32_t)wave * 1024u, off_rest, live ? kb * 128u : 0u);
-      else if (wave == 4) lds_copy4(rsa, st + SCALES, off_rest, live ? kb * (uint32_t)(p.sa_stride_k * 4) : 0u);
-      else if (wave == 5) lds_copy4(rsb, st + SCALES + 256, off_rest, live ? kb * (uint32_t)(p.sb_stride_k * 4) : 0u);
-      else lds_copy4(rsa, base + DUMP, OOB, 0u);
+      if (BM == 64 || wave < 4) lds_copy16(ra, st + (uint32_t)wave * 1024u, off_a, live ? kb * 128u : 0u);
+      if (BM == 64 || wave >= 4) {
+        if (wave == W_SCALES) lds_copy4(rsa, st + SCALES, off_s, live ? kb * (uint32_t)(p.sa_stride_k * 4) : 0u);
+        else if (wave == W_SCALES + 1) lds_copy4(rsb, st + SCALES + 256, off_s, live ? kb * (uint32_t)(p.sb_stride_k * 4) : 0u);
+        else lds_copy4(rsa, base + DUMP, OOB, 0u);
+      }
       --c_left;
       c_kb = c_kb + 1 == nkb ? 0 : c_kb + 1;
     };
@@ -179,13 +183,15 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_rows_kernel(const 
   }
 }
 
-void launch_few_rows(GemmArgs& p, int max_tiles, int out_dtype, hipStream_t st) {
+void launch_few_rows(GemmArgs& p, int max_tiles, int rows, int out_dtype, hipStream_t st) {
   p.tiles_n = p.N / 256;
   p.splits = 1;
   const int64_t tiles = (int64_t)max_tiles * p.tiles_n;
   const dim3 grid((uint32_t)(tiles < p.cus ? tiles : p.cus)), block(FEW_WAVES * 64);
-  if (out_dtype == SGLQ_BF16) gemm_few_rows_kernel<SGLQ_BF16><<<grid, block, 0, st>>>(p);
-  else gemm_few_rows_kernel<SGLQ_FP16><<<grid, block, 0, st>>>(p);
+  if (rows == 32 && out_dtype == SGLQ_BF16) gemm_few_rows_kernel<SGLQ_BF16, 32><<<grid, block, 0, st>>>(p);
+  else if (rows == 32) gemm_few_rows_kernel<SGLQ_FP16, 32><<<grid, block, 0, st>>>(p);
+  else if (out_dtype == SGLQ_BF16) gemm_few_rows_kernel<SGLQ_BF16, 64><<<grid, block, 0, st>>>(p);
+  else gemm_few_rows_kernel<SGLQ_FP16, 64><<<grid, block, 0, st>>>(p);
 }
 
 }  // namespace sglq

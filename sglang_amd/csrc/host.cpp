@@ -66,7 +66,7 @@ namespace {
   X(sglq_prepare_moe_layer_rows)                                                                                    \
   X(sglq_prepare_moe_layer_walks)                                                                                   \
   X(sglq_prepare_moe_layer_quant)                                                                                   \
-  X(sglq_fp8_blockwise_scaled_grouped_mm_silu_32)                                                                   \
+  X(sglq_fp8_blockwise_scaled_grouped_mm_silu_few_rows)                                                                   \
   X(sglq_grouped_few_rows_activates)                                                                                \
   X(sglq_grouped_gathers)                                                                                           \
   X(sglq_grouped_walk_bytes)                                                                                        \
@@ -698,13 +698,13 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     // an expert 0.944 on average, 1.013 at most; on few tiles of more rows 881 x 5 x 2, 3200 x 384 37.1 -> 38.5, 606 x 8 x 3, 3072 x 1024 37.2 -> 38.4).
     int64_t walk2_at = 0;
     const int64_t walk_bytes = walked ? lib.sglq_grouped_walk_bytes(e, rows, n, k, &walk2_at) : 0;
-    // ... and on 32-row tiles, by its tiles (a launch less, 3 to 10 us of 35 to 280)
-    const bool activates_32 = one_block && !walked && !gathers && plan_rows == 32 && lib.sglq_grouped_few_rows_activates(e, m, topk, n, k) != 0;
+    // ... and on 32- and 64-row tiles, by their number (a launch less, 3 to 17 us of 35 to 280)
+    const bool activates_few = one_block && !walked && !gathers && plan_rows <= 64 && lib.sglq_grouped_few_rows_activates(e, m, topk, n, k, plan_rows) != 0;
     const bool activates = walked && (rows < 129 * e || (rows / 256 + e / 2) * (n / 128) >= 96), maps_rows = walked || gathers || !one_block;
     // expert-major rows: quantized activations (dead once GEMM 1 has run) under GEMM 2's output, GEMM 1's
     // output, the quantized intermediate
     const int64_t codes1 = round256(rows * k), scales1 = round256(rows * (k / 128) * 4), c2 = round256(rows * k * 2);
-    const int64_t c1 = activates || activates_32 ? 0 : round256(rows * 2 * n * 2), codes2 = round256(rows * n), scales2 = round256(rows * (n / 128) * 4);
+    const int64_t c1 = activates || activates_few ? 0 : round256(rows * 2 * n * 2), codes2 = round256(rows * n), scales2 = round256(rows * (n / 128) * 4);
     const int64_t head = codes1 + scales1 > c2 ? codes1 + scales1 : c2, map = round256(rows * 4);
     Tensor out;
     int rc;
@@ -767,17 +767,17 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                                                                  2 * n, k, plan, plan_bytes, here.stream);
       } else {
         if (rc == 0 && !joins) rc = lib.sglq_per_token_group_quant_fp8_scatter_cm(x.data_ptr(), code, q1, f1, slot_map, m, k, topk, rows, 1e-10f, here.stream);
-        if (rc == 0 && !activates && !activates_32) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, one_block, walk1, nullptr);
+        if (rc == 0 && !activates && !activates_few) rc = grouped(q1, f1, w1, s1, y1, ps1, k, 2 * n, plan_rows, one_block, walk1, nullptr);
       }
       if (rc == 0 && activates)
         rc = lib.sglq_fp8_blockwise_scaled_grouped_mm_silu(q1, k, gathers ? m : rows, gathers ? row_map : nullptr, w1.data_ptr(), w1.stride(2),
                                                            e > 1 ? w1.stride(0) : 2 * n * k, f1, 1, rows, static_cast<const float*>(s1.data_ptr()),
                                                            s1.stride(0), s1.stride(1), s1.stride(2), q2, f2, code, 1e-10f, e, rows, 2 * n, k, plan,
                                                            plan_bytes, walk1, here.stream);
-      else if (rc == 0 && activates_32)
-        rc = lib.sglq_fp8_blockwise_scaled_grouped_mm_silu_32(q1, k, w1.data_ptr(), w1.stride(2), e > 1 ? w1.stride(0) : 2 * n * k, f1, 1, rows,
+      else if (rc == 0 && activates_few)
+        rc = lib.sglq_fp8_blockwise_scaled_grouped_mm_silu_few_rows(q1, k, w1.data_ptr(), w1.stride(2), e > 1 ? w1.stride(0) : 2 * n * k, f1, 1, rows,
                                                               static_cast<const float*>(s1.data_ptr()), s1.stride(0), s1.stride(1), s1.stride(2), q2, f2,
-                                                              code, 1e-10f, e, rows, 2 * n, k, plan, plan_bytes, here.stream);
+                                                              code, 1e-10f, e, rows, 2 * n, k, plan, plan_bytes, plan_rows, here.stream);
       else if (rc == 0) rc = lib.sglq_silu_and_mul_group_quant_fp8_cm(y1, code, q2, f2, rows, n, 1e-10f, here.stream);
       if (rc == 0) rc = grouped(q2, f2, w2, s2, base, ps2, n, k, plan_rows2, shared_plan, walk2, nullptr);
       if (rc == 0 && float_weights)
