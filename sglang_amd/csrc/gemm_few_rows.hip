@@ -34,7 +34,8 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_rows_kernel(const 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g = lane >> 4, l8 = lane >> 3;
   const int* const plan = static_cast<const int*>(p.ws);
-  const int tiles_m = plan[0], total = tiles_m * p.tiles_n, nkb = p.K >> 7, half = p.N >> 1;
+  const int listed = plan[0], tiles_m = listed < p.tiles_m ? listed : p.tiles_m;
+  const int total = tiles_m * p.tiles_n, nkb = p.K >> 7, half = p.N >> 1;
   const uint32_t base = lds_addr(smem);
   const uint32_t chunk = (uint32_t)(((lane & 7) ^ l8 ^ (wave & 1)) & 7) * 16u;  // (copies of a wave are eight groups of rows apart)
   const int nblocks = (p.N + 127) >> 7;
@@ -184,6 +185,7 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_rows_kernel(const 
 }
 
 void launch_few_rows(GemmArgs& p, int max_tiles, int rows, int out_dtype, hipStream_t st) {
+  p.tiles_m = max_tiles;
   p.tiles_n = p.N / 256;
   p.splits = 1;
   const int64_t tiles = (int64_t)max_tiles * p.tiles_n;
