@@ -62,7 +62,7 @@ def test_activation_on_weights_that_start_k_apart(gpu, tile):
 # around two and above)
 @pytest.mark.parametrize("m,topk,e,n,k,rows,activates", [(16, 4, 16, 1536, 1536, 32, 1), (16, 4, 16, 1536, 1408, 32, 0), (8, 8, 32, 1536, 1536, 32, 0), (32, 8, 64, 1024, 1536, 32, 1),
                                                          (60, 8, 64, 2048, 1536, 32, 0), (40, 1, 4, 384, 1536, 32, 0), (5, 3, 41, 1152, 2944, 32, 1),
-                                                         (100, 4, 16, 1536, 1536, 64, 1), (100, 2, 8, 2048, 1536, 64, 0), (480, 4, 60, 1408, 1536, 64, 1), (256, 8, 64, 1024, 1536, 64, 0),
+                                                         (90, 4, 16, 1024, 2048, 32, 1), (122, 4, 16, 1536, 1536, 32, 0), (122, 4, 16, 1536, 1536, 64, 1), (100, 2, 8, 2048, 1536, 64, 0), (480, 4, 60, 1408, 1536, 64, 1), (256, 8, 64, 1024, 1536, 64, 0),
                                                          (1, 8, 16, 3072, 1536, 64, 0)])
 def test_layer_of_few_rows(gpu, monkeypatch, m, topk, e, n, k, rows, activates):
     import test_moe_tables_gpu as layers
