@@ -324,7 +324,7 @@ int sglq_fp8_blockwise_scaled_grouped_mm_walked(const void* a, int64_t lda, int6
                                                 int64_t num_experts, int64_t total_m, int64_t N, int64_t K, void* plan,
                                                 int64_t plan_bytes, const void* walk, void* stream);
 
-/* ..._walked with the activation behind it: what the GEMM, rounded to act_dtype, sglq_silu_and_mul and the group quantization of its result (groups of 128, the
+/* ..._walked with the activation behind it: what that GEMM, rounded to act_dtype, sglq_silu_and_mul and the group quantization of its result (groups of 128, the
  * lower bound eps of a group's abs-max) return one after the other, bit for bit, in one launch: out_q [total_m, N / 2] e4m3fn (16-byte aligned), out_s its scales,
  * column-major [N / 256][total_m].  N = 2 x intermediate, a multiple of 256. */
 int sglq_fp8_blockwise_scaled_grouped_mm_silu(const void* a, int64_t lda, int64_t num_a_rows, const int32_t* row_map, const void* b,
@@ -333,8 +333,8 @@ int sglq_fp8_blockwise_scaled_grouped_mm_silu(const void* a, int64_t lda, int64_
                                               int64_t sfb_stride_k, int64_t sfb_stride_n, void* out_q, float* out_s,
                                               int act_dtype, float eps, int64_t num_experts, int64_t total_m, int64_t N,
                                               int64_t K, void* plan, int64_t plan_bytes, const void* walk, void* stream);
-/* The same on tiles of `rows` rows, 32 or 64 (expert-major rows, a plan for such tiles; no walk).  sglq_grouped_few_rows_activates: 1 where it is faster than GEMM and
- * activation one after the other. */
+/* The same on tiles of `rows` rows, 32 or 64 (expert-major rows, a plan for such tiles; no walk): what ..._tiled on 32 or 64 rows and the two behind it return, bit for bit (on weight
+ * rows 4 KiB apart the GEMMs of 128- and 256-row tiles sum in another order).  sglq_grouped_few_rows_activates: 1 where it is faster than GEMM and activation one after the other. */
 int sglq_grouped_few_rows_activates(int64_t num_experts, int64_t tokens, int64_t topk, int64_t n, int64_t k, int64_t rows);
 int sglq_fp8_blockwise_scaled_grouped_mm_silu_few_rows(const void* a, int64_t lda, const void* b, int64_t ldb,
                                                  int64_t b_expert_stride, const float* sfa, int64_t sfa_stride_m,

@@ -79,7 +79,7 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_rows_kernel(const 
       const int expert = __builtin_amdgcn_readlane(t_expert, c_tile), tn = __builtin_amdgcn_readlane(t_n, c_tile);
       rb = make_rsrc_sgpr(p.b + (int64_t)expert * p.b_expert_stride, p.b_bytes);
       rsb = make_rsrc_sgpr(p.sb + (int64_t)expert * p.sb_expert_stride, sb_bytes);
-      c_kb = __builtin_amdgcn_readfirstlane(first_k_step(p, (uint32_t)(expert * p.tiles_n + tn), nkb));
+      c_kb = __builtin_amdgcn_readfirstlane(first_k_step(p, grouped_weight_tile(p, expert, tn), nkb));
 #pragma unroll
       for (int j = 0; j < BCOPIES; ++j) {
         const int c = wave + NW * j;  // rows 8 c .. of the stage's weights

@@ -86,7 +86,8 @@ __global__ __launch_bounds__(RING_THREADS) void gemm_ring_kernel(const GemmArgs 
     m_end = __builtin_amdgcn_readfirstlane(entry[2]);
     weight += (int64_t)expert * p.b_expert_stride;
     weight_scale += (int64_t)expert * p.sb_expert_stride;
-    weight_tile = (uint32_t)(expert * p.tiles_n + tn);  // of all experts'
+    static_assert(BN == 128, "a tile's number");
+    weight_tile = grouped_weight_tile(p, expert, tn);
   }
   const int nkb = (p.K + 127) >> 7, T = (nkb + KG - 1) / KG;
   const int k_tail = p.K & 127;  // bytes of the last K block, 0 = all of it

@@ -5,7 +5,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _both(gpu, rows, n, k, dtype, a, w, sa, sw, tile):
+def _both(gpu, rows, n, k, dtype, a, w, sa, sw, tile, gemm=None, nan=False):
     from sglang_amd import _lib
 
     lib, e, m = _lib.load(), len(rows), sum(rows)
@@ -19,7 +19,7 @@ def _both(gpu, rows, n, k, dtype, a, w, sa, sw, tile):
     want_s, s = torch.full((2, n // 128, m), 5.0, device=gpu)
     head = (p(a), k, p(w), w.stride(1), w.stride(0), p(sa), 1, m, p(sw), sw.stride(0), 1, sw.stride(1))
     sizes = (e, m, 2 * n, k, p(plan), plan.numel() * 4)
-    lib.sglq_debug_grouped_tile(tile)
+    lib.sglq_debug_grouped_tile(gemm or tile)
     try:
         _lib.check(lib.sglq_fp8_blockwise_scaled_grouped_mm_planned(*head, p(y), 2 * n, code, tile, *sizes, st), "GEMM")
     finally:
@@ -28,7 +28,9 @@ def _both(gpu, rows, n, k, dtype, a, w, sa, sw, tile):
     call = lambda N=2 * n, out=q.data_ptr(), rows=tile: lib.sglq_fp8_blockwise_scaled_grouped_mm_silu_few_rows(*head, out, p(s), code, 1e-10, e, m, N, *sizes[3:], rows, st)
     _lib.check(call(), "in one launch")
     assert call(N=2 * n - 128) == 1 and call(out=q.data_ptr() + 8) == 1 and call(rows=128) == 1
-    assert torch.equal(q, want_q) and torch.equal(s, want_s)
+    assert torch.equal(q, want_q)
+    torch.testing.assert_close(s, want_s, rtol=0, atol=0, equal_nan=nan)  # (a NaN has no sign to keep)
+    return y
 
 
 # (fewer K blocks than stages; tiles begun, full and one row over; a block's first tile only, several, more than it has lanes for)
@@ -48,7 +50,7 @@ def test_activation_on_few_rows(gpu, rows, n, k, dtype, tile):
 
 @pytest.mark.parametrize("tile", [32, 64])
 def test_activation_on_weights_that_start_k_apart(gpu, tile):
-    """Weight rows 4 KiB apart: the tiles' K starts are others than gemm_kernel's; whole numbers and powers of two, which float32 adds up exactly in any order."""
+    """Weight rows 4 KiB apart, where every tile starts K at a place of its own; whole numbers and powers of two, which float32 adds up exactly in any order."""
     print("few rows, k starts", tile, flush=True)
     g = torch.Generator(device="cuda").manual_seed(3)
     rows, n, k = [7, 70, 0, 2], 640, 4096
@@ -56,6 +58,21 @@ def test_activation_on_weights_that_start_k_apart(gpu, tile):
     whole = lambda *s: torch.randint(-2, 3, s, generator=g, device=gpu).float().to(torch.float8_e4m3fn)
     two_to = lambda *s: 2.0 ** torch.randint(-9, -7, s, generator=g, device=gpu)
     _both(gpu, rows, n, k, torch.bfloat16, whole(m, k), whole(e, 2 * n, k), two_to(k // 128, m), two_to(e, 2 * n // 128, k // 128), tile)
+
+
+# (gemm_kernel's 32 and 64 rows, the ring's 64 x 128; a whole pitch, less than one, more)
+@pytest.mark.parametrize("tile,gemm", [(32, 32), (64, 64), (64, 305)])
+@pytest.mark.parametrize("k,pitch", [(4096, 4096), (1920, 4096), (4224, 8192)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_activation_sums_in_the_gemm_s_order(gpu, tile, gemm, k, pitch, dtype):
+    """Any values on weight rows 4 KiB apart: a tile of gates and partners starts K where the GEMM's tiles of the same columns do."""
+    print("few rows, order of the sums", tile, gemm, k, pitch, dtype, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(k + tile)
+    rows, n = [7, 70, 0, 2], 640
+    e, m = len(rows), sum(rows)
+    w = torch.randn((e, 2 * n, pitch), generator=g, device=gpu).to(torch.float8_e4m3fn)[:, :, :k]
+    sa, sw = torch.rand((k // 128, m), generator=g, device=gpu) + 0.5, torch.rand((e, 2 * n // 128, k // 128), generator=g, device=gpu) * 1e-2 + 1e-3
+    _both(gpu, rows, n, k, dtype, torch.randn((m, k), generator=g, device=gpu).to(torch.float8_e4m3fn), w, sa, sw, tile, gemm)
 
 
 # (tiles of 128 gates: from a quarter round of 256 CUs to one, beyond, from 1.85 rounds, beyond 3.1; all experts and some of them; too few K blocks; 64 rows: from 0.55 rounds,
@@ -71,3 +88,12 @@ def test_layer_of_few_rows(gpu, monkeypatch, m, topk, e, n, k, rows, activates):
 
     assert _lib.load().sglq_grouped_few_rows_activates(e, m, topk, n, k, rows) == activates
     layers.test_layer_host_path(gpu, monkeypatch, m, topk, e, n, k, torch.bfloat16, torch.float32)
+
+
+# (weight rows 4 KiB apart: below 12 rows an expert 32-row tiles, above)
+@pytest.mark.parametrize("m,topk,e,n", [(16, 4, 16, 1536), (32, 8, 64, 1024), (122, 4, 16, 1536)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_layer_on_weights_4_kib_apart(gpu, monkeypatch, m, topk, e, n, dtype):
+    import test_moe_tables_gpu as layers
+
+    layers.test_layer_host_path(gpu, monkeypatch, m, topk, e, n, 4096, dtype, torch.float32)
