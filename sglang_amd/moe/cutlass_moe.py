@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import torch
 
+from .. import _lib
 from .._lib import native
 from ..sgl_kernel import apply_shuffle_mul_sum, fp8_blockwise_scaled_grouped_mm, prepare_moe_input
 from ..sgl_kernel.moe import per_token_group_quant_fp8_to_expert_rows, silu_and_mul_per_token_group_quant_fp8
@@ -55,6 +56,7 @@ def cutlass_fused_experts_fp8(
     assert w1_q.shape[0] == w1_scale.shape[0], "w1 scales expert number mismatch"
     assert w1_q.shape[0] == w2_scale.shape[0], "w2 scales expert number mismatch"
     assert a.dtype in [torch.half, torch.bfloat16], "Invalid output dtype"
+    _lib.load()  # (binds the host path: a process's first layer takes its tiles too, and so gives every later one's bits)
     result = native.experts(a, w1_q, w2_q, w1_scale, w2_scale, topk_weights, topk_ids, expert_offsets, problem_sizes1, problem_sizes2)
     if result is not None:
         return result

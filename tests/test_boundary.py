@@ -278,3 +278,24 @@ def test_the_tuner_offers_every_ring_tile_that_the_tables_take():
         T.load_tuned_configs()  # back to the tables shipped with the package
     for m in (17, 512, 4096):
         assert {tile for tile, _ in candidates(m, 4096, 7168) if tile >= 300} == taken
+
+
+def test_the_first_expert_layer_is_asked_of_the_bound_host_path(monkeypatch):
+    """The host path stands back until the library is bound, and its row tiles are others than the operators': were it bound only by what stands in for it, a process's
+    first layer would differ from every later one of the same inputs."""
+    from sglang_amd import _lib
+    from sglang_amd.moe import cutlass_moe
+
+    bound = []
+
+    class Host:
+        experts = staticmethod(lambda *args: bound.append(_lib._lib is not None) or args[0])
+
+    monkeypatch.setenv("SGLQ_NO_TUNED_CONFIGS", "1")
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(cutlass_moe, "native", Host)
+    m, e, n, k = 3, 2, 128, 256
+    a, t = torch.zeros((m, k), dtype=torch.bfloat16), torch.zeros(1)
+    w1, w2 = torch.zeros((e, k, 2 * n)).to(FP8), torch.zeros((e, n, k)).to(FP8)
+    out = cutlass_moe.cutlass_fused_experts_fp8(a, w1, w2, torch.ones((e, 2, 2)), torch.ones((e, 1, 2)), torch.ones((m, 1)), torch.zeros((m, 1), dtype=torch.int32), *[t] * 13)
+    assert out is a and bound == [True]
