@@ -149,3 +149,32 @@ def moe_layer_case(m, topk, num_experts, n, k, seed, dtype=torch.bfloat16, w_std
         x=x, ids=ids, tw=tw,
         w1_q=torch.stack([t[0] for t in w1q]).transpose(1, 2), w1_s=torch.stack([t[1] for t in w1q]).transpose(1, 2),
         w2_q=torch.stack([t[0] for t in w2q]).transpose(1, 2), w2_s=torch.stack([t[1] for t in w2q]).transpose(1, 2))
+
+
+def launches(fn):
+    """The names (mangled) of the kernels that `fn` launches, in order, from a captured graph that is not replayed: the host path stands back under a profiler, not under capture."""
+
+    class Dim3(ctypes.Structure):
+        _fields_ = [(d, ctypes.c_uint) for d in "xyz"]
+
+    class KernelNode(ctypes.Structure):  # hipKernelNodeParams
+        _fields_ = [("block", Dim3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", Dim3), ("params", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
+    with open("/proc/self/maps") as maps:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))  # (the one that torch has loaded)
+    hip.hipKernelNameRefByPtr.argtypes, hip.hipKernelNameRefByPtr.restype = [ctypes.c_void_p, ctypes.c_void_p], ctypes.c_char_p
+    fn()  # (whatever a first call does besides)
+    torch.cuda.synchronize()
+    captured = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(captured):
+        fn()
+    graph, count = ctypes.c_void_p(captured.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0
+    nodes, names = (ctypes.c_void_p * count.value)(), []
+    assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(count)) == 0
+    for node in nodes:
+        kind, params = ctypes.c_int(-1), KernelNode()
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0 and kind.value == 0, "a node that is no kernel"
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(params)) == 0
+        names.append(hip.hipKernelNameRefByPtr(params.func, None).decode())
+    return names

@@ -60,6 +60,22 @@ def test_activation_on_weights_that_start_k_apart(gpu, tile):
     _both(gpu, rows, n, k, torch.bfloat16, whole(m, k), whole(e, 2 * n, k), two_to(k // 128, m), two_to(e, 2 * n // 128, k // 128), tile)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tile", [32, 64])
+def test_activation_of_extremes_on_few_rows(gpu, tile, dtype):
+    """Rows of infinities, NaN, zeros and values that the 16-bit type cannot hold."""
+    print("few rows, extremes", tile, dtype, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rows, n, k = [100, 0, 61, 3], 384, 512
+    e, m = len(rows), sum(rows)
+    w = torch.randn((e, 2 * n, k), generator=g, device=gpu).to(torch.float8_e4m3fn)
+    sa, sw = torch.rand((k // 128, m), generator=g, device=gpu) + 0.5, torch.rand((e, 2 * n // 128, k // 128), generator=g, device=gpu) * 1e-2 + 1e-3
+    for i, v in enumerate((float("inf"), float("-inf"), float("nan"), 0.0, -0.0, 1e38, 1e4, 1e-20, 1e-38, -1.0)):
+        sa[:, i::13] = v
+    y = _both(gpu, rows, n, k, dtype, torch.randn((m, k), generator=g, device=gpu).to(torch.float8_e4m3fn), w, sa, sw, tile, nan=True)
+    assert not torch.isfinite(y.float()).all()
+
+
 # (gemm_kernel's 32 and 64 rows, the ring's 64 x 128; a whole pitch, less than one, more)
 @pytest.mark.parametrize("tile,gemm", [(32, 32), (64, 64), (64, 305)])
 @pytest.mark.parametrize("k,pitch", [(4096, 4096), (1920, 4096), (4224, 8192)])
@@ -81,13 +97,15 @@ def test_activation_sums_in_the_gemm_s_order(gpu, tile, gemm, k, pitch, dtype):
                                                          (60, 8, 64, 2048, 1536, 32, 0), (40, 1, 4, 384, 1536, 32, 0), (5, 3, 41, 1152, 2944, 32, 1),
                                                          (90, 4, 16, 1024, 2048, 32, 1), (122, 4, 16, 1536, 1536, 32, 0), (122, 4, 16, 1536, 1536, 64, 1), (100, 2, 8, 2048, 1536, 64, 0), (480, 4, 60, 1408, 1536, 64, 1), (256, 8, 64, 1024, 1536, 64, 0),
                                                          (1, 8, 16, 3072, 1536, 64, 0)])
-def test_layer_of_few_rows(gpu, monkeypatch, m, topk, e, n, k, rows, activates):
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_layer_of_few_rows(gpu, monkeypatch, m, topk, e, n, k, rows, activates, dtype):
+    """What the rule says of tiles of that height, whichever height the layer takes (test_moe_dispatch_gpu.py has what it launches), and the layer's results."""
     import test_moe_tables_gpu as layers
 
     from sglang_amd import _lib
 
     assert _lib.load().sglq_grouped_few_rows_activates(e, m, topk, n, k, rows) == activates
-    layers.test_layer_host_path(gpu, monkeypatch, m, topk, e, n, k, torch.bfloat16, torch.float32)
+    layers.test_layer_host_path(gpu, monkeypatch, m, topk, e, n, k, dtype, torch.float32)
 
 
 # (weight rows 4 KiB apart: below 12 rows an expert 32-row tiles, above)

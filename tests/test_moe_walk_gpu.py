@@ -23,9 +23,10 @@ def _tiles(rows):
     return out
 
 
-# (one segment of slots and several, one expert, experts without rows, more than eight row tiles an expert, columns that end inside a tile)
+# (one segment of slots and several, one expert, experts without rows, more than eight row tiles an expert, columns that end inside a tile, fewer tiles than XCDs)
 @pytest.mark.parametrize("m,topk,e,n,k,empty", [(300, 2, 4, 384, 384, True), (515, 3, 4, 512, 640, False), (700, 6, 9, 384, 640, True), (641, 1, 1, 384, 1152, False),
-                                                (2500, 8, 32, 384, 1024, False), (4096, 7, 7, 1408, 512, True), (4096, 8, 250, 384, 384, False)])
+                                                (2500, 8, 32, 384, 1024, False), (4096, 7, 7, 1408, 512, True), (4096, 8, 250, 384, 384, False), (200, 1, 1, 384, 384, False),
+                                                (3, 1, 2, 384, 512, False)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_walks(gpu, m, topk, e, n, k, empty, dtype):
     from sglang_amd import _lib
@@ -69,10 +70,14 @@ def test_walks(gpu, m, topk, e, n, k, empty, dtype):
         sizes = (e, rows, width, depth, p(plan), plan.numel() * 4)
         _lib.check(lib.sglq_fp8_blockwise_scaled_grouped_mm_walked(p(a), depth, m, p(row_map) if row_map_p is not None else None, *tail(y), *sizes,
                                                                    p(walks) + at, st), "walked")
-        if row_map_p is not None:
-            rc = lib.sglq_fp8_blockwise_scaled_grouped_mm_gathered(p(a), depth, m, p(row_map), *tail(z), p(ps1), p(offsets), 256, *sizes, st)
-        else:
-            rc = lib.sglq_fp8_blockwise_scaled_grouped_mm_planned(p(a), depth, *tail(z), 256, *sizes, st)
+        lib.sglq_debug_grouped_tile(256)  # (256 rows where few tiles would take others, too)
+        try:
+            if row_map_p is not None:
+                rc = lib.sglq_fp8_blockwise_scaled_grouped_mm_gathered(p(a), depth, m, p(row_map), *tail(z), p(ps1), p(offsets), 256, *sizes, st)
+            else:
+                rc = lib.sglq_fp8_blockwise_scaled_grouped_mm_planned(p(a), depth, *tail(z), 256, *sizes, st)
+        finally:
+            lib.sglq_debug_grouped_tile(0)
         _lib.check(rc, "in the plan's order")
         assert torch.isfinite(y.float()).all() and torch.equal(y, z)
         assert bool((y[routed:] == 3.0).all())
@@ -146,3 +151,11 @@ def test_layer(gpu, monkeypatch, m, topk, e, n, k, tile):
 
     assert _lib.load().sglq_grouped_layer_rows(e, m, topk, n, k) == tile
     layers.test_layer_host_path(gpu, monkeypatch, m, topk, e, n, k, torch.bfloat16, torch.float32)
+
+
+# (fp16, where neither the layer nor the operators take 128-row tiles, whose last step rounds once)
+@pytest.mark.parametrize("m,topk,e,n,k", [(900, 6, 6, 384, 512), (1400, 6, 6, 384, 512), (1400, 2, 5, 384, 1024), (121, 3, 24, 384, 1152), (1326, 1, 9, 384, 2048)])
+def test_layer_of_halves(gpu, monkeypatch, m, topk, e, n, k):
+    import test_moe_tables_gpu as layers
+
+    layers.test_layer_host_path(gpu, monkeypatch, m, topk, e, n, k, torch.float16, torch.float32)
