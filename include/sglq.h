@@ -393,7 +393,7 @@ int sglq_prepare_moe_layer_walks(const int32_t* topk_ids, int32_t* expert_offset
                                  int64_t topk_length, int64_t num_experts, int64_t n, int64_t k, void* plan, void* walks,
                                  int64_t walks_bytes, void* stream);
 /* ... in one launch with sglq_per_token_group_quant_fp8_scatter_cm or, `once`, ..._scatter_scales_cm of the layer's activations [topk_length / topk, k] (16-bit types):
- * any of the three tables, by whether input_permutation and walks are given.  Up to 1024 slots, 64 a token, k a multiple of 128. */
+ * any of the three tables, by whether input_permutation and walks are given.  Up to 2048 slots, 64 a token, k a multiple of 128. */
 int sglq_prepare_moe_layer_quant(const int32_t* topk_ids, int32_t* expert_offsets, int32_t* problem_sizes1,
                                  int32_t* problem_sizes2, int32_t* output_permutation, int32_t* input_permutation, int64_t topk,
                                  int64_t topk_length, int64_t num_experts, int64_t n, int64_t k, int64_t plan_rows,

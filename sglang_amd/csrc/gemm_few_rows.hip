@@ -154,7 +154,7 @@ __global__ __launch_bounds__(FEW_WAVES * 64, 2) void gemm_few_rows_kernel(const 
         }
       }
       const int m0 = __builtin_amdgcn_readlane(t_m0, tile), end = __builtin_amdgcn_readlane(t_end, tile), tn = __builtin_amdgcn_readlane(t_n, tile);
-      uint16_t* const maxima = reinterpret_cast<uint16_t*>(smem + MAXIMA);  // [32 rows][8 waves]
+      uint16_t* const maxima = reinterpret_cast<uint16_t*>(smem + MAXIMA);  // [BM rows][8 waves]
       uint32_t h[MI][2];
 #pragma unroll
       for (int i = 0; i < MI; ++i) {

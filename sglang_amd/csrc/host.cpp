@@ -640,7 +640,7 @@ PyObject* token_quant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 // ---------------------------------------------------------------------------
 // experts(a, w1_q, w2_q, w1_scale, w2_scale, topk_weights, topk_ids, expert_offsets, problem_sizes1,
 // problem_sizes2) -> [m, k]: cutlass_fused_experts_fp8 (moe/cutlass_moe.py) as four to six launches where the tables
-// fit one launch (prepare and quantize, together on few slots; GEMM, SiLU and quantize, one launch on 256-row tiles; GEMM; combine) from twelve, and
+// fit one launch (prepare and quantize, together on few slots; GEMM, SiLU and quantize, one launch on 256-, 32- and 64-row tiles where that is faster; GEMM; combine) from twelve, and
 // one allocation beside the result's from eleven: a layer of a few tokens was bound by about 95 us of host
 // time around 30-50 us of GPU work.
 // ---------------------------------------------------------------------------
@@ -693,7 +693,7 @@ PyObject* experts(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const bool joins = rows <= 2048 && m <= 512 && e <= 512 && topk <= 64;
     const int64_t plan_bytes = round256(16 * (rows / 16 + e + 1));
     // On 256-row tiles the tables come with both GEMMs' walks, and GEMM 1 with the activation and its quantization behind it.  Up to 128 rows an expert
-    // always, above where tiles fill 3/8 of the CUs: a tile's rows take it up to 8 us, a launch of its own 2.5 us and its bytes (GEMM 1 and the activation's launch -> one launch, us:
+    // always, above from 96 tiles on (3/8 of the 256 CUs, on which this was measured): a tile's rows take it up to 8 us, a launch of its own 2.5 us and its bytes (GEMM 1 and the activation's launch -> one launch, us:
     // 2500 tokens x 32 experts x 8, 7168 x 2048 582 -> 570; 777 tokens 267 -> 252; 2048 x 64 x 8, 4096 x 1024 211 -> 191; 1500 x 8 x 3, 1024 x 640 24.2 -> 20.0; of 40 layers of 20 to 128 rows
     // an expert 0.944 on average, 1.013 at most; on few tiles of more rows 881 x 5 x 2, 3200 x 384 37.1 -> 38.5, 606 x 8 x 3, 3072 x 1024 37.2 -> 38.4).
     int64_t walk2_at = 0;
